@@ -41,6 +41,7 @@ struct xr_plan {
     int n_cond = 0, n_basis = 0, conv = 0, dir = 0;
     std::vector<float> cond_R, cond_t, cond_offset, basis, grating;
     std::vector<char> axis_cond;  // 1: every view of the condition has au[2] = ad[2] = 0
+    std::vector<char> lane_cond;  // lane axis of the condition's tilted forward projections (ViewGeom::lane_axis)
     xr::ViewGeom* d_vg = nullptr;
     xr::ChordGeom* d_cg = nullptr;
     float* d_g2 = nullptr;    // [n_cond*P][K]: (S_k.G)^2
@@ -54,6 +55,12 @@ struct xr_plan {
     const float* d_orient = nullptr;  // caller's orientation field (xr_plan_set_orientation), or null
     xr_tiles tiles{};      // projector tile shape (zeros: defaults)
     float max_factor = 0.f;     // largest per-pixel splat weight sum (set with d_norm)
+    // tilted forward projections: copies of the volume with axis 0 or 1 contiguous (FwdArgs::vol_axis), their
+    // lengths, the stream of the last launch that reads them and the event after it
+    float* d_lane[2] = {nullptr, nullptr};
+    size_t lane_len[2] = {0, 0};
+    hipStream_t lane_stream = nullptr;
+    hipEvent_t lane_done = nullptr;
     float* d_fmax = nullptr;    // device scalar receiving it during the weight pass
 };
 

@@ -41,7 +41,8 @@ constexpr int kMaxBasis = 16;
 // d0: source->voxel vector at x'=0 (d = vs*x' + d0, only its direction is used).
 // fy: un-rotated voxel y at y'=0 (FDK distance weight, fdk.cu:160).
 // G:  grating sensitivity vector (XTT, ir.cu:1901).  axis: 1 when au[2] and
-// ad[2] are exactly zero (u constant along z columns).
+// ad[2] are exactly zero (u constant along z columns).  lane_axis: the volume
+// axis (0 x, 1 y, 2 z) along which tilted forward projections lay their lanes.
 struct ViewGeom {
     float au[4];
     float av[4];
@@ -50,7 +51,8 @@ struct ViewGeom {
     float fy;
     float G[3];
     float axis;
-    float pad[4];
+    float lane_axis;
+    float pad[3];
 };
 static_assert(sizeof(ViewGeom) == 96, "ViewGeom layout");
 
@@ -127,6 +129,8 @@ struct FwdArgs {
     const int32_t* bands;    // untilted views: [code][band][y] columns xs | xe << 16 to scan, or null (all)
     const float* coef;       // XTT orientation field (forwardOrth): phi, cos theta per voxel, chan_stride apart, or null
     float out_scale = 1.0f;  // factor on each new pixel sum before it joins proj's contents (gradient grid: vs)
+    // tilted views: vol with axis 0 (x + N y + N^2 z) or 1 (y + N x + N^2 z) contiguous, or null (read vol strided)
+    const float* vol_axis[2] = {nullptr, nullptr};
     int view_group = 0;      // item order: 0 band-major; G > 0: groups of G views, all bands of a group together
 };
 
@@ -206,6 +210,8 @@ hipError_t launch_fdk_filter(const float* src, float* dst, const float* weight, 
 hipError_t launch_fdk_weight(float* weight, int U, int V, float sdd, float det, hipStream_t stream);
 hipError_t launch_to_internal(const float* ref, float* internal, int N, int channels, hipStream_t stream);
 hipError_t launch_from_internal(const float* internal, float* ref, int N, int channels, hipStream_t stream);
+// Column-layout volume -> the layout of FwdArgs::vol_axis[lane_axis] (0 or 1).
+hipError_t launch_lane_copy(const float* cols, float* out, int N, int channels, int lane_axis, hipStream_t stream);
 hipError_t launch_sqrt_abs(float* vol, int64_t n, hipStream_t stream);
 hipError_t launch_vol_down(const float* fine, float* coarse, int Nc, int f, hipStream_t stream);
 hipError_t launch_orth_normal(const float* vol, float* coef, float* loss, int64_t n, int rot, const float* est,

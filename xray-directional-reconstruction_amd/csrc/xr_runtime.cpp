@@ -146,7 +146,13 @@ void build_view(const xr_plan& p, int cond, int view, ViewGeom& vg, ChordGeom& c
     mat3vec(R, g0, G);
     for (int i = 0; i < 3; i++) vg.G[i] = (float)G[i];
     vg.axis = (vg.au[2] == 0.0f && vg.ad[2] == 0.0f) ? 1.0f : 0.0f;
-    for (int i = 0; i < 4; i++) vg.pad[i] = 0.0f;
+    // lanes of a tilted forward projection: the volume axis closest to the
+    // detector's v direction, which is the condition's for all its views
+    int la = 2;
+    for (int i = 1; i >= 0; i--)
+        if (std::fabs(ev[i]) > std::fabs(ev[la])) la = i;
+    vg.lane_axis = (float)la;
+    for (int i = 0; i < 3; i++) vg.pad[i] = 0.0f;
     // chord geometry of the IR source side (ir.cu:1556-1574)
     cg.det[0] = g.det_size;
     cg.det[1] = (double)g.sdd - (double)g.sod;
@@ -213,6 +219,63 @@ hipEvent_t get_event(xr_context* ctx) {
     return e;
 }
 
+
+// Copies of the volume for the conditions whose lanes run along x or y (see
+// splat_tilted), in buffers of the plan: reading the column layout strided
+// costs one cache line per lane.  A launch of one view would read what it
+// copies only once and goes without, and so does one that may not allocate: a
+// stream under capture, a failed allocation.  The images are the same.
+static int lane_copies(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stride, int code_base, int n_slots,
+                       FwdArgs& a, bool& used) {
+    xr_context* ctx = p->ctx;
+    used = false;
+    if (n_slots < 2) return XR_OK;
+    // a solver's launch over one condition's single volume (vol_cond_stride 0) has that condition's codes alone
+    const int c0 = kind == FWD_PLAIN && vol_cond_stride == 0 ? code_base / p->g.n_proj : 0;
+    const int c1 = kind == FWD_PLAIN && vol_cond_stride == 0 ? c0 + 1 : p->n_cond;
+    bool want[2] = {false, false};
+    for (int c = c0; c < c1; c++)
+        if (p->lane_cond[c] < 2) want[(int)p->lane_cond[c]] = true;
+    if (!want[0] && !want[1]) return XR_OK;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    XR_HIP(ctx, hipStreamIsCapturing(ctx->stream, &st));
+    if (st != hipStreamCaptureStatusNone) return XR_OK;
+    const int N = p->g.n_vox;
+    const int channels = kind == FWD_XTT ? p->n_basis : (vol_cond_stride ? p->n_cond : 1);
+    const size_t len = (size_t)N * N * N * channels;
+    if (!p->lane_done) XR_HIP(ctx, hipEventCreateWithFlags(&p->lane_done, hipEventDisableTiming));
+    for (int la = 0; la < 2; la++) {
+        if (!want[la]) continue;
+        if (p->lane_len[la] < len) {
+            if (p->d_lane[la]) (void)hipFree(p->d_lane[la]);
+            p->d_lane[la] = nullptr;
+            p->lane_len[la] = 0;
+            if (device_malloc((void**)&p->d_lane[la], len * sizeof(float)) != hipSuccess) {
+                (void)hipGetLastError();
+                continue;
+            }
+            p->lane_len[la] = len;
+        }
+        // the previous launch that reads the buffer may be on another stream
+        if (p->lane_stream != ctx->stream) XR_HIP(ctx, hipStreamWaitEvent(ctx->stream, p->lane_done, 0));
+        float* dst = p->d_lane[la];
+        if (kind == FWD_PLAIN && vol_cond_stride) {
+            // only the volumes of the conditions with these lanes
+            const int64_t N3 = (int64_t)N * N * N;
+            for (int c = c0; c < c1; c++)
+                if (p->lane_cond[c] == la)
+                    XR_TRY(timed(ctx, 3, [&] {
+                        return launch_lane_copy(vol + c * N3, dst + c * N3, N, 1, la, ctx->stream);
+                    }));
+        } else {
+            XR_TRY(timed(ctx, 3, [&] { return launch_lane_copy(vol, dst, N, channels, la, ctx->stream); }));
+        }
+        a.vol_axis[la] = dst;
+        used = true;
+    }
+    p->lane_stream = ctx->stream;
+    return XR_OK;
+}
 
 // vol_cond_stride: plain volumes of several conditions side by side (N^3), or 0
 // for a single volume; code_base: proj/sino hold the images of codes >= code_base.
@@ -286,6 +349,8 @@ int forward_launch(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stri
         a.coef = p->d_orient;  // forwardOrth: per-voxel rotation, general path
         axis = false;
     }
+    bool copies = false;
+    if (!axis && kind != FWD_WEIGHT && !no_alloc) XR_TRY(lane_copies(p, kind, vol, vol_cond_stride, code_base, n_slots, a, copies));
     // Detector rows in equal chunks, all in one launch (untilted scans walk
     // only the z range that reaches a chunk's rows).
     const int V = p->g.n_det_v;
@@ -307,7 +372,9 @@ int forward_launch(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stri
         XR_HIP(ctx, launch_forward(a, kind, axis, ctx->stream));
         return XR_OK;
     }
-    return timed(ctx, 0, [&] { return launch_forward(a, kind, axis, ctx->stream); });
+    XR_TRY(timed(ctx, 0, [&] { return launch_forward(a, kind, axis, ctx->stream); }));
+    if (copies) XR_HIP(ctx, hipEventRecord(p->lane_done, ctx->stream));
+    return XR_OK;
 }
 
 int forward_rows(const xr_plan* p, int kind) {
@@ -717,11 +784,13 @@ int xr_plan_create(xr_context* ctx, const xr_geometry* g, const xr_scan* s, int 
     const int KS = kXwStride;
     std::vector<float> xw((size_t)C * P * 5 * KS, 0.f);
     p->axis_cond.assign(C, 1);
+    p->lane_cond.assign(C, 2);
     for (int c = 0; c < C; c++)
         for (int v = 0; v < P; v++) {
             ViewGeom& t = vg[(size_t)c * P + v];
             build_view(*p, c, v, t, cg[(size_t)c * P + v]);
             if (t.axis == 0.0f) p->axis_cond[c] = 0;
+            p->lane_cond[c] = (char)t.lane_axis;
             for (int k = 0; k < s->n_basis; k++) {
                 const double sg = (double)p->basis[3 * k] * t.G[0] + (double)p->basis[3 * k + 1] * t.G[1] +
                                   (double)p->basis[3 * k + 2] * t.G[2];
@@ -802,6 +871,9 @@ void xr_plan_destroy(xr_plan* p) {
     if (p->d_xw) (void)hipFree(p->d_xw);
     if (p->d_norm) (void)hipFree(p->d_norm);
     if (p->d_bands) (void)hipFree(p->d_bands);
+    for (float* v : p->d_lane)
+        if (v) (void)hipFree(v);
+    if (p->lane_done) (void)hipEventDestroy(p->lane_done);
     delete p;
 }
 
