@@ -85,6 +85,8 @@ struct Dims {
     float ratio;     // (vs*vs)/(det*(sod/sdd)*det*(sod/sdd))
     float sod;
     float cfdk;      // 2 pi / P (FP32, fdk.cu:161)
+    float px;        // detector pixels per voxel where the magnification is largest (launch shapes)
+    float tilt_cos, tilt_sin;  // largest z extent of a unit z step on the detector along v, along u (launch shapes)
 };
 
 struct Basis {
@@ -156,6 +158,7 @@ struct BwdArgs {
     int zpl, gx, gy;          // tile shape: z voxels per lane (1, 2, 4), column groups along x, y (gx*gy = 16)
     int tiles_x, tiles_y, tiles_z, n_tiles, per_xcd;
     int axis;                 // batched launches: 1 -> every view is axis aligned
+    int wide;                 // untilted: footprints wider than the fixed staging width (set with the shape)
     unsigned* vmax_out;       // batched MLEM / ART: atomic max of |updated voxel| (float bits), or null
     const float* coef;        // XTT orientation field (backwardOrth): phi, cos theta per voxel, or null
 };
@@ -199,7 +202,6 @@ inline int forward_split(int64_t items, int64_t slots, int tile) {
     return s;
 }
 int batch_blocks_per_cu_backward(int kind, int zpl, int kmax = 0);
-size_t backward_batch_lds_bytes(int kind);
 // out[i] = max |segs[i][0, seg_len[i])| (out zeroed beforehand).
 // blocks per segment for k_absmax_seg over n_seg segments of at most max_len floats
 int absmax_blocks(int64_t max_len, int n_seg);

@@ -84,7 +84,12 @@ __device__ __forceinline__ void split(float u, int& iu, float& fu) {
     fu = t - f;
 }
 
+// lambdas of a kernel body that several places call: without it they become
+// calls, with their captures in scratch memory
+#define XR_INLINE __attribute__((always_inline))
+
 typedef __attribute__((address_space(3))) float lds_float;
+typedef __attribute__((address_space(3))) int lds_int;
 
 // Global-memory view of a pointer.  Kernel-argument pointers are known to be
 // global, but pointers read from a work-item table in memory are not: without
@@ -1135,94 +1140,130 @@ __global__ __launch_bounds__(64 * kFwdWaves) __attribute__((amdgpu_waves_per_eu(
 }
 
 // ---------------------------------------------------------------------------
-// Backprojection gather with fused update.  Block = BwdBlock waves laid out
-// as a gx x gy grid of CPW x CPW column groups; every lane owns ZPL voxels
-// (z = z0 + lane + 64 q) in each of its CPW^2 columns, so the per-column
-// geometry of a view is computed once per ZPL voxels.  The block's detector
-// footprint for each view is staged in LDS: the untilted paths fetch view s+2
-// into registers while view s is accumulated (four buffers, a barrier every
-// second view), the general path view s+1 (two buffers, a barrier per view).
-// The update (MLEM / ART / FDK / raw) is applied at the end: each voxel is
-// read and written once per subset.
+// Backprojection gather with fused update.  A block of WAVES waves laid out as
+// a gx x gy grid owns a voxel tile; a wave owns CX x CY columns, a lane ZPL
+// voxels (z = z0 + lane + 64 q) in each, so the per-column terms of a view are
+// read once per ZPL voxels.  Everything of a view that is the same in all
+// lanes of a wave is computed lane-parallel 16 views at a time into LDS: the
+// block's detector footprints by wave 0 (lane = view x corner pair), the
+// column terms by every wave for its own columns (lane = view x column, or x
+// channel quarter); the view loop reads them back with broadcast LDS loads.
+//
+// The footprints are staged in LDS VB views (a group) ahead, in 2 VB buffers,
+// with one barrier per group.  A footprint is fetched into registers and
+// stored after the view (LOOK = 1) or the group (LOOK = VB) that is accumulated
+// meanwhile.  Large tiles take VB = 2, LOOK = 1: the work of one view covers a
+// load's latency.  Small tiles take VB = LOOK = 8, where it does not: one
+// latency per eight views.
+//
+// The update (MLEM / ART / FDK / raw) is applied at the end: each voxel is read
+// and written once per subset.
+//
+// Bound by VALU issue (about 15 instructions per 64 voxel-views of a whole
+// column), the footprint's edges and, with few views, the tile's start.
+// Measured, before -> now: MLEM 512^3 / 720 views 60.4 -> 48.7 ms, 64^3 / 90
+// views 184 -> 41 us, 203^3 / 20 views 249 -> 154 us; FDK 320^3 / 401 views
+// 18.2 -> 7.3 ms; ART 128^3 tilted by 30 degrees, 45 views 478 -> 210 us.
 // ---------------------------------------------------------------------------
 template <int KIND>
 struct IsXtt {
     static constexpr bool value = (KIND == BWD_XTT_RAW || KIND == BWD_XTT_MLEM || KIND == BWD_XTT_ART);
 };
 
-// Block shape per kind.  The plain kinds (about 110 VGPRs, 4 waves per SIMD)
+constexpr int kBwdBatch = 16;                              // views per batch of per-view terms
+constexpr int kFootWords = 12;  // iu_lo, iv_lo, W, Ws | R, flags, code, -, then the staging words: address (2), range, H
+constexpr int kBwdFootArea = 2 * kBwdBatch * kFootWords;   // words, block-wide, two batches
+enum FootFlag { FOOT_STAGED = 1, FOOT_EMPTY = 2, FOOT_INSIDE = 4 };
+
+// Tile shape and staging of a backprojection kernel.  NP: staged floats per
+// thread and view.  WF > 0: every footprint is staged WF texels wide (a power
+// of two), threads / WF rows per pass, whole passes; the row stride WF + 1 is
+// then a constant, and so are a thread's offsets into the image and the buffer.
+// WF = 0: footprints of any width up to SB floats (tilted views; untilted ones
+// with more than about 1.4 detector pixels per voxel).
+template <int KIND_, int WAVES_, int CX_, int CY_, int ZPL_, int KM_, int VB_, int LOOK_, int WF_, int NP_>
+struct BwdCfg {
+    static constexpr int KIND = KIND_, WAVES = WAVES_, CX = CX_, CY = CY_, ZPL = ZPL_, VB = VB_, LOOK = LOOK_,
+                         WF = WF_, NP = NP_;
+    static constexpr int R = WF_ ? 64 * WAVES_ / (WF_ ? WF_ : 1) : 0;  // rows per pass
+    static constexpr int SB = WF_ ? NP_ * R * (WF_ + 1) : NP_ * 64 * WAVES_;  // floats per staging buffer
+    static constexpr bool XTT = IsXtt<KIND_>::value;
+    static constexpr int KM = XTT ? KM_ : 1;
+    static constexpr int NC = CX_ * CY_;
+    static constexpr int threads = 64 * WAVES_;
+    static constexpr int KP = XTT ? (KM_ + 3) & ~3 : 0;  // channel constants, padded for 16-byte LDS loads
+    // term words of one (view, column).  Untilted: Bc, Ac, fu, base, hi, lu, iu,
+    // wcol or cxy; tilted: nu, nv, nd, -, au2, av2, ad2, wcol or cxy; then ca[KP]
+    static constexpr int TW = 8 + KP;
+    static constexpr int term_area = kBwdBatch * NC * TW;  // words per wave
+    static constexpr int words = 2 * VB_ * SB + kBwdFootArea + WAVES_ * term_area;
+    // past these: WAVES words of per-wave max |voxel|, the persistent launch's item and ticket
+    static constexpr size_t lds_bytes = (words + WAVES_ + 2) * sizeof(float);
+    static_assert(NC == 1 || NC == 2 || NC == 4, "a term batch maps 4 lanes to a view");
+    static_assert(kBwdBatch % (2 * VB_) == 0 && VB_ % LOOK_ == 0, "whole groups per batch");
+};
+
+// The shapes that the persistent launches, the tile settings and large
+// standalone launches use.  The plain kinds (about 110 VGPRs, 4 waves per SIMD)
 // run one 16-wave block per CU; XTT runs 8-wave blocks, two per CU, so one
-// block accumulates while the other waits at its per-view barrier (its
-// footprints are small: 8 columns x 64 z).  Measured: XTT 150 against 167 ms
-// per backprojection at 256^3 x 13 coefficients, 4 x 360 views; the plain
-// kinds in 8-wave blocks (half the tile, 6144-float staging) 70 against 67 ms
-// at 512^3 / 720 views.
-// The untilted paths stage each view two views ahead in four buffers, so
-// that a block meets a barrier every second view; the general (tilted) path
-// double buffers in the first two.
+// block accumulates while the other waits at its barrier (its footprints are
+// small).  Measured with a barrier per view: XTT 150 against 167 ms per
+// backprojection at 256^3 x 13 coefficients, 4 x 360 views; the plain kinds in
+// 8-wave blocks (half the tile, 6144-float staging) 70 against 67 ms at 512^3 /
+// 720 views.
+template <int KIND, int ZPL, int KM>
+struct BwdLarge {
+    static constexpr bool XTT = IsXtt<KIND>::value;
+    typedef typename std::conditional<XTT, BwdCfg<KIND, 8, 1, 1, ZPL, KM, 2, 1, 8, 3>,
+                                      BwdCfg<KIND, 16, 2, 2, ZPL, 1, 2, 1, 16, 7>>::type Cfg;
+    typedef typename std::conditional<XTT, BwdCfg<KIND, 8, 1, 1, ZPL, KM, 2, 1, 0, 7>,
+                                      BwdCfg<KIND, 16, 2, 2, ZPL, 1, 2, 1, 0, 7>>::type Wide;
+};
+// Few tiles (small volumes): one column and 64 voxels per wave, eight views per
+// barrier.
 template <int KIND>
-struct BwdBlock {
-    static constexpr int waves = IsXtt<KIND>::value ? 8 : 16;
-    static constexpr int threads = 64 * waves;
-    static constexpr int nbuf = 4;                                      // staging buffers
-    static constexpr int stage_buf = IsXtt<KIND>::value ? 4000 : 8000;  // floats per staging buffer
-    static constexpr int stage_per = stage_buf / threads;              // staged floats per thread
+struct BwdSmall {
+    typedef BwdCfg<KIND, 8, 1, 1, 1, 1, 8, 8, 8, 2> Cfg;
 };
 
 struct Foot {
     int iu_lo, iv_lo, W, H, Ws, R;  // R: footprint rows staged per pass of the block's threads
-    bool staged, empty;
+    int flags;
 };
 
-template <int KIND>
-__device__ __forceinline__ Foot foot_from_extent(float umn, float umx, float vmn, float vmx, int bad, const Dims& d);
+// What staging a footprint needs: the buffer descriptor's base and range (0 where
+// the footprint is not staged: every load reads 0), the rows; any-width staging
+// also W, Ws and R.
+struct FootSrc {
+    unsigned lo, hi, range;
+    int H, W, Ws, R;
+};
 
-// Footprint of the block box on view g: the projective map's extremes over a box
-// are at its corners while den > 0 there (all lanes compute it identically).
-template <int KIND>
-__device__ __forceinline__ Foot footprint(const ViewGeom& g, const Dims& d, float bx0, float bx1, float by0, float by1,
-                                          float bz0, float bz1, int lane) {
-    const int ci = lane & 7;
-    float cu, cv, cd;
-    {
-        const ColForms c = col_forms(g, (ci & 1) ? bx1 : bx0, (ci & 2) ? by1 : by0);
-        const float czp = (ci & 4) ? bz1 : bz0;
-        cd = fmaf(g.ad[2], czp, c.nd);
-        voxel_uv(g, c, czp, d, cu, cv);
-    }
-    float umn = cu, umx = cu, vmn = cv, vmx = cv;
-    int bad = (!(cd > 0.f) || !(fabsf(cu) < 1e7f) || !(fabsf(cv) < 1e7f)) ? 1 : 0;
-    for (int off = 1; off < 8; off <<= 1) {
-        umn = fminf(umn, __shfl_xor(umn, off));
-        umx = fmaxf(umx, __shfl_xor(umx, off));
-        vmn = fminf(vmn, __shfl_xor(vmn, off));
-        vmx = fmaxf(vmx, __shfl_xor(vmx, off));
-        bad |= __shfl_xor(bad, off);
-    }
-    return foot_from_extent<KIND>(umn, umx, vmn, vmx, bad, d);
-}
-
-// Footprint from the extremes of the projected corners (bad: a corner behind
-// the source or far off the detector, so the extremes bound nothing).
-template <int KIND>
+// Footprint from the extremes of the tile's projected corners (bad: a corner
+// behind the source or far off the detector, so the extremes bound nothing).
+// INSIDE: every voxel of the tile lies in the acceptance window, with a margin
+// far above the rounding of u and v.
+template <class C>
 __device__ __forceinline__ Foot foot_from_extent(float umn, float umx, float vmn, float vmx, int bad, const Dims& d) {
-    Foot f{0, 0, 0, 0, 0, 0, false, false};
+    Foot f{0, 0, 0, 0, 0, 0, 0};
     if (bad) return f;  // direct (unstaged) reads
-    f.iu_lo = max((int)floorf(umn - 0.5f) - 1, 0);
-    const int iu_hi = min((int)floorf(umx - 0.5f) + 2, d.U - 1);
-    f.iv_lo = max((int)floorf(vmn - 0.5f) - 1, 0);
-    const int iv_hi = min((int)floorf(vmx - 0.5f) + 2, d.V - 1);
+    // texels iu and iu + 1 of every voxel, with a margin far above the rounding of u and v
+    f.iu_lo = max((int)floorf(umn - 0.51f), 0);
+    const int iu_hi = min((int)floorf(umx - 0.49f) + 1, d.U - 1);
+    f.iv_lo = max((int)floorf(vmn - 0.51f), 0);
+    const int iv_hi = min((int)floorf(vmx - 0.49f) + 1, d.V - 1);
     f.W = iu_hi - f.iu_lo + 1;
     f.H = iv_hi - f.iv_lo + 1;
     if (f.W <= 1 || f.H <= 1) {
-        f.empty = true;  // entirely off the detector: nothing is accepted
+        f.flags = FOOT_EMPTY;  // entirely off the detector: nothing is accepted
         return f;
     }
-    f.Ws = f.W | 1;
-    f.R = BwdBlock<KIND>::threads / f.W;
-    // the last word of the second buffer is reserved (work-queue ticket of the
-    // persistent launch), so a staged footprint holds at most stage_buf-1 floats
-    f.staged = (f.Ws * f.H <= BwdBlock<KIND>::stage_buf - 1) && (f.H <= BwdBlock<KIND>::stage_per * f.R);
+    f.Ws = C::WF ? C::WF + 1 : f.W | 1;
+    f.R = C::WF ? C::R : C::threads / f.W;
+    if ((C::WF ? f.W <= C::WF : f.Ws * f.H <= C::SB) && f.H <= C::NP * f.R) {
+        f.flags = FOOT_STAGED;
+        if (umn > 0.56f && umx < d.umax - 0.01f && vmn > 0.56f && vmx < d.vmax - 0.01f) f.flags |= FOOT_INSIDE;
+    }
     return f;
 }
 
@@ -1230,24 +1271,53 @@ __device__ __forceinline__ Foot foot_from_extent(float umn, float umx, float vmn
 // swizzle, stride 0): the range check is on the byte offset alone.
 constexpr int kBufferWord3 = 0x00020000;
 
-// Staging of one view's footprint (W x H texels at (iu_lo, iv_lo) of the
-// view's U-wide image) into an LDS buffer of row stride Ws, in passes of
-// R = threads / W rows: thread t owns column c = t % W of rows r0 + k R,
-// r0 = t / W (one division per view).  Only the passes the footprint needs
-// are issued and stored (uniform tests); only the last needs a per-lane row
-// test.  The LDS contents are those of a plain row-by-row copy.
-// BUF: a pass is one raw buffer load at a per-lane byte offset whose range is
-// the view's image, so a row below the image's last reads 0 (it lies outside
-// the footprint and is never stored): no address select, no predication, one
-// add per pass.  Otherwise (kernels whose scalar registers are already
-// scarce: the buffer descriptor takes four) a global load per pass, lanes
-// outside the footprint reading its first texel.
-template <int NP, bool BUF>
+// Staging of one view's footprint (W x H texels of the view's U-wide image,
+// whose first is the descriptor's base) into an LDS buffer of row stride Ws:
+// fetched into registers, stored later.  A pass is one raw buffer load at a
+// per-lane byte offset; its range ends with the image, so a row below the
+// image's last reads 0.
+// Fixed width: thread t owns column t % WF of rows t / WF + k R.  Its byte
+// offsets are the same for every view, and whole passes are loaded and stored:
+// columns past W (which may run into the next image row) and rows past H are
+// never read back.  (Up to two passes are issued without a look at H.)
+template <class C>
 struct FootStage {
-    float pre[NP];
+    float pre[C::NP];
+    unsigned voff;  // byte offset of the thread's first texel from the footprint's
+    int lds0;
+
+    __device__ __forceinline__ void init(int U) {
+        const int r0 = threadIdx.x / C::WF, c = threadIdx.x % C::WF;
+        voff = (unsigned)(r0 * U + c) * 4u;
+        lds0 = r0 * (C::WF + 1) + c;
+    }
+    __device__ __forceinline__ void fetch(const FootSrc& f, int U) {
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)(((uint64_t)f.hi << 32) | f.lo), (short)0,
+                                                            (int)f.range, kBufferWord3);
+        const unsigned step = (unsigned)(C::R * U) * 4u;
+#pragma unroll
+        for (int k = 0; k < C::NP; k++)
+            if (C::NP <= 2 || k * C::R < f.H)
+                pre[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff + k * step, 0, 0));
+    }
+    __device__ __forceinline__ void store(lds_float* buf, const FootSrc& f) const {
+#pragma unroll
+        for (int k = 0; k < C::NP; k++)
+            if (C::NP <= 2 || k * C::R < f.H) buf[lds0 + k * C::R * (C::WF + 1)] = pre[k];
+    }
+};
+
+// Any width: passes of R = threads / W rows, thread t owning column t % W of
+// rows r0 + k R, r0 = t / W (one division per view).  Only the passes the
+// footprint needs are issued and stored (uniform tests); only the last needs a
+// per-lane row test.
+template <class C>
+struct FootStageAny {
+    float pre[C::NP];
     int r0, lds0;  // lds0 = r0 Ws + c; r0 >= R: the thread stages nothing
 
-    __device__ __forceinline__ void fetch(const float* img, int img_bytes, const Foot& f, int U) {
+    __device__ __forceinline__ void init(int) {}
+    __device__ __forceinline__ void fetch(const FootSrc& f, int U) {
         r0 = (int)((float)threadIdx.x * rcpf((float)f.W));  // within 1 of t / W: corrected below
         int c = (int)threadIdx.x - r0 * f.W;
         if (c < 0) {
@@ -1258,39 +1328,23 @@ struct FootStage {
             c -= f.W;
         }
         lds0 = r0 * f.Ws + c;
-        if constexpr (BUF) {
-            // the image (one view's, the same for the whole block) in scalar
-            // registers, as a buffer descriptor must be
-            const uint64_t ip = (uint64_t)(uintptr_t)img;
-            const uint64_t up = ((uint64_t)(unsigned)uniformi((int)(ip >> 32)) << 32) | (unsigned)uniformi((int)ip);
-            const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)up, (short)0, uniformi(img_bytes),
-                                                                kBufferWord3);
-            unsigned voff = ((unsigned)(f.iv_lo + r0) * (unsigned)U + (unsigned)(f.iu_lo + c)) * 4u;
-            // opaque to the optimiser, so that pass k adds the uniform k * step
-            // (one add) instead of recomputing (row + k R) * U (a quarter-rate multiply)
-            asm volatile("" : "+v"(voff));
-            const unsigned step = (unsigned)f.R * (unsigned)U * 4u;
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)(((uint64_t)f.hi << 32) | f.lo), (short)0,
+                                                            (int)f.range, kBufferWord3);
+        unsigned voff = ((unsigned)r0 * (unsigned)U + (unsigned)c) * 4u;
+        // opaque to the optimiser, so that pass k adds the uniform k * step
+        // (one add) instead of recomputing (row + k R) * U (a quarter-rate multiply)
+        asm volatile("" : "+v"(voff));
+        const unsigned step = (unsigned)f.R * (unsigned)U * 4u;
 #pragma unroll
-            for (int k = 0; k < NP; k++)
-                if (k * f.R < f.H)
-                    pre[k] =
-                        __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff + k * step, 0, 0));
-        } else {
-            const auto g = to_global(img);
-            const bool act = r0 < f.R;
-            const auto src = g + (int64_t)(f.iv_lo + r0) * U + f.iu_lo + c;
-            const auto safe = g + (int64_t)f.iv_lo * U + f.iu_lo;  // inside the image
-            const int64_t step = (int64_t)f.R * U;
-#pragma unroll
-            for (int k = 0; k < NP; k++)
-                if (k * f.R < f.H) pre[k] = *((act && r0 + k * f.R < f.H) ? src + k * step : safe);
-        }
+        for (int k = 0; k < C::NP; k++)
+            if (k * f.R < f.H)
+                pre[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff + k * step, 0, 0));
     }
-    __device__ __forceinline__ void store(lds_float* buf, const Foot& f) const {
+    __device__ __forceinline__ void store(lds_float* buf, const FootSrc& f) const {
         if (r0 >= f.R) return;
         const int rs = f.R * f.Ws;
 #pragma unroll
-        for (int k = 0; k < NP; k++) {
+        for (int k = 0; k < C::NP; k++) {
             if ((k + 1) * f.R <= f.H)
                 buf[lds0 + k * rs] = pre[k];
             else if (k * f.R < f.H && r0 + k * f.R < f.H)
@@ -1307,47 +1361,43 @@ struct FootStage {
 // fixed-point scale from it.  A tile skipped for any reason (say, outside the
 // field of view) would leave that bound too small.  (Layers z >= nz are not
 // visited; a plan sets nz < N only where those layers are held at zero.)
-template <int KIND, int CPW, int ZPL, int KA>
-__device__ __forceinline__ float backward_update(const BwdArgs& a, const float (&tmp)[CPW * CPW][ZPL][KA],
-                                                 const float (&fac)[CPW * CPW][ZPL][KA], const int (&nwhole)[CPW * CPW],
+template <class C>
+__device__ __forceinline__ float backward_update(const BwdArgs& a, const float (&tmp)[C::NC][C::ZPL][C::KM],
+                                                 const float (&fac)[C::NC][C::ZPL][C::KM], const int (&nwhole)[C::NC],
                                                  int xb, int yb, int z0, int lane) {
     // returns max |updated voxel| of this lane (MLEM / ART kinds)
-    constexpr bool XTT = IsXtt<KIND>::value;
+    constexpr int KIND = C::KIND;
     const Dims& d = a.d;
     const auto vol = to_global(a.vol);
     float vmx = 0.f;
 #pragma unroll
-    for (int j = 0; j < CPW; j++) {
+    for (int cidx = 0; cidx < C::NC; cidx++) {
+        const int x = xb + cidx % C::CX, y = yb + cidx / C::CX;
+        if (x >= d.N || y >= d.N) continue;
 #pragma unroll
-        for (int i = 0; i < CPW; i++) {
-            const int x = xb + i, y = yb + j;
-            if (x >= d.N || y >= d.N) continue;
-            const int cidx = j * CPW + i;
+        for (int q = 0; q < C::ZPL; q++) {
+            const int z = z0 + lane + 64 * q;
+            if (z >= d.N) continue;
+            const int64_t idx = ((int64_t)y * d.N + x) * d.N + z;
 #pragma unroll
-            for (int q = 0; q < ZPL; q++) {
-                const int z = z0 + lane + 64 * q;
-                if (z >= d.N) continue;
-                const int64_t idx = ((int64_t)y * d.N + x) * d.N + z;
-#pragma unroll
-                for (int k = 0; k < KA; k++) {
-                    if (XTT && k >= d.K) continue;
-                    const int64_t vi = idx + (int64_t)k * a.chan_stride;
-                    const float t = tmp[cidx][q][k], fc = fac[cidx][q][k] + (float)nwhole[cidx];
-                    if (KIND == BWD_RAW || KIND == BWD_XTT_RAW) {
-                        to_global(a.tmp)[vi] += t;
-                        to_global(a.factor)[vi] += fc;
-                    } else if (KIND == BWD_MLEM || KIND == BWD_XTT_MLEM) {
-                        const float mu = vol[vi];
-                        const float nv = (fc == 0.0f) ? 0.0f : mu * t / fc;
-                        vol[vi] = nv;
-                        vmx = fmaxf(vmx, fabsf(nv));
-                    } else if (KIND == BWD_ART || KIND == BWD_XTT_ART) {
-                        const float nv = vol[vi] + a.alpha * t;
-                        vol[vi] = nv;
-                        vmx = fmaxf(vmx, fabsf(nv));
-                    } else {  // BWD_FDK
-                        vol[vi] = a.overwrite ? t : vol[vi] + t;
-                    }
+            for (int k = 0; k < C::KM; k++) {
+                if (C::XTT && k >= d.K) continue;
+                const int64_t vi = idx + (int64_t)k * a.chan_stride;
+                const float t = tmp[cidx][q][k], fc = fac[cidx][q][k] + (float)nwhole[cidx];
+                if (KIND == BWD_RAW || KIND == BWD_XTT_RAW) {
+                    to_global(a.tmp)[vi] += t;
+                    to_global(a.factor)[vi] += fc;
+                } else if (KIND == BWD_MLEM || KIND == BWD_XTT_MLEM) {
+                    const float mu = vol[vi];
+                    const float nv = (fc == 0.0f) ? 0.0f : mu * t / fc;
+                    vol[vi] = nv;
+                    vmx = fmaxf(vmx, fabsf(nv));
+                } else if (KIND == BWD_ART || KIND == BWD_XTT_ART) {
+                    const float nv = vol[vi] + a.alpha * t;
+                    vol[vi] = nv;
+                    vmx = fmaxf(vmx, fabsf(nv));
+                } else {  // BWD_FDK
+                    vol[vi] = a.overwrite ? t : vol[vi] + t;
                 }
             }
         }
@@ -1355,77 +1405,76 @@ __device__ __forceinline__ float backward_update(const BwdArgs& a, const float (
     return vmx;
 }
 
-// ---------------------------------------------------------------------------
-// Untilted backprojection of the plain kinds (raw, MLEM, ART, FDK).  The
-// per-view quantities of a wave are the same in all its lanes: the block
-// footprint (8 projected corners) and, for each of the wave's 4 columns, the
-// column's u split, the affine t(z) = v - 0.5 and the acceptance window.  They
-// are computed lane-parallel, 16 views at a time, into LDS: the footprints of
-// a batch by wave 0 (lane = view x corner pair, published by the per-view
-// barrier two views before the batch starts), the column terms by every wave
-// for its own columns (lane = view x column).  The view loop reads them back
-// with broadcast LDS loads.  Arithmetic and accumulation order are those of
-// the general path, so results are bitwise the same.
-// ---------------------------------------------------------------------------
-constexpr int kBwdBatch = 16;    // views per batch of per-view terms
-constexpr int kFootWords = 8;    // iu_lo, iv_lo, W, H, Ws, R, staged | empty << 1, -
-constexpr int kTermWords = 8;    // Bc, Ac, fu, hi (+inf: whole z extent accepted), wcol, lu, iu, base
-constexpr int kTermCols = 4;     // columns per wave (CPW = 2)
-constexpr int kBwdFootArea = 2 * kBwdBatch * kFootWords;          // words, block-wide, two batches
-constexpr int kBwdTermArea = kBwdBatch * kTermCols * kTermWords;  // words per wave
-template <int KIND>
-constexpr int bwd_extra_words() {
-    return kBwdFootArea + BwdBlock<KIND>::waves * kBwdTermArea;
-}
-static_assert(64 % kTermCols == 0 && 64 / kTermCols >= kBwdBatch, "one lane per (view, column) of a batch");
-
-typedef __attribute__((address_space(3))) int lds_int;
-
-template <int KIND, int ZPL>
-__device__ __forceinline__ float backward_item_untilted(const BwdArgs& a, int o, int step, float* stage) {
-    constexpr int CPW = 2, NC = CPW * CPW;
-    static_assert(NC == kTermCols, "term layout");
+// One voxel tile o of a backprojection launch; step selects the view list
+// views + step*n_views (a solver's subset step).  stage: the block's LDS.
+// Returns the lane's max |updated voxel| (MLEM / ART kinds).
+//
+// Untilted views: u, hence (iu, fu), is constant along a column, the bilinear
+// weights factor into (1-fu, fu) x (1-fv, fv), and t = v - 0.5 is affine in z.
+// The acceptance window 0.55 < u, v < U, V - 0.55 becomes 0.05 < t < hi (hi < 0
+// rejects the column).  A column whose whole z extent is accepted (t at the
+// tile's first and last z bounds every lane's t: fmaf is monotone in z) runs
+// without tests and counts once for all its voxels.
+// Tilted views: (u, v) per voxel by col_forms and voxel_uv; a tile that lies
+// inside the window (FOOT_INSIDE) runs without tests.
+// XTT: per channel w_k = g2s_k - q_k^2/|d|^2 with q_k = dz sig_k S_k,z + ca_k
+// (ir.cu:1832-1840), ca_k = sig_k (d_x S_k,x + d_y S_k,y) among the column
+// terms; sig_k S_k,z and g2s_k are scalar loads of the plan's weight table.
+// Channels k >= K have zero constants (table padding) and are never stored.
+template <class C, bool TILT>
+__device__ __forceinline__ float backward_item(const BwdArgs& a, int o, int step, float* stage) {
+    constexpr int KIND = C::KIND, NC = C::NC, ZPL = C::ZPL, KM = C::KM, VB = C::VB, SB = C::SB, TW = C::TW;
+    constexpr bool XTT = C::XTT;
+    constexpr int xws = kXwStride;  // >= KM: whole rows, zero padded
     const Dims& d = a.d;
     const auto views = to_global(a.views + (int64_t)step * a.n_views);
     const auto vg = to_global(a.vg);
+    const auto vgc = to_const(a.vg);
     const int gx = a.gx;
-    const int bcx = CPW * gx, bcy = CPW * a.gy;  // block columns along x, y
+    const int bcx = C::CX * gx, bcy = C::CY * a.gy;  // block columns along x, y
     const int tx = o % a.tiles_x, ty = (o / a.tiles_x) % a.tiles_y, tz = o / (a.tiles_x * a.tiles_y);
     // the wave index as a wave-uniform value: the column tests and counts below stay scalar
     const int lane = threadIdx.x & 63, wave = uniformi(threadIdx.x >> 6);
-    const int xb = tx * bcx + (wave % gx) * CPW, yb = ty * bcy + (wave / gx) * CPW;
+    const int xb = tx * bcx + (wave % gx) * C::CX, yb = ty * bcy + (wave / gx) * C::CY;
     const int z0 = tz * 64 * ZPL;
+    const int z_last = min(z0 + 64 * ZPL, d.N) - 1;  // the tile's last z
     const float bx0 = (float)(tx * bcx) - d.xc, bx1 = (float)min(tx * bcx + bcx - 1, d.N - 1) - d.xc;
     const float by0 = (float)(ty * bcy) - d.xc, by1 = (float)min(ty * bcy + bcy - 1, d.N - 1) - d.xc;
-    const float bz0 = (float)z0 - d.xc, bz1 = (float)min(z0 + 64 * ZPL - 1, d.N - 1) - d.xc;
+    const float bz0 = (float)z0 - d.xc, bz1 = (float)z_last - d.xc;
     const int nv = a.n_views;
     if (nv == 0) return 0.f;
+    const int64_t img_len = (int64_t)d.V * d.U;
 
-    float tmp[NC][ZPL][1], fac[NC][ZPL][1];
+    float tmp[NC][ZPL][KM], fac[NC][ZPL][KM];
 #pragma unroll
     for (int c = 0; c < NC; c++)
 #pragma unroll
-        for (int q = 0; q < ZPL; q++) {
-            tmp[c][q][0] = 0.f;
-            fac[c][q][0] = 0.f;
-        }
+        for (int q = 0; q < ZPL; q++)
+#pragma unroll
+            for (int k = 0; k < KM; k++) {
+                tmp[c][q][k] = 0.f;
+                fac[c][q][k] = 0.f;
+            }
     int nwhole[NC];  // views accepting a column's whole z extent (added to the counts at the end)
 #pragma unroll
     for (int c = 0; c < NC; c++) nwhole[c] = 0;
+    // lanes past the volume's end repeat its last voxel (never stored), so that
+    // they neither leave the footprint nor fail a column's whole-extent test
     float zpq[ZPL];
 #pragma unroll
-    for (int q = 0; q < ZPL; q++) zpq[q] = (float)(z0 + lane + 64 * q) - d.xc;
+    for (int q = 0; q < ZPL; q++) zpq[q] = (float)min(z0 + lane + 64 * q, z_last) - d.xc;
 
     lds_float* const lds = (lds_float*)stage;
-    lds_int* const foot = (lds_int*)(stage + BwdBlock<KIND>::nbuf * BwdBlock<KIND>::stage_buf);
-    lds_float* const term =
-        (lds_float*)(stage + BwdBlock<KIND>::nbuf * BwdBlock<KIND>::stage_buf + kBwdFootArea + wave * kBwdTermArea);
+    lds_int* const foot = (lds_int*)(stage + 2 * VB * SB);
+    lds_float* const term = (lds_float*)(stage + 2 * VB * SB + kBwdFootArea + wave * C::term_area);
 
     // footprints of views b0 .. b0+15 into buffer buf: lane = 4 x view + corner
     // pair (x, y corner; both z corners), extremes over the 4 lanes of a view
-    auto foot_batch = [&](int b0, int buf) {
+    // (the projective map's extremes over a box are at its corners while den > 0 there)
+    auto foot_batch = [&](int b0, int buf) XR_INLINE {
         const int j = lane >> 2, c = lane & 3;
-        const ViewGeom g = vg[views[min(b0 + j, nv - 1)]];
+        const int code = views[min(b0 + j, nv - 1)];
+        const ViewGeom g = vg[code];
         const ColForms cf = col_forms(g, (c & 1) ? bx1 : bx0, (c & 2) ? by1 : by0);
         float umn = 0.f, umx = 0.f, vmn = 0.f, vmx = 0.f;
         int bad = 0;
@@ -1448,49 +1497,55 @@ __device__ __forceinline__ float backward_item_untilted(const BwdArgs& a, int o,
             vmx = fmaxf(vmx, __shfl_xor(vmx, off));
             bad |= __shfl_xor(bad, off);
         }
-        const Foot f = foot_from_extent<KIND>(umn, umx, vmn, vmx, bad, d);
+        const Foot f = foot_from_extent<C>(umn, umx, vmn, vmx, bad, d);
         if (c == 0) {
             lds_int* p = foot + (buf * kBwdBatch + j) * kFootWords;
             p[0] = f.iu_lo;
             p[1] = f.iv_lo;
             p[2] = f.W;
-            p[3] = f.H;
-            p[4] = f.Ws;
-            p[5] = f.R;
-            p[6] = (f.staged ? 1 : 0) | (f.empty ? 2 : 0);
+            p[3] = f.Ws | (f.R << 16);
+            p[4] = f.flags;
+            p[5] = code;
+            const bool staged = (f.flags & FOOT_STAGED) != 0;
+            const int64_t first = (int64_t)f.iv_lo * d.U + f.iu_lo;
+            const uint64_t at = (uint64_t)(uintptr_t)(a.proj + (int64_t)(code - a.code_base) * img_len + first);
+            p[8] = (int)(unsigned)at;
+            p[9] = (int)(unsigned)(at >> 32);
+            p[10] = staged ? (int)((img_len - first) * 4) : 0;
+            p[11] = staged ? f.H : 0;
         }
     };
-    auto load_foot = [&](int buf, int j) {
-        const lds_int* p = foot + (buf * kBwdBatch + j) * kFootWords;
-        Foot f;
-        f.iu_lo = uniformi(p[0]);
-        f.iv_lo = uniformi(p[1]);
-        f.W = uniformi(p[2]);
-        f.H = uniformi(p[3]);
-        f.Ws = uniformi(p[4]);
-        f.R = uniformi(p[5]);
-        const int fl = uniformi(p[6]);
-        f.staged = (fl & 1) != 0;
-        f.empty = (fl & 2) != 0;
+    auto foot_of = [&](int v) XR_INLINE { return foot + (((v / kBwdBatch) & 1) * kBwdBatch + (v & (kBwdBatch - 1))) * kFootWords; };
+    auto load_src = [&](int v) XR_INLINE {
+        const lds_int* p = foot_of(v);
+        FootSrc f;
+        f.lo = (unsigned)uniformi(p[8]);
+        f.hi = (unsigned)uniformi(p[9]);
+        f.range = (unsigned)uniformi(p[10]);
+        f.H = uniformi(p[11]);
+        f.W = f.Ws = f.R = 0;
+        if (C::WF == 0) {
+            const int w = uniformi(p[3]);
+            f.W = uniformi(p[2]);
+            f.Ws = w & 0xffff;
+            f.R = w >> 16;
+        }
         return f;
     };
-    // column terms of views b0 .. b0+15 for this wave's columns: lane = 4 x view + column
-    auto term_batch = [&](int b0, int buf) {
-        const int j = lane >> 2, cidx = lane & 3;
-        const ViewGeom g = vg[views[min(b0 + j, nv - 1)]];
-        const lds_int* fp = foot + (buf * kBwdBatch + j) * kFootWords;
-        const int iu_lo = fp[0], iv_lo = fp[1], W = fp[2], Ws = fp[4], fl = fp[6];
-        const float xp = (float)(xb + (cidx & 1)) - d.xc, yp = (float)(yb + (cidx >> 1)) - d.xc;
+    unsigned long long wholes = 0;
+    // column terms of views b0 .. b0+15 for this wave's columns: lane = 4 x view
+    // + column (plain) or channel quarter (XTT)
+    auto term_batch = [&](int b0) XR_INLINE {
+        const int j = lane >> 2, p = lane & 3;
+        const lds_int* fp = foot_of(b0 + j);
+        const int code = fp[5];
+        const ViewGeom g = vg[code];
+        const int iu_lo = fp[0], iv_lo = fp[1], W = fp[2], Ws = fp[3] & 0xffff, fl = fp[4];
+        const int cidx = XTT ? 0 : (p & (NC - 1));
+        const float xp = (float)(xb + cidx % C::CX) - d.xc, yp = (float)(yb + cidx / C::CX) - d.xc;
         const ColForms c = col_forms(g, xp, yp);
-        const float inv_c = rcpf(c.nd);
-        const float u_c = fmaf(c.nu, inv_c, d.hu);
-        int iu;
-        float fu;
-        split(u_c, iu, fu);
-        const float Bc = g.av[2] * inv_c;
-        const float Ac = fmaf(c.nv, inv_c, d.hv - 0.5f);
-        const float hi = accept_u(u_c, d) ? d.vmax - 0.5f : -1.0f;
-        const int lu = min(max(iu - iu_lo, 0), W - 2);
+        lds_float* tp = term + (j * NC + cidx) * TW;
+        lds_int* ti = (lds_int*)tp;
         float wcol = 0.f;
         if (KIND == BWD_FDK) {
             // vol += Ud^2 * (2 pi/P) * sum c p, Ud = sod/(sod + y_unrotated) (fdk.cu:160-169)
@@ -1498,21 +1553,58 @@ __device__ __forceinline__ float backward_item_untilted(const BwdArgs& a, int o,
             const float Ud = d.sod / (d.sod + Xy);
             wcol = Ud * Ud * d.cfdk;
         }
-        // whole extent accepted: t at the tile's first and last z bound every
-        // lane's t (fmaf is monotone in z)
-        const float ta = fmaf(Bc, bz0, Ac);
-        const float tb = fmaf(Bc, (float)(z0 + 64 * ZPL - 1) - d.xc, Ac);
-        const bool whole = (fl & 1) && fminf(ta, tb) > 0.05f && fmaxf(ta, tb) < hi;
-        lds_float* tp = term + (j * kTermCols + cidx) * kTermWords;
-        lds_int* ti = (lds_int*)tp;
-        tp[0] = Bc;
-        tp[1] = Ac;
-        tp[2] = fu;
-        tp[3] = whole ? __int_as_float(0x7f800000) : hi;
-        tp[4] = wcol;
-        ti[5] = lu;
-        ti[6] = iu;
-        ti[7] = (lu - iv_lo * Ws) * 4;  // LDS byte offset of texel (iu, 0) in a staging buffer
+        if (XTT) {
+            const float dx = fmaf(d.vs, xp, g.d0[0]);
+            const float dy = fmaf(d.vs, yp, g.d0[1]);
+            wcol = fmaf(dy, dy, dx * dx);
+        }
+        bool whole = false;
+        if (XTT ? p == 0 : p < NC) {
+            tp[7] = wcol;
+            if (TILT) {
+                tp[0] = c.nu;
+                tp[1] = c.nv;
+                tp[2] = c.nd;
+                tp[4] = g.au[2];
+                tp[5] = g.av[2];
+                tp[6] = g.ad[2];
+                whole = (fl & FOOT_INSIDE) != 0;
+            } else {
+                const float inv_c = rcpf(c.nd);
+                const float u_c = fmaf(c.nu, inv_c, d.hu);
+                int iu;
+                float fu;
+                split(u_c, iu, fu);
+                const float Bc = g.av[2] * inv_c;
+                const float Ac = fmaf(c.nv, inv_c, d.hv - 0.5f);
+                const float hi = (accept_u(u_c, d) && !(fl & FOOT_EMPTY)) ? d.vmax - 0.5f : -1.0f;
+                const int lu = min(max(iu - iu_lo, 0), W - 2);
+                const float ta = fmaf(Bc, bz0, Ac), tb = fmaf(Bc, bz1, Ac);
+                whole = (fl & FOOT_STAGED) && fminf(ta, tb) > 0.05f && fmaxf(ta, tb) < hi;
+                tp[0] = Bc;
+                tp[1] = Ac;
+                tp[2] = fu;
+                ti[3] = (lu - iv_lo * Ws) * 4;  // LDS byte offset of texel (iu, 0) in a staging buffer
+                tp[4] = hi;
+                ti[5] = lu;
+                ti[6] = iu;
+            }
+        }
+        // bit 4 j + c: column c's whole extent is accepted in view b0 + j
+        wholes = __ballot(whole);
+        if (KIND != BWD_FDK && !XTT) {
+            const unsigned long long seen = nv - b0 >= kBwdBatch ? ~0ull : (1ull << (4 * (nv - b0))) - 1;
+#pragma unroll
+            for (int c = 0; c < NC; c++) nwhole[c] += __popcll(wholes & seen & (0x1111111111111111ull << c));
+        }
+        if constexpr (XTT) {
+            const auto row = to_global(a.xw + (int64_t)code * 5 * xws);
+#pragma unroll
+            for (int m = 0; m < C::KP / 4; m++) {
+                const int k = p + 4 * m;
+                tp[8 + k] = fmaf(xp, row[2 * xws + k], fmaf(yp, row[3 * xws + k], row[4 * xws + k]));  // 0 for k >= K
+            }
+        }
     };
     // a wave's own LDS writes, then its lanes read each other's words
     auto wave_sync = [] {
@@ -1521,382 +1613,59 @@ __device__ __forceinline__ float backward_item_untilted(const BwdArgs& a, int o,
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
 
-    // staging of one view's footprint: prefetch into registers, store later
-    FootStage<BwdBlock<KIND>::stage_per, true> st;
-    const int img_bytes = d.V * d.U * 4;
-    auto fetch = [&](const Foot& f, int code) {
-        st.fetch(a.proj + (int64_t)(code - a.code_base) * d.V * d.U, img_bytes, f, d.U);
+    // staging: view v in buffer v % (2 VB); fetched into registers a group
+    // ahead, stored into a buffer whose last reads (view v - 2 VB) a barrier has
+    // followed, read after the barrier that ends the group
+    typename std::conditional<(C::WF > 0), FootStage<C>, FootStageAny<C>>::type st[C::LOOK];
+#pragma unroll
+    for (int i = 0; i < C::LOOK; i++) st[i].init(d.U);
+    FootSrc kept[C::LOOK];  // fetched and not yet stored
+    auto fetch = [&](int v, int i) XR_INLINE {
+        kept[i] = load_src(v);
+        st[i].fetch(kept[i], d.U);
     };
+    auto store = [&](int v, int i) XR_INLINE { st[i].store(lds + (v & (2 * VB - 1)) * SB, kept[i]); };
 
-    // View v is staged in buffer v % 4 two views ahead (fetched into registers
-    // during view v-2, stored after it) and the block meets a barrier after
-    // every odd view.  A store into buffer v % 4 then follows, across at least
-    // one barrier, the last reads of view v-4 there, and precedes the reads of
-    // view v across one; footprint batches are written four views ahead.
-    static_assert(BwdBlock<KIND>::nbuf == 4, "four staging buffers");
-    constexpr int SB = BwdBlock<KIND>::stage_buf;
-    if (wave == 0) foot_batch(0, 0);
-    __syncthreads();
-    term_batch(0, 0);
-    int code = views[0], code1 = 0;
-    Foot f = load_foot(0, 0), f1{0, 0, 0, 0, 0, 0, false, false};
-    if (f.staged) {
-        fetch(f, code);
-        st.store(lds, f);
-    }
-    if (nv > 1) {
-        code1 = views[1];
-        f1 = load_foot(0, 1);
-        if (f1.staged) {
-            fetch(f1, code1);
-            st.store(lds + SB, f1);
-        }
-    }
-    __syncthreads();
-
-    for (int s = 0; s < nv; s++) {
-        const int j = s & (kBwdBatch - 1);
-        if (j == 0 && s > 0) term_batch(s, (s / kBwdBatch) & 1);
-        wave_sync();
-        // the footprints of the batch after this one: read from view s + 2 on
-        if (wave == 0 && j == kBwdBatch - 4 && s + 4 < nv) foot_batch(s + 4, ((s + 4) / kBwdBatch) & 1);
-        lds_float* cur = lds + (s & 3) * SB;
-        lds_float* nxt = lds + ((s + 2) & 3) * SB;
-        int ncode = 0;
-        Foot nf{0, 0, 0, 0, 0, 0, false, false};
-        if (s + 2 < nv) {
-            ncode = views[s + 2];
-            nf = load_foot(((s + 2) / kBwdBatch) & 1, (s + 2) & (kBwdBatch - 1));
-            if (nf.staged) fetch(nf, ncode);
-        }
-        if (!f.empty) {
-            const auto img = to_global(a.proj + (int64_t)(code - a.code_base) * d.V * d.U);
+    // Accumulation of the samples nb of column cidx (view s).  all: every voxel
+    // accepted (and counted with the column); otherwise an accepted voxel counts `one`.
+    auto accumulate = [&](int s, int cidx, const lds_float* tp, const float (&nb)[ZPL], const bool (&ok)[ZPL],
+                          auto all_c, float one) XR_INLINE {
+        constexpr bool all = decltype(all_c)::value;
+        if constexpr (!XTT) {
 #pragma unroll
-            for (int cidx = 0; cidx < NC; cidx++) {
-                const int x = xb + (cidx & 1), y = yb + (cidx >> 1);
-                if (x >= d.N || y >= d.N) continue;
-                const lds_float* tp = term + (j * kTermCols + cidx) * kTermWords;
-                const lds_int* ti = (const lds_int*)tp;
-                const float Bc = tp[0], Ac = tp[1], fu = tp[2], hi = tp[3], wcol = tp[4];
-                const int lu = ti[5], iu = ti[6], boff = ti[7];
-                const float a0 = 1.0f - fu;
-                // the column's samples; both branches leave them in nbq and the
-                // accumulation after them is shared, so the accumulators are
-                // updated in place (no copies where the branches meet)
-                float nbq[ZPL];
-                if (uniformi(__float_as_int(hi)) == 0x7f800000) {
-                    // all reads of the column first (LDS latency), then the sums
-                    const unsigned ws4 = (unsigned)f.Ws * 4u;
-                    const unsigned base = (unsigned)(uintptr_t)cur + (unsigned)boff;
-                    float fv[ZPL], r[ZPL][4];
-#pragma unroll
-                    for (int q = 0; q < ZPL; q++) {
-                        const float t = fmaf(Bc, zpq[q], Ac);
-                        fv[q] = __builtin_amdgcn_fractf(t);
-                        const unsigned at = __umul24((unsigned)floor_int(t), ws4) + base;
-                        const lds_float* p0 = (const lds_float*)(uintptr_t)at;
-                        const lds_float* p1 = (const lds_float*)(uintptr_t)(at + ws4);
-                        r[q][0] = p0[0];
-                        r[q][1] = p0[1];
-                        r[q][2] = p1[0];
-                        r[q][3] = p1[1];
-                    }
-#pragma unroll
-                    for (int q = 0; q < ZPL; q++) {
-                        const float top = fmaf(fu, r[q][1], a0 * r[q][0]);
-                        const float bot = fmaf(fu, r[q][3], a0 * r[q][2]);
-                        nbq[q] = fmaf(fv[q], bot - top, top);
-                    }
-                    if (KIND != BWD_FDK) nwhole[cidx]++;
+            for (int q = 0; q < ZPL; q++) {
+                if (KIND == BWD_FDK) {
+                    tmp[cidx][q][0] = fmaf(tp[7], nb[q], tmp[cidx][q][0]);
                 } else {
-                    // Window test per voxel: 0.55 < v < V - 0.55 becomes 0.05 < t < hi
-                    // (hi < 0 rejects the column).  Branch free: a rejected voxel reads
-                    // an in-bounds texel and adds zero.  Lanes with z >= N accumulate
-                    // but are never stored.
-#pragma unroll
-                    for (int q = 0; q < ZPL; q++) {
-                        const float t = fmaf(Bc, zpq[q], Ac);
-                        const bool ok = t > 0.05f && t < hi;
-                        const float fl = floorf(t);
-                        const float fv = t - fl;
-                        const int iv = (int)fl;
-                        float r00, r01, r10, r11;
-                        if (f.staged) {
-                            const int qi = (ok ? iv - f.iv_lo : 0) * f.Ws + lu;
-                            r00 = cur[qi];
-                            r01 = cur[qi + 1];
-                            r10 = cur[qi + f.Ws];
-                            r11 = cur[qi + f.Ws + 1];
-                        } else {
-                            // direct reads: a distinct (nontemporal) load form next to the LDS reads
-                            const int64_t qi = (int64_t)min(max(iv, 0), d.V - 2) * d.U + min(max(iu, 0), d.U - 2);
-                            r00 = __builtin_nontemporal_load(img + qi);
-                            r01 = __builtin_nontemporal_load(img + qi + 1);
-                            r10 = __builtin_nontemporal_load(img + qi + d.U);
-                            r11 = __builtin_nontemporal_load(img + qi + d.U + 1);
-                        }
-                        const float top = fmaf(fu, r01, a0 * r00);
-                        const float bot = fmaf(fu, r11, a0 * r10);
-                        nbq[q] = ok ? fmaf(fv, bot - top, top) : 0.0f;
-                        if (KIND != BWD_FDK) fac[cidx][q][0] += ok ? 1.0f : 0.0f;
-                    }
+                    tmp[cidx][q][0] += nb[q];
+                    if (!all) fac[cidx][q][0] += ok[q] ? one : 0.0f;
                 }
+            }
+        } else {
+            const int code = uniformi(foot_of(s)[5]);
+            const float cxy = tp[7], d0z = vgc[code].d0[2];
+            if (TILT && a.coef) {
+                // backwardOrth: the basis rotated per voxel
+                const ViewGeom& g = a.vg[code];
+                const float dx = fmaf(d.vs, (float)xb - d.xc, g.d0[0]), dy = fmaf(d.vs, (float)yb - d.xc, g.d0[1]);
 #pragma unroll
                 for (int q = 0; q < ZPL; q++) {
-                    if (KIND == BWD_FDK)
-                        tmp[cidx][q][0] = fmaf(wcol, nbq[q], tmp[cidx][q][0]);
-                    else
-                        tmp[cidx][q][0] += nbq[q];
+                    if (!all && !ok[q]) continue;
+                    const float dz = fmaf(d.vs, zpq[q], d0z);
+                    const float id2 = rcpf(fmaf(dz, dz, cxy));
+                    const int64_t vi = ((int64_t)yb * d.N + xb) * d.N + (int)(zpq[q] + d.xc);
+                    float R[9];
+                    orth_rotation(a.coef[vi], a.coef[vi + a.chan_stride], R);
+#pragma unroll
+                    for (int k = 0; k < KM; k++)
+                        if (k < d.K) {
+                            const float w = orth_weight(R, a.b, k, dx, dy, dz, id2, g);
+                            tmp[cidx][q][k] = fmaf(w, nb[q], tmp[cidx][q][k]);
+                            fac[cidx][q][k] += w;
+                        }
                 }
+                return;
             }
-        }
-        if (s + 2 < nv && nf.staged) st.store(nxt, nf);
-        code = code1;
-        f = f1;
-        code1 = ncode;
-        f1 = nf;
-        if (s & 1) __syncthreads();
-    }
-    return backward_update<KIND, CPW, ZPL, 1>(a, tmp, fac, nwhole, xb, yb, z0, lane);
-}
-
-// ---------------------------------------------------------------------------
-// Untilted XTT backprojection.  A wave owns one column and ZPL voxels per lane
-// in each of its K channels.  Per view and voxel the work is the bilinear
-// gather, dz and 1/|d|^2, then per channel w_k = g2s_k - q_k^2/|d|^2 with
-// q_k = dz sig_k S_k,z + ca_k (ir.cu:1832-1840) and two accumulations.
-// Everything else is the same for all lanes of a wave and is computed
-// lane-parallel 16 views at a time, as in the plain untilted path: the block
-// footprints by wave 0 (lane = view x corner pair), the column terms and the
-// K column constants ca_k = sig_k (d_x S_k,x + d_y S_k,y) by every wave for
-// its own column (lane = view x channel quarter), all into LDS; the view loop
-// reads them back with broadcast LDS loads.  The view's sig_k S_k,z and g2s_k
-// are scalar loads of the plan's weight table.  Footprints are staged in
-// LDS two views ahead in four buffers, with as many fetch passes as the
-// footprint needs (at most kXttStagePer; a taller one is read from global
-// memory directly).
-// ---------------------------------------------------------------------------
-constexpr int kXttStagePer = 4;
-
-template <int KIND, int ZPL, int KM>
-__device__ __forceinline__ float backward_item_untilted_xtt(const BwdArgs& a, int o, int step, float* stage) {
-    constexpr int KP = (KM + 3) & ~3;  // channel constants per view, padded for 16-byte LDS loads
-    constexpr int TW = 8 + KP;         // term words per view: Bc, Ac, fu, hi, cxy, lu, iu, boff, ca[KP]
-    static_assert(kBwdBatch * TW <= kBwdTermArea, "term layout");
-    const Dims& d = a.d;
-    constexpr int xws = kXwStride;  // >= KM: whole rows, zero padded
-    const auto views = to_global(a.views + (int64_t)step * a.n_views);
-    const auto vg = to_global(a.vg);
-    const auto vgc = to_const(a.vg);
-    const int gx = a.gx;
-    const int tx = o % a.tiles_x, ty = (o / a.tiles_x) % a.tiles_y, tz = o / (a.tiles_x * a.tiles_y);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int xb = tx * gx + (wave % gx), yb = ty * a.gy + (wave / gx);
-    const int z0 = tz * 64 * ZPL;
-    const float bx0 = (float)(tx * gx) - d.xc, bx1 = (float)min(tx * gx + gx - 1, d.N - 1) - d.xc;
-    const float by0 = (float)(ty * a.gy) - d.xc, by1 = (float)min(ty * a.gy + a.gy - 1, d.N - 1) - d.xc;
-    const float bz0 = (float)z0 - d.xc, bz1 = (float)min(z0 + 64 * ZPL - 1, d.N - 1) - d.xc;
-    const float xp = (float)xb - d.xc, yp = (float)yb - d.xc;
-    const bool col_in = xb < d.N && yb < d.N;
-    const int nv = a.n_views;
-    if (nv == 0) return 0.f;
-
-    float tmp[1][ZPL][KM], fac[1][ZPL][KM];
-#pragma unroll
-    for (int q = 0; q < ZPL; q++)
-#pragma unroll
-        for (int k = 0; k < KM; k++) {
-            tmp[0][q][k] = 0.f;
-            fac[0][q][k] = 0.f;
-        }
-    const int nwhole[1] = {0};
-    float zpq[ZPL];
-#pragma unroll
-    for (int q = 0; q < ZPL; q++) zpq[q] = (float)(z0 + lane + 64 * q) - d.xc;
-
-    lds_float* const lds = (lds_float*)stage;
-    lds_int* const foot = (lds_int*)(stage + BwdBlock<KIND>::nbuf * BwdBlock<KIND>::stage_buf);
-    lds_float* const term =
-        (lds_float*)(stage + BwdBlock<KIND>::nbuf * BwdBlock<KIND>::stage_buf + kBwdFootArea + wave * kBwdTermArea);
-    // staged only when the footprint fits the fetch passes of this path
-    auto staged_here = [](int fl, int H, int R) { return (fl & 1) != 0 && H <= kXttStagePer * R; };
-
-    auto foot_batch = [&](int b0, int buf) {
-        const int j = lane >> 2, c = lane & 3;
-        const ViewGeom g = vg[views[min(b0 + j, nv - 1)]];
-        const ColForms cf = col_forms(g, (c & 1) ? bx1 : bx0, (c & 2) ? by1 : by0);
-        float umn = 0.f, umx = 0.f, vmn = 0.f, vmx = 0.f;
-        int bad = 0;
-#pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const float czp = k ? bz1 : bz0;
-            const float cd = fmaf(g.ad[2], czp, cf.nd);
-            float cu, cv;
-            voxel_uv(g, cf, czp, d, cu, cv);
-            umn = k ? fminf(umn, cu) : cu;
-            umx = k ? fmaxf(umx, cu) : cu;
-            vmn = k ? fminf(vmn, cv) : cv;
-            vmx = k ? fmaxf(vmx, cv) : cv;
-            bad |= (!(cd > 0.f) || !(fabsf(cu) < 1e7f) || !(fabsf(cv) < 1e7f)) ? 1 : 0;
-        }
-        for (int off = 1; off < 4; off <<= 1) {
-            umn = fminf(umn, __shfl_xor(umn, off));
-            umx = fmaxf(umx, __shfl_xor(umx, off));
-            vmn = fminf(vmn, __shfl_xor(vmn, off));
-            vmx = fmaxf(vmx, __shfl_xor(vmx, off));
-            bad |= __shfl_xor(bad, off);
-        }
-        const Foot f = foot_from_extent<KIND>(umn, umx, vmn, vmx, bad, d);
-        if (c == 0) {
-            lds_int* p = foot + (buf * kBwdBatch + j) * kFootWords;
-            p[0] = f.iu_lo;
-            p[1] = f.iv_lo;
-            p[2] = f.W;
-            p[3] = f.H;
-            p[4] = f.Ws;
-            p[5] = f.R;
-            p[6] = (f.staged ? 1 : 0) | (f.empty ? 2 : 0);
-        }
-    };
-    auto load_foot = [&](int buf, int j) {
-        const lds_int* p = foot + (buf * kBwdBatch + j) * kFootWords;
-        Foot f;
-        f.iu_lo = uniformi(p[0]);
-        f.iv_lo = uniformi(p[1]);
-        f.W = uniformi(p[2]);
-        f.H = uniformi(p[3]);
-        f.Ws = uniformi(p[4]);
-        f.R = uniformi(p[5]);
-        const int fl = uniformi(p[6]);
-        f.staged = staged_here(fl, f.H, f.R);
-        f.empty = (fl & 2) != 0;
-        return f;
-    };
-    // column terms of views b0 .. b0+15: lane = 4 x view + channel quarter
-    auto term_batch = [&](int b0, int buf) {
-        const int j = lane >> 2, p = lane & 3;
-        const int code = views[min(b0 + j, nv - 1)];
-        const ViewGeom g = vg[code];
-        const lds_int* fp = foot + (buf * kBwdBatch + j) * kFootWords;
-        const int iu_lo = fp[0], iv_lo = fp[1], W = fp[2], H = fp[3], Ws = fp[4], R = fp[5], fl = fp[6];
-        const ColForms c = col_forms(g, xp, yp);
-        const float inv_c = rcpf(c.nd);
-        const float u_c = fmaf(c.nu, inv_c, d.hu);
-        int iu;
-        float fu;
-        split(u_c, iu, fu);
-        const float Bc = g.av[2] * inv_c;
-        const float Ac = fmaf(c.nv, inv_c, d.hv - 0.5f);
-        const float hi = accept_u(u_c, d) ? d.vmax - 0.5f : -1.0f;
-        const int lu = min(max(iu - iu_lo, 0), W - 2);
-        const float dx = fmaf(d.vs, xp, g.d0[0]);
-        const float dy = fmaf(d.vs, yp, g.d0[1]);
-        const float ta = fmaf(Bc, bz0, Ac);
-        const float tb = fmaf(Bc, (float)(z0 + 64 * ZPL - 1) - d.xc, Ac);
-        const bool whole = staged_here(fl, H, R) && fminf(ta, tb) > 0.05f && fmaxf(ta, tb) < hi;
-        lds_float* tp = term + j * TW;
-        lds_int* ti = (lds_int*)tp;
-        if (p == 0) {
-            tp[0] = Bc;
-            tp[1] = Ac;
-            tp[2] = fu;
-            tp[3] = whole ? __int_as_float(0x7f800000) : hi;
-            tp[4] = fmaf(dy, dy, dx * dx);
-            ti[5] = lu;
-            ti[6] = iu;
-            ti[7] = (lu - iv_lo * Ws) * 4;  // LDS byte offset of texel (iu, 0) in a staging buffer
-        }
-        const auto row = to_global(a.xw + (int64_t)code * 5 * xws);
-#pragma unroll
-        for (int m = 0; m < KP / 4; m++) {
-            const int k = p + 4 * m;
-            tp[8 + k] = fmaf(xp, row[2 * xws + k], fmaf(yp, row[3 * xws + k], row[4 * xws + k]));  // 0 for k >= K
-        }
-    };
-    auto wave_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-
-    float pre[kXttStagePer];
-    int pidx[kXttStagePer];
-    auto fetch = [&](const Foot& f, int code) {
-        const auto img = to_global(a.proj + (int64_t)(code - a.code_base) * d.V * d.U);
-        int r0 = (int)((float)threadIdx.x * rcpf((float)f.W));  // within 1 of t / W: corrected below
-        int c = (int)threadIdx.x - r0 * f.W;
-        if (c < 0) {
-            r0--;
-            c += f.W;
-        } else if (c >= f.W) {
-            r0++;
-            c -= f.W;
-        }
-        const bool act = r0 < f.R;
-        const auto src = img + (int64_t)(f.iv_lo + r0) * d.U + f.iu_lo + c;
-        const int64_t rstep = (int64_t)f.R * d.U;
-#pragma unroll
-        for (int k = 0; k < kXttStagePer; k++) {
-            pidx[k] = -1;
-            if (k * f.R < f.H) {  // uniform: only the passes the footprint needs
-                const int r = r0 + k * f.R;
-                const bool in = act && r < f.H;
-                pidx[k] = in ? r * f.Ws + c : -1;
-                pre[k] = in ? src[k * rstep] : 0.f;
-            }
-        }
-    };
-    auto store = [&](const Foot& f, lds_float* buf) {
-#pragma unroll
-        for (int k = 0; k < kXttStagePer; k++)
-            if (k * f.R < f.H && pidx[k] >= 0) buf[pidx[k]] = pre[k];
-    };
-
-    // the staging schedule of the plain untilted path: view v in buffer v % 4,
-    // fetched during view v-2, a barrier after every odd view, footprint
-    // batches written four views ahead
-    static_assert(BwdBlock<KIND>::nbuf == 4, "four staging buffers");
-    constexpr int SB = BwdBlock<KIND>::stage_buf;
-    if (wave == 0) foot_batch(0, 0);
-    __syncthreads();
-    term_batch(0, 0);
-    int code = views[0], code1 = 0;
-    Foot f = load_foot(0, 0), f1{0, 0, 0, 0, 0, 0, false, false};
-    if (f.staged) {
-        fetch(f, code);
-        store(f, lds);
-    }
-    if (nv > 1) {
-        code1 = views[1];
-        f1 = load_foot(0, 1);
-        if (f1.staged) {
-            fetch(f1, code1);
-            store(f1, lds + SB);
-        }
-    }
-    __syncthreads();
-
-    for (int s = 0; s < nv; s++) {
-        const int j = s & (kBwdBatch - 1);
-        if (j == 0 && s > 0) term_batch(s, (s / kBwdBatch) & 1);
-        wave_sync();
-        if (wave == 0 && j == kBwdBatch - 4 && s + 4 < nv) foot_batch(s + 4, ((s + 4) / kBwdBatch) & 1);
-        lds_float* cur = lds + (s & 3) * SB;
-        lds_float* nxt = lds + ((s + 2) & 3) * SB;
-        int ncode = 0;
-        Foot nf{0, 0, 0, 0, 0, 0, false, false};
-        if (s + 2 < nv) {
-            ncode = views[s + 2];
-            nf = load_foot(((s + 2) / kBwdBatch) & 1, (s + 2) & (kBwdBatch - 1));
-            if (nf.staged) fetch(nf, ncode);
-        }
-        if (!f.empty && col_in) {
-            const lds_float* tp = term + j * TW;
-            const lds_int* ti = (const lds_int*)tp;
-            const float Bc = tp[0], Ac = tp[1], fu = tp[2], hi = tp[3], cxy = tp[4];
-            const int lu = ti[5], iu = ti[6], boff = ti[7];
-            const float a0 = 1.0f - fu;
-            const float d0z = vgc[code].d0[2];
             const auto row = to_const(a.xw + (int64_t)code * 5 * xws);
             float ca[KM], sz[KM], g2s[KM];
 #pragma unroll
@@ -1905,413 +1674,243 @@ __device__ __forceinline__ float backward_item_untilted_xtt(const BwdArgs& a, in
                 sz[k] = row[k];
                 g2s[k] = row[xws + k];
             }
-            // channels k >= K have zero constants (table padding): they add zero and
-            // are never stored
-            auto accumulate = [&](int q, float nb) {
+#pragma unroll
+            for (int q = 0; q < ZPL; q++) {
+                if (!all && !ok[q]) continue;
                 const float dz = fmaf(d.vs, zpq[q], d0z);
                 const float id2 = rcpf(fmaf(dz, dz, cxy));
 #pragma unroll
                 for (int k = 0; k < KM; k++) {
                     const float qk = fmaf(dz, sz[k], ca[k]);
                     const float w = fmaf(-qk * qk, id2, g2s[k]);
-                    tmp[0][q][k] = fmaf(w, nb, tmp[0][q][k]);
-                    fac[0][q][k] += w;
-                }
-            };
-            if (uniformi(__float_as_int(hi)) == 0x7f800000) {
-                // the whole z extent accepted: all reads first (LDS latency), then the sums
-                const unsigned ws4 = (unsigned)f.Ws * 4u;
-                const unsigned base = (unsigned)(uintptr_t)cur + (unsigned)boff;
-                float fv[ZPL], r[ZPL][4];
-#pragma unroll
-                for (int q = 0; q < ZPL; q++) {
-                    const float t = fmaf(Bc, zpq[q], Ac);
-                    fv[q] = __builtin_amdgcn_fractf(t);
-                    const unsigned at = __umul24((unsigned)floor_int(t), ws4) + base;
-                    const lds_float* p0 = (const lds_float*)(uintptr_t)at;
-                    const lds_float* p1 = (const lds_float*)(uintptr_t)(at + ws4);
-                    r[q][0] = p0[0];
-                    r[q][1] = p0[1];
-                    r[q][2] = p1[0];
-                    r[q][3] = p1[1];
-                }
-#pragma unroll
-                for (int q = 0; q < ZPL; q++) {
-                    const float top = fmaf(fu, r[q][1], a0 * r[q][0]);
-                    const float bot = fmaf(fu, r[q][3], a0 * r[q][2]);
-                    accumulate(q, fmaf(fv[q], bot - top, top));
-                }
-            } else {
-                // window test per voxel, 0.05 < t < hi (hi < 0 rejects the column); a
-                // rejected voxel reads an in-bounds texel and skips the sums.  Lanes
-                // with z >= N accumulate but are never stored.
-                const auto img = to_global(a.proj + (int64_t)(code - a.code_base) * d.V * d.U);
-#pragma unroll
-                for (int q = 0; q < ZPL; q++) {
-                    const float t = fmaf(Bc, zpq[q], Ac);
-                    const bool ok = t > 0.05f && t < hi;
-                    const float fl = floorf(t);
-                    const float fv = t - fl;
-                    const int iv = (int)fl;
-                    float r00, r01, r10, r11;
-                    if (f.staged) {
-                        const int qi = (ok ? iv - f.iv_lo : 0) * f.Ws + lu;
-                        r00 = cur[qi];
-                        r01 = cur[qi + 1];
-                        r10 = cur[qi + f.Ws];
-                        r11 = cur[qi + f.Ws + 1];
-                    } else {
-                        const int64_t qi = (int64_t)min(max(iv, 0), d.V - 2) * d.U + min(max(iu, 0), d.U - 2);
-                        r00 = __builtin_nontemporal_load(img + qi);
-                        r01 = __builtin_nontemporal_load(img + qi + 1);
-                        r10 = __builtin_nontemporal_load(img + qi + d.U);
-                        r11 = __builtin_nontemporal_load(img + qi + d.U + 1);
-                    }
-                    const float top = fmaf(fu, r01, a0 * r00);
-                    const float bot = fmaf(fu, r11, a0 * r10);
-                    if (ok) accumulate(q, fmaf(fv, bot - top, top));
+                    tmp[cidx][q][k] = fmaf(w, nb[q], tmp[cidx][q][k]);
+                    fac[cidx][q][k] += w;
                 }
             }
         }
-        if (s + 2 < nv && nf.staged) store(nf, nxt);
-        code = code1;
-        f = f1;
-        code1 = ncode;
-        f1 = nf;
-        if (s & 1) __syncthreads();
-    }
-    return backward_update<KIND, 1, ZPL, KM>(a, tmp, fac, nwhole, xb, yb, z0, lane);
-}
-
-// One voxel tile o of a backprojection launch; step selects the view list
-// views + step*n_views (a solver's subset step).  stage: nbuf x stage_buf floats, then the footprint and term areas.
-// Returns the lane's max |updated voxel| (MLEM / ART kinds).
-template <int KIND, bool AXIS, int CPW, int ZPL, int KM>
-__device__ __forceinline__ float backward_item(const BwdArgs& a, int o, int step, float* stage) {
-    constexpr bool XTT = IsXtt<KIND>::value;
-    constexpr int NC = CPW * CPW;
-    constexpr int KA = XTT ? KM : 1;
-    if constexpr (AXIS && !XTT && CPW == 2) {
-        return backward_item_untilted<KIND, ZPL>(a, o, step, stage);
-    }
-    if constexpr (AXIS && XTT && CPW == 1) {
-        return backward_item_untilted_xtt<KIND, ZPL, KM>(a, o, step, stage);
-    }
-    const Dims& d = a.d;
-    const auto views = to_const(a.views + (int64_t)step * a.n_views);
-    const auto vg = to_const(a.vg);
-    const int gx = a.gx;
-    const int bcx = CPW * gx, bcy = CPW * a.gy;  // block columns along x, y
-    const int tx = o % a.tiles_x, ty = (o / a.tiles_x) % a.tiles_y, tz = o / (a.tiles_x * a.tiles_y);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int xb = tx * bcx + (wave % gx) * CPW, yb = ty * bcy + (wave / gx) * CPW;
-    const int z0 = tz * 64 * ZPL;
-    const float bx0 = (float)(tx * bcx) - d.xc, bx1 = (float)min(tx * bcx + bcx - 1, d.N - 1) - d.xc;
-    const float by0 = (float)(ty * bcy) - d.xc, by1 = (float)min(ty * bcy + bcy - 1, d.N - 1) - d.xc;
-    const float bz0 = (float)z0 - d.xc, bz1 = (float)min(z0 + 64 * ZPL - 1, d.N - 1) - d.xc;
-
-    float tmp[NC][ZPL][KA], fac[NC][ZPL][KA];
-#pragma unroll
-    for (int c = 0; c < NC; c++)
-#pragma unroll
-        for (int q = 0; q < ZPL; q++)
-#pragma unroll
-            for (int k = 0; k < KA; k++) {
-                tmp[c][q][k] = 0.f;
-                fac[c][q][k] = 0.f;
-            }
-    // untilted: views that accept the whole z extent of a column (counted once
-    // per column, added to the per-voxel counts at the end; all integers, so
-    // the sums are exact in any order)
-    int nwhole[NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) nwhole[c] = 0;
-
-    // staging of one view's footprint: prefetch into registers, store later
-    FootStage<BwdBlock<KIND>::stage_per, !XTT> st;
-    const int img_bytes = d.V * d.U * 4;
-    auto fetch = [&](const Foot& f, int code) {
-        st.fetch(a.proj + (int64_t)(code - a.code_base) * d.V * d.U, img_bytes, f, d.U);
     };
 
-    if (a.n_views == 0) return 0.f;
-    // view-independent per-lane z terms
-    float zpq[ZPL];
+    // A column whose whole extent is accepted: all reads first (LDS latency),
+    // then the sums.
+    auto whole_column = [&](int s, int cidx) XR_INLINE {
+        const lds_float* tp = term + ((s & (kBwdBatch - 1)) * NC + cidx) * TW;
+        const lds_int* ti = (const lds_int*)tp;
+        const unsigned cur = (unsigned)(uintptr_t)(lds + (s & (2 * VB - 1)) * SB);
+        const lds_int* const fp = foot_of(s);
+        const unsigned ws4 = C::WF ? (unsigned)(C::WF + 1) * 4u : (unsigned)(fp[3] & 0xffff) * 4u;
+        float nb[ZPL];
+        bool ok[ZPL];
+        float fu[ZPL], fv[ZPL], r[ZPL][4];
+        unsigned base;
+        if (TILT)
+            base = cur - __umul24((unsigned)fp[1], ws4) - (unsigned)fp[0] * 4u;
+        else
+            base = cur + (unsigned)ti[3];
 #pragma unroll
-    for (int q = 0; q < ZPL; q++) zpq[q] = (float)(z0 + lane + 64 * q) - d.xc;
-    int code = views[0];
-    ViewGeom g = vg[code];
-    Foot f = footprint<KIND>(g, d, bx0, bx1, by0, by1, bz0, bz1, lane);
-    lds_float* const lds = (lds_float*)stage;
-    if (f.staged) {
-        fetch(f, code);
-        st.store(lds, f);
+        for (int q = 0; q < ZPL; q++) {
+            float t;
+            unsigned at = base;
+            if (TILT) {
+                // voxel_uv's arithmetic, with the column's half of the forms in the terms
+                const float inv = rcpf(fmaf(tp[6], zpq[q], tp[2]));
+                const float tu = fmaf(fmaf(tp[4], zpq[q], tp[0]), inv, d.hu) - 0.5f;
+                t = fmaf(fmaf(tp[5], zpq[q], tp[1]), inv, d.hv) - 0.5f;
+                fu[q] = __builtin_amdgcn_fractf(tu);
+                at += (unsigned)floor_int(tu) * 4u;
+            } else {
+                t = fmaf(tp[0], zpq[q], tp[1]);
+                fu[q] = tp[2];
+            }
+            fv[q] = __builtin_amdgcn_fractf(t);
+            at = __umul24((unsigned)floor_int(t), ws4) + at;
+            const lds_float* p0 = (const lds_float*)(uintptr_t)at;
+            const lds_float* p1 = C::WF ? p0 + (C::WF + 1) : (const lds_float*)(uintptr_t)(at + ws4);
+            r[q][0] = p0[0];
+            r[q][1] = p0[1];
+            r[q][2] = p1[0];
+            r[q][3] = p1[1];
+        }
+        const float a0 = 1.0f - fu[0];
+#pragma unroll
+        for (int q = 0; q < ZPL; q++) {
+            const float top = TILT ? fmaf(fu[q], r[q][1] - r[q][0], r[q][0]) : fmaf(fu[q], r[q][1], a0 * r[q][0]);
+            const float bot = TILT ? fmaf(fu[q], r[q][3] - r[q][2], r[q][2]) : fmaf(fu[q], r[q][3], a0 * r[q][2]);
+            nb[q] = fmaf(fv[q], bot - top, top);
+            ok[q] = true;
+        }
+        accumulate(s, cidx, tp, nb, ok, std::true_type(), 0.0f);
+    };
+
+    // Any column: a window test per voxel; a rejected voxel reads an in-bounds
+    // texel and adds zero.  counted: the view is in the column's count already.
+    auto tested_column = [&](int s, int cidx, bool counted) XR_INLINE {
+        const lds_float* tp = term + ((s & (kBwdBatch - 1)) * NC + cidx) * TW;
+        const lds_int* ti = (const lds_int*)tp;
+        const lds_float* cur = lds + (s & (2 * VB - 1)) * SB;
+        const lds_int* const fp = foot_of(s);
+        const int fl = uniformi(fp[4]);
+        const float hi = TILT ? 0.f : tp[4];
+        if (TILT ? xb + cidx % C::CX >= d.N || yb + cidx / C::CX >= d.N : uniformf(hi) < 0.f) return;
+        const int iu_lo = fp[0], iv_lo = fp[1], W = fp[2], Ws = C::WF ? C::WF + 1 : fp[3] & 0xffff;
+        const bool staged = (fl & FOOT_STAGED) != 0;
+        const auto img = to_global(a.proj + (int64_t)(uniformi(fp[5]) - a.code_base) * img_len);
+        float nb[ZPL];
+        bool ok[ZPL];
+#pragma unroll
+        for (int q = 0; q < ZPL; q++) {
+            float tv, fu;
+            int iu, lu;
+            if (TILT) {
+                const float inv = rcpf(fmaf(tp[6], zpq[q], tp[2]));
+                const float u = fmaf(fmaf(tp[4], zpq[q], tp[0]), inv, d.hu);
+                const float v = fmaf(fmaf(tp[5], zpq[q], tp[1]), inv, d.hv);
+                ok[q] = accept_u(u, d) && accept_v(v, d);
+                split(u, iu, fu);
+                lu = min(max(iu - iu_lo, 0), W - 2);
+                tv = v - 0.5f;
+            } else {
+                tv = fmaf(tp[0], zpq[q], tp[1]);
+                ok[q] = tv > 0.05f && tv < hi;
+                fu = tp[2];
+                lu = ti[5];
+                iu = ti[6];
+            }
+            const float fl_v = floorf(tv);
+            const float fv = tv - fl_v;
+            const int iv = (int)fl_v;
+            float r00, r01, r10, r11;
+            if (staged) {
+                const int qi = (ok[q] ? iv - iv_lo : 0) * Ws + lu;
+                r00 = cur[qi];
+                r01 = cur[qi + 1];
+                r10 = cur[qi + Ws];
+                r11 = cur[qi + Ws + 1];
+            } else {
+                // direct reads: a distinct (nontemporal) load form next to the LDS reads
+                // (the gfx950 backend rejects the two merged into one flat access)
+                const int64_t qi = (int64_t)min(max(iv, 0), d.V - 2) * d.U + min(max(iu, 0), d.U - 2);
+                r00 = __builtin_nontemporal_load(img + qi);
+                r01 = __builtin_nontemporal_load(img + qi + 1);
+                r10 = __builtin_nontemporal_load(img + qi + d.U);
+                r11 = __builtin_nontemporal_load(img + qi + d.U + 1);
+            }
+            const float top = TILT ? fmaf(fu, r01 - r00, r00) : fmaf(fu, r01, (1.0f - fu) * r00);
+            const float bot = TILT ? fmaf(fu, r11 - r10, r10) : fmaf(fu, r11, (1.0f - fu) * r10);
+            nb[q] = ok[q] ? fmaf(fv, bot - top, top) : 0.0f;
+        }
+        accumulate(s, cidx, tp, nb, ok, std::false_type(), counted ? 0.0f : 1.0f);
+    };
+
+    constexpr unsigned kAllCols = (1u << NC) - 1;  // of the four bits of a view in `wholes`
+    auto view = [&](int s) XR_INLINE {
+        const unsigned w = (unsigned)(wholes >> (4 * (s & (kBwdBatch - 1)))) & kAllCols;
+        if (w == kAllCols) {
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                whole_column(s, c);
+                if (ZPL > 4) __builtin_amdgcn_sched_barrier(0);
+            }
+        } else if (!(uniformi(foot_of(s)[4]) & FOOT_EMPTY)) {
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                tested_column(s, c, (w >> c & 1) != 0);
+                // one column at a time: interleaved, their values would not fit the registers
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+
+    if (wave == 0) foot_batch(0, 0);
+    __syncthreads();
+    term_batch(0);
+#pragma unroll
+    for (int g = 0; g < VB; g += C::LOOK) {
+#pragma unroll
+        for (int i = 0; i < C::LOOK; i++)
+            if (g + i < nv) fetch(g + i, i);
+#pragma unroll
+        for (int i = 0; i < C::LOOK; i++)
+            if (g + i < nv) store(g + i, i);
     }
+    wave_sync();
     __syncthreads();
 
-    for (int s = 0; s < a.n_views; s++) {
-        lds_float* cur = lds + (s & 1) * BwdBlock<KIND>::stage_buf;
-        lds_float* nxt = lds + ((s + 1) & 1) * BwdBlock<KIND>::stage_buf;
-        // prefetch the next view's footprint
-        int ncode = 0;
-        ViewGeom ng;
-        Foot nf{0, 0, 0, 0, 0, 0, false, false};
-        if (s + 1 < a.n_views) {
-            ncode = views[s + 1];
-            ng = vg[ncode];
-            nf = footprint<KIND>(ng, d, bx0, bx1, by0, by1, bz0, bz1, lane);
-            if (nf.staged) fetch(nf, ncode);
+    for (int s0 = 0; s0 < nv; s0 += VB) {
+        const int j = s0 & (kBwdBatch - 1);
+        if (j == 0 && s0 > 0) {
+            term_batch(s0);
+            wave_sync();
         }
-        if (!f.empty) {
-            const auto img = to_global(a.proj + (int64_t)(code - a.code_base) * d.V * d.U);
-            float g2[KA];
-            if (XTT && !AXIS) {
+        // the footprints of the batch after this one: read from a group later on
+        if (wave == 0 && j == kBwdBatch - 2 * VB && s0 + 2 * VB < nv)
+            foot_batch(s0 + 2 * VB, ((s0 + 2 * VB) / kBwdBatch) & 1);
+        if constexpr (C::LOOK == VB) {
 #pragma unroll
-                for (int k = 0; k < KA; k++) g2[k] = (k < d.K) ? to_const(a.g2)[(int64_t)code * d.K + k] : 0.f;
+            for (int i = 0; i < VB; i++)
+                if (s0 + VB + i < nv) fetch(s0 + VB + i, i);
+            constexpr unsigned long long kGroup = (NC == 1 ? 0x1111111111111111ull : NC == 2 ? 0x3333333333333333ull : ~0ull) &
+                                                  (VB == 16 ? ~0ull : (1ull << (4 * VB % 64)) - 1);
+            if (s0 + VB <= nv && (wholes >> (4 * j) & kGroup) == kGroup) {
+                // every column whole in every view of the group: no test in sight
+#pragma unroll
+                for (int i = 0; i < VB; i++)
+#pragma unroll
+                    for (int c = 0; c < NC; c++) whole_column(s0 + i, c);
+            } else {
+                for (int s = s0; s < min(s0 + VB, nv); s++) view(s);
             }
 #pragma unroll
-            for (int j = 0; j < CPW; j++) {
-#pragma unroll
-                for (int i = 0; i < CPW; i++) {
-                    const int x = xb + i, y = yb + j;
-                    if (x >= d.N || y >= d.N) continue;
-                    const int cidx = j * CPW + i;
-                    const float xp = (float)x - d.xc, yp = (float)y - d.xc;
-                    const ColForms c = col_forms(g, xp, yp);
-                    float inv_c = 0.f, u_c = 0.f;
-                    if (AXIS) {
-                        inv_c = rcpf(c.nd);
-                        u_c = fmaf(c.nu, inv_c, d.hu);
-                    }
-                    float wcol = 0.f;
-                    if (KIND == BWD_FDK) {
-                        // vol += Ud^2 * (2 pi/P) * sum c p, Ud = sod/(sod + y_unrotated) (fdk.cu:160-169)
-                        const float Xy = fmaf(d.vs, yp, g.fy);
-                        const float Ud = d.sod / (d.sod + Xy);
-                        wcol = Ud * Ud * d.cfdk;
-                    }
-                    float dx = 0.f, dy = 0.f;
-                    if (XTT) {
-                        dx = fmaf(d.vs, xp, g.d0[0]);
-                        dy = fmaf(d.vs, yp, g.d0[1]);
-                    }
-                    if (AXIS && !XTT) {
-                        // Untilted: u, hence (iu, fu), is constant along the column, the
-                        // bilinear weights factor into (1-fu, fu) x (1-fv, fv), and
-                        // t = v - 0.5 is affine in z.  The acceptance window 0.55 < u, v <
-                        // U, V - 0.55 becomes 0.05 < t < hi (hi < 0 rejects the column).
-                        // Branch free: a rejected voxel reads an in-bounds texel and adds
-                        // zero.  Lanes with z >= N accumulate but are never stored.
-                        int iu;
-                        float fu;
-                        split(u_c, iu, fu);
-                        const float a0 = 1.0f - fu;
-                        const float Bc = g.av[2] * inv_c;
-                        const float Ac = fmaf(c.nv, inv_c, d.hv - 0.5f);
-                        const float hi = accept_u(u_c, d) ? d.vmax - 0.5f : -1.0f;
-                        const int lu = min(max(iu - f.iu_lo, 0), f.W - 2);
-                        if (f.staged) {
-                            // Whole extent accepted: t at the tile's first and last z bound
-                            // every lane's t (fmaf is monotone in z), so one wave-uniform
-                            // test replaces the per-voxel window test and the select.
-                            const float ta = fmaf(Bc, (float)z0 - d.xc, Ac);
-                            const float tb = fmaf(Bc, (float)(z0 + 64 * ZPL - 1) - d.xc, Ac);
-                            if (uniformi(fminf(ta, tb) > 0.05f && fmaxf(ta, tb) < hi)) {
-                                // LDS byte address of texel (iu, iv): iv*Ws*4 + base
-                                const unsigned ws4 = (unsigned)f.Ws * 4u;
-                                const unsigned base =
-                                    (unsigned)(uintptr_t)cur + (unsigned)((lu - f.iv_lo * f.Ws) * 4);
-                                // all reads of the column first (LDS latency), then the sums
-                                float fv[ZPL], r[ZPL][4];
-#pragma unroll
-                                for (int q = 0; q < ZPL; q++) {
-                                    const float t = fmaf(Bc, zpq[q], Ac);
-                                    fv[q] = __builtin_amdgcn_fractf(t);
-                                    const unsigned at = __umul24((unsigned)floor_int(t), ws4) + base;
-                                    const lds_float* p0 = (const lds_float*)(uintptr_t)at;
-                                    const lds_float* p1 = (const lds_float*)(uintptr_t)(at + ws4);
-                                    r[q][0] = p0[0];
-                                    r[q][1] = p0[1];
-                                    r[q][2] = p1[0];
-                                    r[q][3] = p1[1];
-                                }
-#pragma unroll
-                                for (int q = 0; q < ZPL; q++) {
-                                    const float top = fmaf(fu, r[q][1], a0 * r[q][0]);
-                                    const float bot = fmaf(fu, r[q][3], a0 * r[q][2]);
-                                    const float nb = fmaf(fv[q], bot - top, top);
-                                    if (KIND == BWD_FDK)
-                                        tmp[cidx][q][0] = fmaf(wcol, nb, tmp[cidx][q][0]);
-                                    else
-                                        tmp[cidx][q][0] += nb;
-                                }
-                                if (KIND != BWD_FDK) nwhole[cidx]++;
-                                continue;
-                            }
-                        }
-#pragma unroll
-                        for (int q = 0; q < ZPL; q++) {
-                            const float t = fmaf(Bc, zpq[q], Ac);
-                            const bool ok = t > 0.05f && t < hi;
-                            const float fl = floorf(t);
-                            const float fv = t - fl;
-                            const int iv = (int)fl;
-                            float r00, r01, r10, r11;
-                            if (f.staged) {
-                                const int qi = (ok ? iv - f.iv_lo : 0) * f.Ws + lu;
-                                r00 = cur[qi];
-                                r01 = cur[qi + 1];
-                                r10 = cur[qi + f.Ws];
-                                r11 = cur[qi + f.Ws + 1];
-                            } else {
-                                // direct reads (see the general path below)
-                                const int64_t qi = (int64_t)min(max(iv, 0), d.V - 2) * d.U + min(max(iu, 0), d.U - 2);
-                                r00 = __builtin_nontemporal_load(img + qi);
-                                r01 = __builtin_nontemporal_load(img + qi + 1);
-                                r10 = __builtin_nontemporal_load(img + qi + d.U);
-                                r11 = __builtin_nontemporal_load(img + qi + d.U + 1);
-                            }
-                            const float top = fmaf(fu, r01, a0 * r00);
-                            const float bot = fmaf(fu, r11, a0 * r10);
-                            const float nb = ok ? fmaf(fv, bot - top, top) : 0.0f;
-                            if (KIND == BWD_FDK) {
-                                tmp[cidx][q][0] = fmaf(wcol, nb, tmp[cidx][q][0]);
-                            } else {
-                                tmp[cidx][q][0] += nb;
-                                fac[cidx][q][0] += ok ? 1.0f : 0.0f;
-                            }
-                        }
-                        continue;
-                    }
-#pragma unroll
-                    for (int q = 0; q < ZPL; q++) {
-                        const int z = z0 + lane + 64 * q;
-                        const float zp = (float)z - d.xc;
-                        float u, v;
-                        if (AXIS) {
-                            u = u_c;
-                            v = fmaf(fmaf(g.av[2], zp, c.nv), inv_c, d.hv);
-                        } else {
-                            voxel_uv(g, c, zp, d, u, v);
-                        }
-                        if (!(z < d.N && accept_u(u, d) && accept_v(v, d))) continue;
-                        int iu, iv;
-                        float fu, fv;
-                        split(u, iu, fu);
-                        split(v, iv, fv);
-                        float r00, r01, r10, r11;  // (iu,iv) (iu+1,iv) (iu,iv+1) (iu+1,iv+1)
-                        if (f.staged) {
-                            const int lu = min(max(iu - f.iu_lo, 0), f.W - 2);
-                            const int lv = min(max(iv - f.iv_lo, 0), f.H - 2);
-                            const int qi = lv * f.Ws + lu;
-                            r00 = cur[qi];
-                            r01 = cur[qi + 1];
-                            r10 = cur[qi + f.Ws];
-                            r11 = cur[qi + f.Ws + 1];
-                        } else {
-                            // Footprint too large for LDS: read the image directly.  These
-                            // loads must not be merged with the LDS reads above into one
-                            // flat access (the gfx950 backend rejects that form), hence the
-                            // distinct nontemporal load.
-                            const int64_t qi = (int64_t)iv * d.U + iu;
-                            r00 = __builtin_nontemporal_load(img + qi);
-                            r01 = __builtin_nontemporal_load(img + qi + 1);
-                            r10 = __builtin_nontemporal_load(img + qi + d.U);
-                            r11 = __builtin_nontemporal_load(img + qi + d.U + 1);
-                        }
-                        const float c1 = (1.0f - fu) * fv, c2 = fu * fv;
-                        const float c3 = fu * (1.0f - fv), c4 = (1.0f - fu) * (1.0f - fv);
-                        const float nb = c1 * r10 + c2 * r11 + c3 * r01 + c4 * r00;
-                        if (KIND == BWD_FDK) {
-                            tmp[cidx][q][0] = fmaf(wcol, nb, tmp[cidx][q][0]);
-                        } else if (!XTT) {
-                            tmp[cidx][q][0] += nb;
-                            fac[cidx][q][0] += 1.0f;
-                        } else {
-                            const float dz = fmaf(d.vs, zp, g.d0[2]);
-                            const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                            const float id2 = rcpf(d2);
-                            if (a.coef) {
-                                // backwardOrth: the basis rotated per voxel
-                                const int64_t vi = ((int64_t)y * d.N + x) * d.N + z;
-                                float R[9];
-                                orth_rotation(a.coef[vi], a.coef[vi + a.chan_stride], R);
-#pragma unroll
-                                for (int k = 0; k < KA; k++) {
-                                    if (k < d.K) {
-                                        const float w = orth_weight(R, a.b, k, dx, dy, dz, id2, g);
-                                        tmp[cidx][q][k] = fmaf(w, nb, tmp[cidx][q][k]);
-                                        fac[cidx][q][k] += w;
-                                    }
-                                }
-                                continue;
-                            }
-#pragma unroll
-                            for (int k = 0; k < KA; k++) {
-                                if (k < d.K) {
-                                    const float ds = fmaf(dz, a.b.S[k][2], fmaf(dy, a.b.S[k][1], dx * a.b.S[k][0]));
-                                    const float w = fmaxf(fmaf(-ds * ds, id2, a.b.S2[k]), 0.f) * g2[k];
-                                    tmp[cidx][q][k] = fmaf(w, nb, tmp[cidx][q][k]);
-                                    fac[cidx][q][k] += w;
-                                }
-                            }
-                        }
-                    }
-                }
+            for (int i = 0; i < VB; i++)
+                if (s0 + VB + i < nv) store(s0 + VB + i, i);
+        } else {
+            for (int s = s0; s < min(s0 + VB, nv); s++) {
+                if (s + VB < nv) fetch(s + VB, 0);
+                view(s);
+                if (s + VB < nv) store(s + VB, 0);
             }
-        }
-        if (s + 1 < a.n_views) {
-            if (nf.staged) st.store(nxt, nf);
-            code = ncode;
-            g = ng;
-            f = nf;
         }
         __syncthreads();
     }
-    return backward_update<KIND, CPW, ZPL, KA>(a, tmp, fac, nwhole, xb, yb, z0, lane);
+    return backward_update<C>(a, tmp, fac, nwhole, xb, yb, z0, lane);
 }
 
-template <int KIND, bool AXIS, int CPW, int ZPL, int KM>
 // at least 4 waves per SIMD (at most 128 VGPRs): two 8-wave blocks, or one
 // 16-wave block, per CU
-__global__ __launch_bounds__(BwdBlock<KIND>::threads) __attribute__((amdgpu_waves_per_eu(4))) void k_backward(
-    const BwdArgs a) {
-    extern __shared__ float stage[];  // nbuf x stage_buf staging, footprint and term areas
+template <class C, bool TILT>
+__global__ __launch_bounds__(C::threads) __attribute__((amdgpu_waves_per_eu(4))) void k_backward(const BwdArgs a) {
+    extern __shared__ float stage[];
     const int o = (blockIdx.x % 8) * a.per_xcd + blockIdx.x / 8;
     if (o >= a.n_tiles) return;
-    float m = backward_item<KIND, AXIS, CPW, ZPL, KM>(a, o, 0, stage);
-    if constexpr (KIND == BWD_MLEM || KIND == BWD_ART) {
+    float m = backward_item<C, TILT>(a, o, 0, stage);
+    if constexpr (C::KIND == BWD_MLEM || C::KIND == BWD_ART) {
         if (a.vmax_out) {
             // the tile's max |updated voxel|: one atomic per block
-            lds_float* const wmax =
-                (lds_float*)(stage + BwdBlock<KIND>::nbuf * BwdBlock<KIND>::stage_buf + bwd_extra_words<KIND>());
+            lds_float* const wmax = (lds_float*)(stage + C::words);
             for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
             if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
             __syncthreads();
             if (threadIdx.x == 0) {
                 float t = 0.f;
-                for (int w = 0; w < BwdBlock<KIND>::waves; w++) t = fmaxf(t, wmax[w]);
+                for (int w = 0; w < C::WAVES; w++) t = fmaxf(t, wmax[w]);
                 __hip_atomic_fetch_max(a.vmax_out, __float_as_uint(t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
     }
 }
 
-// Persistent backprojection over many problems (plain MLEM / ART kinds): the
-// same work queue as k_forward_batch; items[i] is one problem with
-// item_end[i] - item_end[i-1] tiles, and its own tile shape (zpl, gx).
-template <int KIND, int ZPL, int CPW = 2, int KM = 1>
-__global__ __launch_bounds__(BwdBlock<KIND>::threads) __attribute__((amdgpu_waves_per_eu(4))) void k_backward_batch(
-    const BwdArgs* __restrict__ items,
-                                                                const int* __restrict__ item_end, int n_items,
-                                                                unsigned* queue, int step) {
-    extern __shared__ float stage[];  // nbuf x stage_buf; the last word of buffer 1 holds the ticket
+// Persistent backprojection over many problems: the same work queue as
+// k_forward_batch; items[i] is one problem with item_end[i] - item_end[i-1]
+// tiles, and its own tile shape.  W: the configuration of the tilted and wide
+// items (the same block).
+template <class C, class W>
+__global__ __launch_bounds__(C::threads) __attribute__((amdgpu_waves_per_eu(4))) void k_backward_batch(
+    const BwdArgs* __restrict__ items, const int* __restrict__ item_end, int n_items, unsigned* queue, int step) {
+    extern __shared__ float stage[];
     typedef __attribute__((address_space(3))) unsigned lds_uint;
-    lds_uint* const tk = (lds_uint*)stage + (2 * BwdBlock<KIND>::stage_buf - 1);
-    // past the staging and term areas: the last tile's per-wave max |voxel| and its item
-    lds_float* const wmax =
-        (lds_float*)(stage + BwdBlock<KIND>::nbuf * BwdBlock<KIND>::stage_buf + bwd_extra_words<KIND>());
-    lds_int* const witem = (lds_int*)(wmax + BwdBlock<KIND>::waves);
+    // past the staging and term areas: the last tile's per-wave max |voxel|, its item, the ticket
+    lds_float* const wmax = (lds_float*)(stage + (C::words > W::words ? C::words : W::words));
+    lds_int* const witem = (lds_int*)(wmax + C::WAVES);
+    lds_uint* const tk = (lds_uint*)(wmax + C::WAVES + 1);
     const int total = item_end[n_items - 1];
     if (threadIdx.x == 0) *witem = -1;
     for (;;) {
@@ -2322,7 +1921,7 @@ __global__ __launch_bounds__(BwdBlock<KIND>::threads) __attribute__((amdgpu_wave
             unsigned* const dst = pi >= 0 ? items[pi].vmax_out : nullptr;
             if (dst) {
                 float m = 0.f;
-                for (int w = 0; w < BwdBlock<KIND>::waves; w++) m = fmaxf(m, wmax[w]);
+                for (int w = 0; w < C::WAVES; w++) m = fmaxf(m, wmax[w]);
                 __hip_atomic_fetch_max(dst, __float_as_uint(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             *witem = -1;  // flushed: only a tile that sets it again sends a max
@@ -2335,8 +1934,9 @@ __global__ __launch_bounds__(BwdBlock<KIND>::threads) __attribute__((amdgpu_wave
         const int i = find_item(item_end, n_items, t);
         const BwdArgs& a = items[i];
         const int o = t - (i ? item_end[i - 1] : 0);
-        float m = a.axis ? backward_item<KIND, true, CPW, ZPL, KM>(a, o, step, stage)
-                         : backward_item<KIND, false, CPW, ZPL, KM>(a, o, step, stage);
+        float m = !a.axis ? backward_item<W, true>(a, o, step, stage)
+                          : (a.wide ? backward_item<W, false>(a, o, step, stage)
+                                    : backward_item<C, false>(a, o, step, stage));
         if (a.vmax_out) {
             for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
             if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
@@ -3058,110 +2658,166 @@ hipError_t launch_forward(const FwdArgs& a, int kind, bool axis, hipStream_t str
 
 int default_zpl(int N) { return N > 128 ? 4 : (N > 64 ? 2 : 1); }
 
-// staging buffers, per-view footprint and term areas, per-wave max slots (and
-// the persistent launch's item slot)
-template <int KD>
-constexpr size_t backward_lds_bytes(bool batch) {
-    return (BwdBlock<KD>::nbuf * BwdBlock<KD>::stage_buf + bwd_extra_words<KD>() + BwdBlock<KD>::waves +
-            (batch ? 1 : 0)) *
-           sizeof(float);
-}
-
 inline bool bwd_xtt(int kind) { return kind == BWD_XTT_RAW || kind == BWD_XTT_MLEM || kind == BWD_XTT_ART; }
 
 int backward_threads(int kind) {
-    return bwd_xtt(kind) ? BwdBlock<BWD_XTT_MLEM>::threads : BwdBlock<BWD_MLEM>::threads;
+    return bwd_xtt(kind) ? BwdLarge<BWD_XTT_MLEM, 1, 4>::Cfg::threads : BwdLarge<BWD_MLEM, 1, 1>::Cfg::threads;
 }
 
-size_t backward_batch_lds_bytes(int kind) {
-    return bwd_xtt(kind) ? backward_lds_bytes<BWD_XTT_MLEM>(true) : backward_lds_bytes<BWD_MLEM>(true);
+// Estimated footprint of a tile of cx x cy columns and 64 zpl voxels: its
+// diagonal and, along z, its extent at the tilt, at the largest magnification
+// in the volume.  Launch shapes only: a footprint that turns out larger is read
+// from the image directly.
+static void backward_footprint(const Dims& d, int cx, int cy, int zpl, float& w, float& h) {
+    const float diag = std::sqrt((float)((cx - 1) * (cx - 1) + (cy - 1) * (cy - 1))), z = 64.0f * zpl - 1.0f;
+    w = (diag + z * d.tilt_sin) * d.px + 2.02f;
+    h = (z * d.tilt_cos + diag * d.tilt_sin) * d.px + 2.02f;
+}
+
+// Tile counts of a grid of `waves` waves, gx along x, each of cpw x cpw columns
+// and 64 zpl voxels.
+static void backward_tiles(BwdArgs& a, int waves, int cpw, int zpl, int gx) {
+    const int N = a.d.N;
+    a.zpl = zpl;
+    a.gx = gx;
+    a.gy = waves / gx;
+    a.tiles_x = (N + cpw * a.gx - 1) / (cpw * a.gx);
+    a.tiles_y = (N + cpw * a.gy - 1) / (cpw * a.gy);
+    a.tiles_z = (a.d.nz + 64 * zpl - 1) / (64 * zpl);  // z >= nz: never visited
+    a.n_tiles = a.tiles_x * a.tiles_y * a.tiles_z;
+    a.per_xcd = (a.n_tiles + 7) / 8;
+    // wider footprints than the fixed width (a tile's diagonal, see backward_footprint)
+    float w, h;
+    backward_footprint(a.d, cpw * a.gx, cpw * a.gy, zpl, w, h);
+    a.wide = w > (cpw == 1 ? 8.0f : 16.0f) || h > (cpw == 1 ? 64.0f * 3 : 64.0f * 7);
 }
 
 bool backward_shape(BwdArgs& a, int zpl, int gx, bool xtt) {
-    const int N = a.d.N;
     // Plain / FDK: 2x2 columns x zpl z per lane, 16 waves as gx x gy column
     // groups (a (2gx) x (2gy)-column tile, 64*zpl z).  XTT (2K accumulators per
     // voxel): one column x zpl (1 or 2) z per lane, 8 waves.
-    const int CPW = xtt ? 1 : 2;
     if (xtt && zpl == 0) zpl = 1;
     if (xtt && zpl > 2) return false;
-    if (zpl == 0) zpl = default_zpl(N);
+    if (zpl == 0) zpl = default_zpl(a.d.N);
     // default column layout: 8 x 8 columns (plain); 2 x 4 for XTT (measured
     // 144.6 against 146.2 ms for 4 x 2 at 256^3 x 13, 4 x 360 views)
     if (gx == 0) gx = xtt ? 2 : 4;
     if (!(zpl == 1 || zpl == 2 || zpl == 4)) return false;
     if (!(gx == 1 || gx == 2 || gx == 4 || gx == 8 || gx == 16)) return false;
-    const int waves = xtt ? BwdBlock<BWD_XTT_MLEM>::waves : BwdBlock<BWD_MLEM>::waves;
+    const int waves = xtt ? 8 : 16;
     gx = std::min(gx, waves);  // XTT blocks have 8 waves: gx 16 is taken as 8
-    a.zpl = zpl;
-    a.gx = gx;
-    a.gy = waves / gx;
-    a.tiles_x = (N + CPW * a.gx - 1) / (CPW * a.gx);
-    a.tiles_y = (N + CPW * a.gy - 1) / (CPW * a.gy);
-    a.tiles_z = (a.d.nz + 64 * zpl - 1) / (64 * zpl);  // z >= nz: never visited
-    a.n_tiles = a.tiles_x * a.tiles_y * a.tiles_z;
-    a.per_xcd = (a.n_tiles + 7) / 8;
+    backward_tiles(a, waves, xtt ? 1 : 2, zpl, gx);
     return true;
 }
 
+// Shape of a standalone launch where the plan leaves it open (zpl and gx 0);
+// true: the kernel for few tiles (BwdSmall).
+// Plain, untilted: the z depth zpl (1 to 5) that covers the volume's 64-voxel
+// chunks with the least work, tiles_z (zpl + 2): a column's terms and a
+// footprint's edges cost about as much per view as two chunks (three chunks,
+// 160^3 / 180 views: zpl 3 615, 4 724, 2 971 us; five chunks, 320^3 / 60 views:
+// zpl 5 1171, 2 1605, 4 1759 us).
+// Fewer than kSmallTiles such tiles leave most of the chip idle: BwdSmall
+// (64^3 / 90 views, 64 tiles: 41 against 95 us; but at 96^3 / 90 views, 144
+// tiles: 177 against 125 us).
+// Tilted: the largest depth whose footprint fits the staging buffer.
+// XTT: two voxels per lane halve the per-view overhead of a column (35.1
+// against 23.0 ms for ART at 256^3 x 13, 4 x 90 views) where the volume has
+// more than 64 layers, the footprint fits and the accumulators do.
+constexpr int kSmallTiles = 96;
+static bool backward_choose(BwdArgs& a, int kind, bool axis) {
+    const Dims& d = a.d;
+    const int chunks = (d.nz + 63) / 64;
+    float w, h;
+    if (bwd_xtt(kind)) {
+        backward_footprint(d, 2, 4, 2, w, h);
+        const bool fits = axis ? h <= 192.0f : w * h <= 0.9f * 3584.0f;
+        // (26 accumulators per voxel of 13 coefficients: two voxels spill where both sums are kept)
+        const bool regs = a.d.K <= 8 || (kind == BWD_XTT_ART && (axis || a.d.K <= 13));
+        backward_tiles(a, 8, 1, chunks > 1 && fits && regs ? 2 : 1, 2);
+        return false;
+    }
+    int zpl = 1;
+    if (axis) {
+        int best = 0;
+        for (int z = 5; z >= 1; z--) {
+            backward_footprint(d, 8, 8, z, w, h);
+            if (z > 1 && (w <= 16.0f ? h > 448.0f : (z % 2 == 1 || w * h > 0.9f * 7168.0f))) continue;
+            const int cost = (chunks + z - 1) / z * (z + 2);
+            if (best == 0 || cost < best) {
+                best = cost;
+                zpl = z;
+            }
+        }
+    } else {
+        for (int z : {4, 2}) {
+            backward_footprint(d, 8, 8, z, w, h);
+            if (zpl == 1 && z <= default_zpl(d.nz) && w * h <= 0.9f * 7168.0f) zpl = z;
+        }
+    }
+    backward_tiles(a, 16, 2, zpl, 4);
+    backward_footprint(d, 4, 2, 1, w, h);
+    if (axis && a.n_tiles < kSmallTiles && w <= 8.0f && h <= 128.0f) {
+        backward_tiles(a, 8, 1, 1, 4);
+        return true;
+    }
+    return false;
+}
+
+template <class C, bool TILT>
+static hipError_t start_backward(const BwdArgs& a, hipStream_t stream) {
+    hipLaunchKernelGGL((k_backward<C, TILT>), dim3((unsigned)(8 * a.per_xcd)), dim3(C::threads), C::lds_bytes, stream,
+                       a);
+    return hipGetLastError();
+}
+
+template <int KIND, int ZPL, int KM>
+static hipError_t start_backward_large(const BwdArgs& a, bool axis, hipStream_t stream) {
+    if (!axis) return start_backward<typename BwdLarge<KIND, ZPL, KM>::Wide, true>(a, stream);
+    if (a.wide) return start_backward<typename BwdLarge<KIND, ZPL, KM>::Wide, false>(a, stream);
+    return start_backward<typename BwdLarge<KIND, ZPL, KM>::Cfg, false>(a, stream);
+}
+
+template <int KIND>
+static hipError_t start_backward_plain(const BwdArgs& a, bool axis, bool small, hipStream_t stream) {
+    if (small) return start_backward<typename BwdSmall<KIND>::Cfg, false>(a, stream);
+    switch (a.zpl) {
+        case 1: return start_backward_large<KIND, 1, 1>(a, axis, stream);
+        case 2: return start_backward_large<KIND, 2, 1>(a, axis, stream);
+        case 4: return start_backward_large<KIND, 4, 1>(a, axis, stream);
+        case 3: if (axis) return start_backward<typename BwdLarge<KIND, 3, 1>::Cfg, false>(a, stream); break;
+        case 5: if (axis) return start_backward<typename BwdLarge<KIND, 5, 1>::Cfg, false>(a, stream); break;
+    }
+    return hipErrorInvalidValue;
+}
+
+template <int KIND, int ZPL>
+static hipError_t start_backward_xtt(const BwdArgs& a, bool axis, hipStream_t stream) {
+    if (a.d.K <= 4) return start_backward_large<KIND, ZPL, 4>(a, axis, stream);
+    if (a.d.K <= 8) return start_backward_large<KIND, ZPL, 8>(a, axis, stream);
+    if (a.d.K <= 13) return start_backward_large<KIND, ZPL, 13>(a, axis, stream);
+    return start_backward_large<KIND, ZPL, 16>(a, axis, stream);
+}
+
 hipError_t launch_backward(BwdArgs a, int kind, bool axis, hipStream_t stream) {
-    const bool xtt = (kind == BWD_XTT_RAW || kind == BWD_XTT_MLEM || kind == BWD_XTT_ART);
-    if (!backward_shape(a, a.zpl, a.gx, xtt)) return hipErrorInvalidValue;
-    const int zpl = a.zpl;
-    const unsigned grid = (unsigned)(8 * a.per_xcd);
-#define XR_BWD(KD, A, C, Z, KM)                                                                          \
-    hipLaunchKernelGGL((k_backward<KD, A, C, Z, KM>), dim3(grid), dim3(BwdBlock<KD>::threads),          \
-                       backward_lds_bytes<KD>(false), stream, a)
-#define XR_BWD_AX(KD, C, Z, KM)         \
-    do {                                \
-        if (axis)                       \
-            XR_BWD(KD, true, C, Z, KM); \
-        else                            \
-            XR_BWD(KD, false, C, Z, KM); \
-    } while (0)
-#define XR_BWD_PLAIN(KD)             \
-    do {                             \
-        if (zpl == 4)                \
-            XR_BWD_AX(KD, 2, 4, 1);  \
-        else if (zpl == 2)           \
-            XR_BWD_AX(KD, 2, 2, 1);  \
-        else                         \
-            XR_BWD_AX(KD, 2, 1, 1);  \
-    } while (0)
-#define XR_BWD_XTT_Z(KD, Z)              \
-    do {                                 \
-        if (a.d.K <= 4)                  \
-            XR_BWD_AX(KD, 1, Z, 4);      \
-        else if (a.d.K <= 8)             \
-            XR_BWD_AX(KD, 1, Z, 8);      \
-        else if (a.d.K <= 13)            \
-            XR_BWD_AX(KD, 1, Z, 13);     \
-        else                             \
-            XR_BWD_AX(KD, 1, Z, 16);     \
-    } while (0)
-#define XR_BWD_XTT(KD)             \
-    do {                           \
-        if (zpl == 2)              \
-            XR_BWD_XTT_Z(KD, 2);   \
-        else                       \
-            XR_BWD_XTT_Z(KD, 1);   \
-    } while (0)
+    bool small = false;
+    if (a.zpl == 0 && a.gx == 0)
+        small = backward_choose(a, kind, axis);
+    else if (!backward_shape(a, a.zpl, a.gx, bwd_xtt(kind)))
+        return hipErrorInvalidValue;
     switch (kind) {
-        case BWD_RAW: XR_BWD_PLAIN(BWD_RAW); break;
-        case BWD_MLEM: XR_BWD_PLAIN(BWD_MLEM); break;
-        case BWD_ART: XR_BWD_PLAIN(BWD_ART); break;
-        case BWD_FDK: XR_BWD_PLAIN(BWD_FDK); break;
-        case BWD_XTT_RAW: XR_BWD_XTT(BWD_XTT_RAW); break;
-        case BWD_XTT_MLEM: XR_BWD_XTT(BWD_XTT_MLEM); break;
-        case BWD_XTT_ART: XR_BWD_XTT(BWD_XTT_ART); break;
+        case BWD_RAW: return start_backward_plain<BWD_RAW>(a, axis, small, stream);
+        case BWD_MLEM: return start_backward_plain<BWD_MLEM>(a, axis, small, stream);
+        case BWD_ART: return start_backward_plain<BWD_ART>(a, axis, small, stream);
+        case BWD_FDK: return start_backward_plain<BWD_FDK>(a, axis, small, stream);
+        case BWD_XTT_RAW:
+            return a.zpl == 2 ? start_backward_xtt<BWD_XTT_RAW, 2>(a, axis, stream) : start_backward_xtt<BWD_XTT_RAW, 1>(a, axis, stream);
+        case BWD_XTT_MLEM:
+            return a.zpl == 2 ? start_backward_xtt<BWD_XTT_MLEM, 2>(a, axis, stream) : start_backward_xtt<BWD_XTT_MLEM, 1>(a, axis, stream);
+        case BWD_XTT_ART:
+            return a.zpl == 2 ? start_backward_xtt<BWD_XTT_ART, 2>(a, axis, stream) : start_backward_xtt<BWD_XTT_ART, 1>(a, axis, stream);
         default: return hipErrorInvalidValue;
     }
-#undef XR_BWD_XTT
-#undef XR_BWD_XTT_Z
-#undef XR_BWD_PLAIN
-#undef XR_BWD_AX
-#undef XR_BWD
-    return hipGetLastError();
 }
 
 // Basis count rounded up to a compiled size of the XTT kernels.
@@ -3196,14 +2852,32 @@ hipError_t launch_forward_batch(const FwdArgs* items, const int* item_end, int n
     return hipGetLastError();
 }
 
+template <int KIND, int ZPL, int KM>
+static constexpr size_t batch_lds_of() {
+    typedef BwdLarge<KIND, ZPL, KM> L;
+    return L::Cfg::lds_bytes > L::Wide::lds_bytes ? L::Cfg::lds_bytes : L::Wide::lds_bytes;
+}
+
+static size_t backward_batch_lds_bytes(int kind, int zpl, int kmax) {
+    if (!bwd_xtt(kind))
+        return zpl == 4 ? batch_lds_of<BWD_MLEM, 4, 1>()
+                        : (zpl == 2 ? batch_lds_of<BWD_MLEM, 2, 1>() : batch_lds_of<BWD_MLEM, 1, 1>());
+    switch (xtt_km(kmax)) {
+        case 4: return batch_lds_of<BWD_XTT_MLEM, 1, 4>();
+        case 8: return batch_lds_of<BWD_XTT_MLEM, 1, 8>();
+        case 13: return batch_lds_of<BWD_XTT_MLEM, 1, 13>();
+        default: return batch_lds_of<BWD_XTT_MLEM, 1, 16>();
+    }
+}
+
 // Batched backprojection kernel of (kind, zpl) (XTT kinds: zpl 1, one column
 // per wave, kmax basis vectors at most), or nullptr.
 const void* backward_batch_kernel(int kind, int zpl, int kmax) {
 #define XR_BB(KD)                                                        \
     if (kind == KD) {                                                    \
-        if (zpl == 4) return (const void*)k_backward_batch<KD, 4>;       \
-        if (zpl == 2) return (const void*)k_backward_batch<KD, 2>;       \
-        if (zpl == 1) return (const void*)k_backward_batch<KD, 1>;       \
+        if (zpl == 4) return (const void*)k_backward_batch<BwdLarge<KD, 4, 1>::Cfg, BwdLarge<KD, 4, 1>::Wide>;       \
+        if (zpl == 2) return (const void*)k_backward_batch<BwdLarge<KD, 2, 1>::Cfg, BwdLarge<KD, 2, 1>::Wide>;       \
+        if (zpl == 1) return (const void*)k_backward_batch<BwdLarge<KD, 1, 1>::Cfg, BwdLarge<KD, 1, 1>::Wide>;       \
     }
     XR_BB(BWD_MLEM)
     XR_BB(BWD_ART)
@@ -3211,10 +2885,10 @@ const void* backward_batch_kernel(int kind, int zpl, int kmax) {
 #define XR_BBX(KD)                                                                \
     if (kind == KD && zpl == 1) {                                                 \
         switch (xtt_km(kmax)) {                                                   \
-            case 4: return (const void*)k_backward_batch<KD, 1, 1, 4>;            \
-            case 8: return (const void*)k_backward_batch<KD, 1, 1, 8>;            \
-            case 13: return (const void*)k_backward_batch<KD, 1, 1, 13>;          \
-            default: return (const void*)k_backward_batch<KD, 1, 1, 16>;          \
+            case 4: return (const void*)k_backward_batch<BwdLarge<KD, 1, 4>::Cfg, BwdLarge<KD, 1, 4>::Wide>;            \
+            case 8: return (const void*)k_backward_batch<BwdLarge<KD, 1, 8>::Cfg, BwdLarge<KD, 1, 8>::Wide>;            \
+            case 13: return (const void*)k_backward_batch<BwdLarge<KD, 1, 13>::Cfg, BwdLarge<KD, 1, 13>::Wide>;          \
+            default: return (const void*)k_backward_batch<BwdLarge<KD, 1, 16>::Cfg, BwdLarge<KD, 1, 16>::Wide>;          \
         }                                                                         \
     }
     XR_BBX(BWD_XTT_MLEM)
@@ -3229,7 +2903,8 @@ hipError_t launch_backward_batch(const BwdArgs* items, const int* item_end, int 
     const void* k = backward_batch_kernel(kind, zpl, kmax);
     if (!k) return hipErrorInvalidValue;
     void* args[] = {(void*)&items, (void*)&item_end, (void*)&n_items, (void*)&queue, (void*)&step};
-    return hipLaunchKernel(k, dim3(grid), dim3(backward_threads(kind)), args, backward_batch_lds_bytes(kind), stream);
+    return hipLaunchKernel(k, dim3(grid), dim3(backward_threads(kind)), args, backward_batch_lds_bytes(kind, zpl, kmax),
+                           stream);
 }
 
 int batch_blocks_per_cu_forward(int kind, size_t lds_bytes, bool axis_all, int kmax) {
@@ -3269,7 +2944,8 @@ int batch_blocks_per_cu_backward(int kind, int zpl, int kmax) {
     int n = 0;
     const void* k = backward_batch_kernel(kind, zpl, kmax);
     if (!k) return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, backward_threads(kind), backward_batch_lds_bytes(kind)) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, backward_threads(kind),
+                                                     backward_batch_lds_bytes(kind, zpl, kmax)) !=
         hipSuccess)
         return 0;
     return n;

@@ -832,6 +832,17 @@ int xr_plan_create(xr_context* ctx, const xr_geometry* g, const xr_scan* s, int 
     }
     d.sod = g->sod;
     d.cfdk = 2.0f * (float)M_PI / (float)P;
+    {
+        // launch shapes only: no result depends on these
+        const double near_den = 1.0 - 0.5 * std::sqrt(3.0) * g->n_vox * (double)g->vox_size / g->sod;
+        d.px = (float)((double)g->sdd / g->det_size / g->sod * g->vox_size / std::max(near_den, 0.05));
+        d.tilt_cos = d.tilt_sin = 0.0f;
+        for (int c = 0; c < C; c++) {
+            const float zz = std::min(std::fabs(p->cond_R[9 * c + 8]), 1.0f);
+            d.tilt_cos = std::max(d.tilt_cos, zz);
+            if (!p->axis_cond[c]) d.tilt_sin = std::max(d.tilt_sin, std::sqrt(1.0f - zz * zz));
+        }
+    }
     for (int k = 0; k < s->n_basis; k++) {
         float g2max = 0.f;
         for (size_t i = 0; i < (size_t)C * P; i++) g2max = std::max(g2max, g2[i * K + k]);
