@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 namespace xr {
@@ -191,10 +192,30 @@ int batch_blocks_per_cu_forward(int kind, size_t lds_bytes, bool axis_all, int k
 // Dynamic LDS of a standalone forward launch of vb detector rows.
 size_t forward_lds_bytes(int kind, int vb);
 // Resident blocks per CU of the standalone forward kernel.
-int forward_blocks_per_cu(int kind, bool axis, size_t lds_bytes);
-// Sub-bands per detector band (1, 2, 4) for a launch of `items` band items on
-// `slots` resident blocks: split while the items would leave the chip under-
-// filled (a forced value `tile` > 0 wins).
+int forward_blocks_per_cu(int kind, bool axis, const Dims& d, size_t lds_bytes);
+// Sub-bands per detector band (1, 2, 4) of a standalone launch of `items` band
+// items on `slots` resident blocks, volume edge N: the least of (rounds of the
+// chip, and three quarters of one for the last items) x (work of an item).  An
+// item of 16/s columns visits 16/s + 1 columns' worth of voxels and has fixed
+// costs (its scan, its accumulator) that weigh less the larger the volume.
+// Measured (us for s = 1, 2, 4): 64^3 / 90 views 73 65 85, 128^3 / 9 109 76 72,
+// 128^3 / 60 201 163 220, 203^3 / 20 346 204 213, 512^3 / 5 940 767 641.
+inline int forward_split_alone(int64_t items, int64_t slots, int N) {
+    int best = 1;
+    float least = 0.0f;
+    for (int s = 1; s <= 4; s *= 2) {
+        const float rounds = std::max(1.0f, (float)(items * s) / (float)std::max<int64_t>(slots, 1) + 0.75f);
+        const float cost = rounds * (16.0f / (float)s + 1.5f + 192.0f / (float)N);
+        if (s == 1 || cost < least) {
+            best = s;
+            least = cost;
+        }
+    }
+    return best;
+}
+// The same for a persistent launch (its blocks take one item after another):
+// split while the items would leave the chip underfilled (a forced value `tile`
+// > 0 wins).
 inline int forward_split(int64_t items, int64_t slots, int tile) {
     if (tile > 0) return tile;
     int s = 1;

@@ -178,13 +178,10 @@ __device__ double chord_length(const ChordGeom& c, int u, int v, const Dims& d) 
 
 // ---------------------------------------------------------------------------
 // Forward projection: one block = (detector band of kBandU columns, one view,
-// a chunk of detector rows).  The block's waves (kFwdWaves, or kFwdBatchWaves in
-// the persistent multi-problem launch) walk the volume rows y (round
+// a chunk of detector rows).  The block's waves walk the volume rows y (round
 // robin), find the z-columns whose footprint touches the band (ballot over 64 x
-// per step), and splat them with lanes = z.  Two columns are in flight per wave
-// and all z chunks of a column are loaded before any is used.
+// per step), and splat them with lanes = z.
 // ---------------------------------------------------------------------------
-constexpr int kFwdChunks = 8;  // z chunks of 64 loaded per column per step (512 z)
 constexpr int kXttChunks = 2;  // untilted XTT: z chunks of 64 (x K channels) loaded per step
 
 typedef __attribute__((address_space(3))) unsigned long long lds_u64;
@@ -611,10 +608,253 @@ __device__ __forceinline__ void splat_tilted(const FwdArgs& a, const ViewGeom& g
     }
 }
 
+// ---------------------------------------------------------------------------
+// Untilted views: the splat of one band.  u is constant along a z column, so a
+// column either touches the band or does not, and its terms (u split, t = v -
+// 0.5 = B (z - xc) + A) are computed once by the lane that scans it and read
+// from there.  CH chunks of 64 z are loaded per column and step, of as many
+// columns at once as make 16 loads (at most 8): with one column pair a step
+// whatever the depth, a 64-layer volume had two loads in flight per wave and
+// spent its time waiting.
+// Columns whose z extent lies inside the window (t is monotone in z) run
+// without tests; a partial last chunk only masks its lanes (such depths used to
+// take masked loads and tests throughout).
+// Measured, before -> now: 64^3 / 90 views 94 -> 64 us; 203^3 / 20 views 321 ->
+// 226 us; 512^3 / 720 views, bound by VALU issue, 58.8 -> 57.2 ms.
+// ---------------------------------------------------------------------------
+template <int KIND, int WAVES, int KM, int CH>
+__device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& g, int code, gptr<const float> vol,
+                                              float wscale, lds_ptr<typename FwdAcc<KIND>::T> acc, int band, int u0,
+                                              int cs, int W, int v0, int vb) {
+    typedef typename FwdAcc<KIND>::T AccT;
+    typedef typename FwdAcc<KIND>::S AccS;
+    constexpr bool XTT = KIND == FWD_XTT;
+    constexpr int NCOL = XTT ? 1 : (CH >= 2 ? 16 / CH : 8);
+    constexpr int xws = kXwStride;
+    const Dims& d = a.d;
+    const int lane = threadIdx.x & 63, wave = uniformi(threadIdx.x >> 6);
+    const auto xrow = to_const(a.xw ? a.xw + (int64_t)code * 5 * xws : nullptr);
+    // the window of t: 0.55 < v < V - 0.55 (ir.cu:1501) and v0 - 1 <= floor(t) < v0 + vb
+    const float t_lo = (v0 >= 2) ? __int_as_float(__float_as_int((float)(v0 - 1)) - 1) : 0.05f;
+    const float t_hi = fminf(d.vmax - 0.5f, (float)(v0 + vb));
+    const int spare_row = min(lane, vb);  // rows spare_row, spare_row + 1 lie in the band
+    const bool rows_all = v0 <= 0 && v0 + vb >= d.V;  // this launch covers every detector row
+    const float z_first = -d.xc, z_end = (float)(d.nz - 1) - d.xc;
+    float lanef[CH];  // z offset of the lane in each chunk of a step
+#pragma unroll
+    for (int c = 0; c < CH; c++) lanef[c] = (float)(c * 64 + lane);
+
+    const auto bands = to_global(a.bands ? a.bands + ((int64_t)code * a.n_bands + band) * d.N : nullptr);
+    for (int y0 = wave; y0 < d.N; y0 += 64 * WAVES) {
+        // the scan bounds of the wave's next 64 rows: lane i holds row y0 + i WAVES
+        const int yl = y0 + lane * WAVES;
+        const int scan = yl < d.N ? (a.bands ? bands[yl] : d.N << 16) : 0;
+        for (int i = 0; i < 64; i++) {
+            const int y = y0 + i * WAVES;
+            if (y >= d.N) break;
+            const float yp = (float)y - d.xc;
+            const int xb = lane_i(scan, i);  // columns of this row to scan (the test below is exact)
+            const int xs = xb & 0xffff, xe = xb >> 16;
+            for (int x0 = xs & ~63; x0 < xe; x0 += 64) {
+                const int x = x0 + lane;
+                bool cand = false, in = false;
+                // this lane's column terms, kept for the candidate loop: t = B (z - xc) + A,
+                // the two u weights with the fixed-point scale, the band column
+                float sB = 0.f, sA = 0.f, sw0 = 0.f, sw1 = 0.f;
+                int scp = 0;
+                if (x < d.N) {
+                    const ColForms c = col_forms(g, (float)x - d.xc, yp);
+                    const float inv = rcpf(c.nd);
+                    const float u = fmaf(c.nu, inv, d.hu);
+                    if (accept_u(u, d)) {
+                        int iu;
+                        float fu;
+                        split(u, iu, fu);
+                        cand = (unsigned)(iu - (u0 + cs - 1)) <= (unsigned)W;
+                        sB = g.av[2] * inv;
+                        sA = fmaf(c.nv, inv, d.hv - 0.5f);
+                        sw0 = (1.0f - fu) * wscale;
+                        sw1 = fu * wscale;
+                        scp = iu - u0 + 1;
+                        // t at the first and last z bounds every lane's t: z - xc is exact and
+                        // fmaf is monotone in it
+                        const float ta = fmaf(sB, z_first, sA), tb = fmaf(sB, z_end, sA);
+                        in = rows_all && fminf(ta, tb) > t_lo && fmaxf(ta, tb) < t_hi;
+                    }
+                }
+                // XTT: |d|^2 - dz^2 of the column's source->voxel vector d and
+                // sig_k (d_x S_k,x + d_y S_k,y), so that sig_k (d.S_k) = dz sig_k S_k,z + xck_k
+                float xcxy = 0.f, xck[KM];
+                if (XTT) {
+                    const float xp = (float)x - d.xc;
+                    const float dx = fmaf(d.vs, xp, g.d0[0]), dy = fmaf(d.vs, yp, g.d0[1]);
+                    xcxy = fmaf(dy, dy, dx * dx);
+#pragma unroll
+                    for (int k = 0; k < KM; k++)
+                        xck[k] = fmaf(xp, xrow[2 * xws + k], fmaf(yp, xrow[3 * xws + k], xrow[4 * xws + k]));
+                }
+                const auto row = vol + ((int64_t)y * d.N + x0) * d.N;  // column b of the scan at b N
+                // LDS byte address of band row floor(t) = 0 of a column
+                auto row0_of = [&](int b) XR_INLINE {
+                    return (unsigned)(uintptr_t)(acc + lane_i(scp, b)) +
+                           (unsigned)((1 - v0) * kBandStride * (int)sizeof(AccT));
+                };
+                const unsigned long long mc = __ballot(cand), mi = __ballot(cand && in);
+                // columns of mask m, NCOL at a time.  INSIDE: whole columns in the window.
+                auto columns = [&](unsigned long long m, auto inside_c) XR_INLINE {
+                    constexpr bool INSIDE = decltype(inside_c)::value;
+                    while (m) {
+                        int b[NCOL], n = 0;
+#pragma unroll
+                        for (int k = 0; k < NCOL; k++) {
+                            b[k] = m ? __ffsll(m) - 1 : b[0];
+                            n += m ? 1 : 0;
+                            m &= m ? m - 1 : 0;
+                        }
+                        int zb = 0, ze = d.nz;
+                        if (!INSIDE && !rows_all) {
+                            zb = d.nz;
+                            ze = 0;
+#pragma unroll
+                            for (int k = 0; k < NCOL; k++) {
+                                int zb_k, ze_k;
+                                col_zrange_t(lane_f(sB, b[k]), lane_f(sA, b[k]), d, v0, vb, zb_k, ze_k);
+                                zb = min(zb, zb_k);
+                                ze = max(ze, ze_k);
+                            }
+                        }
+                        // one step: chunks zg, zg + 64, ... of the n columns.  MODE 2: NCOL columns, CH
+                        // whole chunks (XTT: and K the compiled count); 1: the last chunk partial; 0: any.
+                        auto step = [&](int zg, auto mode_c) XR_INLINE {
+                            constexpr int MODE = decltype(mode_c)::value;
+                            constexpr bool FULL = MODE > 0;
+                            // t = B (z - xc) + A: z - xc is exact in FP32 (half-integers below
+                            // 2^23), so t depends on z alone and not on where the step starts
+                            const float zoff = (float)zg - d.xc;
+                            const int rem = d.nz - zg;  // layers left
+                            const auto there = [&](int c) XR_INLINE { return FULL || zg + c * 64 < ze; };
+                            // a chunk that ends past the volume masks its lanes
+                            auto in_chunk = [&](int c) XR_INLINE {
+                                return MODE == 2 || (MODE == 1 && c < CH - 1) || c * 64 + 64 <= rem || lane < rem - c * 64;
+                            };
+                            auto splat = [&](int c, float val, float B, float A, unsigned row0, lds_ptr<AccT> spare,
+                                             float w0, float w1) XR_INLINE {
+                                const float t = fmaf(B, lanef[c] + zoff, A);
+                                if (in_chunk(c)) {
+                                    if (XTT ? (mi >> b[0] & 1) != 0 : INSIDE)
+                                        splat_inside<AccT, AccS>(t, val, row0, w0, w1);
+                                    else
+                                        splat_untilted<AccT, AccS>(t, val, row0, spare, w0, w1, t_lo, t_hi);
+                                }
+                            };
+                            if constexpr (!XTT) {
+                                float mu[NCOL][CH];
+                                if (KIND != FWD_WEIGHT) {
+#pragma unroll
+                                    for (int k = 0; k < NCOL; k++)
+                                        if (FULL || k < n) {
+                                            const auto col = row + (int64_t)b[k] * d.N + lane;
+#pragma unroll
+                                            for (int c = 0; c < CH; c++)
+                                                if (there(c) && in_chunk(c)) mu[k][c] = col[zg + c * 64];
+                                        }
+                                }
+#pragma unroll
+                                for (int k = 0; k < NCOL; k++) {
+                                    if (!FULL && k >= n) break;
+                                    const float B = lane_f(sB, b[k]), A = lane_f(sA, b[k]);
+                                    const float w0 = lane_f(sw0, b[k]), w1 = lane_f(sw1, b[k]);
+                                    const unsigned row0 = row0_of(b[k]);
+                                    const lds_ptr<AccT> spare = acc + lane_i(scp, b[k]) + spare_row * kBandStride;
+#pragma unroll
+                                    for (int c = 0; c < CH; c++) {
+                                        if (!there(c)) break;
+                                        splat(c, KIND == FWD_WEIGHT ? 1.f : mu[k][c], B, A, row0, spare, w0, w1);
+                                    }
+                                }
+                            } else {
+                                // Per voxel the value sum_k mu_k (S_k.G)^2 |B x S_k|^2 (ir.cu:1780-1794)
+                                // is sum_k mu_k (g2s_k - q_k^2 / |d|^2), q_k = sig_k (d.S_k) affine in z;
+                                // vs * ratio rides in the splat weights.  k is the outer loop of a chunk
+                                // pair, so only one k's constants are live at a time.
+                                const float cxy = lane_f(xcxy, b[0]);
+                                float mu[CH][KM];
+                                if (MODE == 2) {
+                                    // one address per channel walked from the previous one (the chunks
+                                    // are immediate offsets); opaque, or the compiler keeps all K
+                                    // channels' lane addresses in registers across the columns
+                                    auto col = row + (int64_t)b[0] * d.N + (zg + lane);
+                                    asm volatile("" : "+v"(col));
+#pragma unroll
+                                    for (int k = 0; k < KM; k++) {
+#pragma unroll
+                                        for (int c = 0; c < CH; c++) mu[c][k] = col[c * 64];
+                                        col += a.chan_stride;
+                                    }
+                                } else {
+                                    // lanes past the end read the last layer (one offset for all channels)
+                                    const auto col = row + (int64_t)b[0] * d.N + zg;
+                                    unsigned zl[CH];
+#pragma unroll
+                                    for (int c = 0; c < CH; c++) zl[c] = (unsigned)min(c * 64 + lane, rem - 1);
+#pragma unroll
+                                    for (int k = 0; k < KM; k++)
+#pragma unroll
+                                        for (int c = 0; c < CH; c++)
+                                            if (k < d.K) mu[c][k] = col[zl[c] + (int64_t)k * a.chan_stride];
+                                }
+                                float dz[CH], id2[CH], val[CH];
+#pragma unroll
+                                for (int c = 0; c < CH; c++) {
+                                    dz[c] = fmaf(d.vs, lanef[c] + zoff, g.d0[2]);
+                                    id2[c] = rcpf(fmaf(dz[c], dz[c], cxy));
+                                    val[c] = 0.f;
+                                }
+#pragma unroll
+                                for (int k = 0; k < KM; k++) {
+                                    if (MODE == 2 || k < d.K) {
+                                        const float ck = lane_f(xck[k], b[0]), sS2 = xrow[k], g2s = xrow[xws + k];
+#pragma unroll
+                                        for (int c = 0; c < CH; c++) {
+                                            const float q = fmaf(dz[c], sS2, ck);
+                                            val[c] = fmaf(fmaf(-q * q, id2[c], g2s), mu[c][k], val[c]);
+                                        }
+                                    }
+                                }
+                                const float B = lane_f(sB, b[0]), A = lane_f(sA, b[0]);
+                                const float w0 = lane_f(sw0, b[0]), w1 = lane_f(sw1, b[0]);
+                                const unsigned row0 = row0_of(b[0]);
+                                const lds_ptr<AccT> spare = acc + lane_i(scp, b[0]) + spare_row * kBandStride;
+#pragma unroll
+                                for (int c = 0; c < CH; c++) {
+                                    if (!there(c)) break;
+                                    splat(c, val[c], B, A, row0, spare, w0, w1);
+                                }
+                            }
+                        };
+                        for (int zg = zb & ~63; zg < ze; zg += 64 * CH) {
+                            const int left = ze - zg;
+                            if (n == NCOL && left >= 64 * CH && (!XTT || d.K == KM))
+                                step(zg, std::integral_constant<int, 2>());
+                            else if (!XTT && INSIDE && n == NCOL && left > 64 * (CH - 1))
+                                step(zg, std::integral_constant<int, 1>());
+                            else
+                                step(zg, std::integral_constant<int, 0>());
+                        }
+                    }
+                };
+                // XTT: one copy of the loop (its registers), the window decided per column
+                if constexpr (!XTT) columns(mi, std::true_type());
+                columns(XTT ? mc : mc & ~mi, std::false_type());
+            }
+        }
+    }
+}
+
 // One (band, view) work item o = band * n_slots + slot of a forward launch.
 // step selects the view list views + step*n_slots (a solver's subset step);
 // loss receives the item's share of sum |y - p|.
-template <int KIND, bool AXIS, int WAVES, int KM = kMaxBasis>
+template <int KIND, bool AXIS, int WAVES, int KM, int CH>
 __device__ __forceinline__ void forward_item(const FwdArgs& a, int o, int step, double* loss,
                                              unsigned long long* acc_raw, int v0, int vb) {
     typedef typename FwdAcc<KIND>::T AccT;
@@ -666,274 +906,13 @@ __device__ __forceinline__ void forward_item(const FwdArgs& a, int o, int step, 
 
     const int lane = threadIdx.x & 63, wave = uniformi(threadIdx.x >> 6);
     const auto vol = to_global(a.vol + (KIND == FWD_PLAIN ? (int64_t)cond * a.vol_cond_stride : 0));
-    // XTT: the view's row of the per-plan weight table (BwdArgs::xw)
-    constexpr int xws = kXwStride;
-    const auto xrow = to_const(a.xw ? a.xw + (int64_t)code * 5 * xws : nullptr);
     // value scale folded into the untilted splat weights: ratio (ir.cu:1513-1518),
     // XTT vs * ratio (ir.cu:1791)
     const float scalev = (KIND == FWD_PLAIN) ? d.ratio : (KIND == FWD_XTT ? d.vs * d.ratio : 1.f);
-    // untilted path: lane offsets of the z chunks, and the window of t = v - 0.5:
-    // 0.55 < v < V - 0.55 (ir.cu:1501) and v0 - 1 <= floor(t) < v0 + vb
-    float lanef[kFwdChunks];
-#pragma unroll
-    for (int c = 0; c < kFwdChunks; c++) lanef[c] = (float)(c * 64 + lane);
-    const float t_lo = (v0 >= 2) ? __int_as_float(__float_as_int((float)(v0 - 1)) - 1) : 0.05f;
-    const float t_hi = fminf(d.vmax - 0.5f, (float)(v0 + vb));
-    const int spare_row = min(lane, vb);  // rows spare_row, spare_row + 1 lie in the band
-    const bool rows_all = v0 <= 0 && v0 + vb >= d.V;  // this launch covers every detector row
-
-    if constexpr (!AXIS) splat_tilted<KIND, WAVES, KM>(a, g, code, scale, acc, u0, cs, W, v0, vb);
-
-    const auto bands = to_global(a.bands ? a.bands + ((int64_t)code * a.n_bands + band) * d.N : nullptr);
-    for (int y = wave; AXIS && y < d.N; y += WAVES) {
-        const float yp = (float)y - d.xc;
-        int xs = 0, xe = d.N;  // columns of this row to scan (the test below is exact)
-        if (a.bands) {
-            const int v = uniformi(bands[y]);
-            xs = v & 0xffff;
-            xe = v >> 16;
-        }
-        for (int x0 = xs & ~63; x0 < xe; x0 += 64) {
-            const int x = x0 + lane;
-            bool cand = false;
-            // untilted: this lane's column terms, kept for the candidate loop (which
-            // reads a candidate's terms from its lane): t = v - 0.5 = B (z - xc) + A,
-            // the two u weights with the fixed-point scale, the band column, the z range
-            float sB = 0.f, sA = 0.f, sw0 = 0.f, sw1 = 0.f;
-            int scp = 0;
-            // untilted XTT: |d|^2 - dz^2 of the column's source->voxel vector d and
-            // sig_k (d_x S_k,x + d_y S_k,y), so that sig_k (d.S_k) = dz sig_k S_k,z + xck_k
-            float xcxy = 0.f, xck[KM];
-            if (KIND == FWD_XTT) {
-                const float xp = (float)x - d.xc;
-                const float dx = fmaf(d.vs, xp, g.d0[0]), dy = fmaf(d.vs, yp, g.d0[1]);
-                xcxy = fmaf(dy, dy, dx * dx);
-#pragma unroll
-                for (int k = 0; k < KM; k++)
-                    xck[k] = fmaf(xp, xrow[2 * xws + k], fmaf(yp, xrow[3 * xws + k], xrow[4 * xws + k]));
-            }
-            if (x < d.N) {
-                const ColForms c = col_forms(g, (float)x - d.xc, yp);
-                const float inv = rcpf(c.nd);
-                const float u = fmaf(c.nu, inv, d.hu);
-                if (accept_u(u, d)) {
-                    int iu;
-                    float fu;
-                    split(u, iu, fu);
-                    cand = (unsigned)(iu - (u0 + cs - 1)) <= (unsigned)W;
-                    sB = g.av[2] * inv;
-                    sA = fmaf(c.nv, inv, d.hv - 0.5f);
-                    sw0 = (1.0f - fu) * (scale * scalev);
-                    sw1 = fu * (scale * scalev);
-                    scp = iu - u0 + 1;
-                }
-            }
-            unsigned long long m = __ballot(cand);
-            if (KIND == FWD_XTT) {
-                // Untilted XTT: a candidate's column terms come from its lane; per voxel
-                // the value sum_k mu_k (S_k.G)^2 |B x S_k|^2 (ir.cu:1780-1794) is
-                // sum_k mu_k (g2s_k - q_k^2 / |d|^2), q_k = sig_k (d.S_k) affine in z;
-                // vs * ratio rides in the splat weights.
-                // EXACT: d.K == KM (the k loops need no bound).  k is the outer loop of a
-                // chunk pair, so only one k's constants are live at a time.
-                auto candidates = [&](auto exact_c) {
-                    constexpr bool EXACT = decltype(exact_c)::value;
-                    while (m) {
-                        const int b = __ffsll(m) - 1;
-                        m &= m - 1;
-                        const float Bc = lane_f(sB, b), Ac = lane_f(sA, b);
-                        const float w0 = lane_f(sw0, b), w1 = lane_f(sw1, b);
-                        const float cxy = lane_f(xcxy, b);
-                        const lds_ptr<AccT> cp = acc + lane_i(scp, b);
-                        int zb = 0, ze = d.nz;
-                        if (!rows_all) col_zrange_t(Bc, Ac, d, v0, vb, zb, ze);
-                        const int64_t cbase = ((int64_t)y * d.N + x0 + b) * d.N;
-                        const unsigned row0 =
-                            (unsigned)(uintptr_t)cp + (unsigned)((1 - v0) * kBandStride * (int)sizeof(AccT));
-                        const lds_ptr<AccT> spare = cp + spare_row * kBandStride;
-                        const bool whole = (d.nz & 63) == 0 && zb == 0 && ze == d.nz;
-                        // every voxel of the column inside the window (t monotone in z)
-                        const float ta = fmaf(Bc, -d.xc, Ac), tb = fmaf(Bc, (float)(d.nz - 1) - d.xc, Ac);
-                        const bool inside = whole && fminf(ta, tb) > t_lo && fmaxf(ta, tb) < t_hi;
-                        const auto col = vol + cbase + lane;
-                        for (int zg = zb & ~63; zg < ze; zg += 64 * kXttChunks) {
-                            float mu[kXttChunks][KM];
-                            if (EXACT && whole && zg + 64 * kXttChunks <= d.nz) {
-                                // every lane in range: unmasked loads, one address per channel
-                                // walked from the previous one (the chunks are immediate offsets)
-#pragma unroll
-                                for (int k = 0; k < KM; k++)
-#pragma unroll
-                                    for (int c = 0; c < kXttChunks; c++)
-                                        mu[c][k] = col[zg + c * 64 + (int64_t)k * a.chan_stride];
-                            } else {
-#pragma unroll
-                                for (int c = 0; c < kXttChunks; c++) {
-                                    const int z = zg + c * 64 + lane;
-                                    const bool in = whole ? (zg + c * 64 < d.nz) : (z >= zb && z < ze);
-#pragma unroll
-                                    for (int k = 0; k < KM; k++)
-                                        mu[c][k] = (in && (EXACT || k < d.K))
-                                                       ? col[zg + c * 64 + (int64_t)k * a.chan_stride]
-                                                       : 0.f;
-                                }
-                            }
-                            const float zoff = (float)zg - d.xc;
-                            float dz[kXttChunks], id2[kXttChunks], val[kXttChunks];
-#pragma unroll
-                            for (int c = 0; c < kXttChunks; c++) {
-                                dz[c] = fmaf(d.vs, lanef[c] + zoff, g.d0[2]);
-                                id2[c] = rcpf(fmaf(dz[c], dz[c], cxy));
-                                val[c] = 0.f;
-                            }
-#pragma unroll
-                            for (int k = 0; k < KM; k++) {
-                                if (EXACT || k < d.K) {
-                                    const float ck = lane_f(xck[k], b), sS2 = xrow[k], g2s = xrow[xws + k];
-#pragma unroll
-                                    for (int c = 0; c < kXttChunks; c++) {
-                                        const float q = fmaf(dz[c], sS2, ck);
-                                        val[c] = fmaf(fmaf(-q * q, id2[c], g2s), mu[c][k], val[c]);
-                                    }
-                                }
-                            }
-#pragma unroll
-                            for (int c = 0; c < kXttChunks; c++) {
-                                if (zg + c * 64 >= ze) break;
-                                const float t = fmaf(Bc, lanef[c] + zoff, Ac);
-                                if (inside)
-                                    splat_inside<AccT, AccS>(t, val[c], row0, w0, w1);
-                                else
-                                    splat_untilted<AccT, AccS>(t, val[c], row0, spare, w0, w1, t_lo, t_hi);
-                            }
-                        }
-                    }
-                };
-                if (d.K == KM)
-                    candidates(std::true_type());
-                else
-                    candidates(std::false_type());
-            } else {
-                while (m) {
-                    const int b0 = __ffsll(m) - 1;
-                    m &= m - 1;
-                    const bool two = m != 0;
-                    const int b1 = two ? __ffsll(m) - 1 : b0;
-                    if (two) m &= m - 1;
-                    // the candidates' terms, computed by their lanes in the scan
-                    const float B0 = lane_f(sB, b0), B1 = lane_f(sB, b1);
-                    const float A0 = lane_f(sA, b0), A1 = lane_f(sA, b1);
-                    const float w00 = lane_f(sw0, b0), w01 = lane_f(sw1, b0);
-                    const float w10 = lane_f(sw0, b1), w11 = lane_f(sw1, b1);
-                    const lds_ptr<AccT> cp0 = acc + lane_i(scp, b0), cp1 = acc + lane_i(scp, b1);
-                    int zb0 = 0, ze0 = d.nz, zb1 = 0, ze1 = d.nz;
-                    if (!rows_all) {
-                        col_zrange_t(B0, A0, d, v0, vb, zb0, ze0);
-                        col_zrange_t(B1, A1, d, v0, vb, zb1, ze1);
-                    }
-                    const int zb = min(zb0, zb1), ze = max(ze0, ze1);
-                    const int64_t base0 = ((int64_t)y * d.N + x0 + b0) * d.N;
-                    const int64_t base1 = ((int64_t)y * d.N + x0 + b1) * d.N;
-                    // LDS byte address of band row floor(t) = 0 of each column, and each
-                    // lane's spare row for rejected voxels
-                    const unsigned row00 =
-                        (unsigned)(uintptr_t)cp0 + (unsigned)((1 - v0) * kBandStride * (int)sizeof(AccT));
-                    const unsigned row01 =
-                        (unsigned)(uintptr_t)cp1 + (unsigned)((1 - v0) * kBandStride * (int)sizeof(AccT));
-                    const lds_ptr<AccT> spare0 = cp0 + spare_row * kBandStride;
-                    const lds_ptr<AccT> spare1 = cp1 + spare_row * kBandStride;
-                    // t = v - 0.5 = B*(z - xc) + (nv*inv + hv - 0.5); z - xc is exact in
-                    // FP32 (half-integers below 2^23), so t depends on z alone and not on
-                    // where the chunk group starts.
-                    // Whole columns (both z ranges are [0, N), N a multiple of 64): every
-                    // loaded z is in range, so the loads need no masks and share one
-                    // address per column.  Wave-uniform.
-                    const bool whole = KIND != FWD_WEIGHT && (d.nz & 63) == 0 && zb0 == 0 && ze0 == d.nz &&
-                                       zb1 == 0 && ze1 == d.nz;
-                    const auto col0 = vol + base0 + lane, col1 = vol + base1 + lane;
-                    // Inside: every voxel of a whole column lies in the window (t at the
-                    // first and last z bound every lane's t: z - xc is exact and fmaf is
-                    // monotone in it), so the splat needs no window test.
-                    auto inside_col = [&](float B, float A) {
-                        const float ta = fmaf(B, -d.xc, A), tb = fmaf(B, (float)(d.nz - 1) - d.xc, A);
-                        return fminf(ta, tb) > t_lo && fmaxf(ta, tb) < t_hi;
-                    };
-                    const bool inside = whole && inside_col(B0, A0) && (!two || inside_col(B1, A1));
-                    // one or two columns, whole or clipped, inside the window or not:
-                    // template constants, so that no per-chunk test of any remains
-                    auto columns = [&](auto two_c, auto whole_c, auto inside_c) {
-                        constexpr bool TWO = decltype(two_c)::value;
-                        constexpr bool WHOLE = decltype(whole_c)::value;
-                        constexpr bool INSIDE = decltype(inside_c)::value;
-                        // z chunks start at multiples of 64 so that a lane always holds the
-                        // same z residue: the splat's lane pairing (hence its rounding) does
-                        // not depend on where the row chunk clips the column.
-                        for (int zg = zb & ~63; zg < ze; zg += 64 * kFwdChunks) {
-                            float m0[kFwdChunks], m1[kFwdChunks];
-                            if (WHOLE && zg + 64 * kFwdChunks <= d.nz) {
-                                // all chunks in range: plain loads at immediate offsets
-#pragma unroll
-                                for (int c = 0; c < kFwdChunks; c++) {
-                                    m0[c] = col0[zg + c * 64];
-                                    if (TWO) m1[c] = col1[zg + c * 64];
-                                }
-                            } else {
-#pragma unroll
-                            for (int c = 0; c < kFwdChunks; c++) {
-                                const int z = zg + c * 64 + lane;
-                                if (WHOLE) {
-                                    const bool in = zg + c * 64 < d.nz;
-                                    m0[c] = in ? col0[zg + c * 64] : 0.f;
-                                    if (TWO) m1[c] = in ? col1[zg + c * 64] : 0.f;
-                                } else if (KIND == FWD_WEIGHT) {
-                                    // zero outside the column's z range: the splat has no z test
-                                    m0[c] = (z < ze0 && z >= zb0) ? 1.f : 0.f;
-                                    if (TWO) m1[c] = (z < ze1 && z >= zb1) ? 1.f : 0.f;
-                                } else {
-                                    m0[c] = (z < ze0 && z >= zb0) ? vol[base0 + z] : 0.f;
-                                    if (TWO) m1[c] = (z < ze1 && z >= zb1) ? vol[base1 + z] : 0.f;
-                                }
-                            }
-                            }
-                            const float zoff = (float)zg - d.xc;
-#pragma unroll
-                            for (int c = 0; c < kFwdChunks; c++) {
-                                if (zg + c * 64 >= ze) break;
-                                const float zp = lanef[c] + zoff;
-                                if (INSIDE) {
-                                    splat_inside<AccT, AccS>(fmaf(B0, zp, A0), m0[c], row00, w00, w01);
-                                    if (TWO) splat_inside<AccT, AccS>(fmaf(B1, zp, A1), m1[c], row01, w10, w11);
-                                } else {
-                                    splat_untilted<AccT, AccS>(fmaf(B0, zp, A0), m0[c], row00, spare0, w00, w01,
-                                                               t_lo, t_hi);
-                                    if (TWO)
-                                        splat_untilted<AccT, AccS>(fmaf(B1, zp, A1), m1[c], row01, spare1, w10,
-                                                                   w11, t_lo, t_hi);
-                                }
-                            }
-                        }
-                    };
-                    using T_ = std::true_type;
-                    using F_ = std::false_type;
-                    if (two) {
-                        if (inside)
-                            columns(T_(), T_(), T_());
-                        else if (whole)
-                            columns(T_(), T_(), F_());
-                        else
-                            columns(T_(), F_(), F_());
-                    } else {
-                        if (inside)
-                            columns(F_(), T_(), T_());
-                        else if (whole)
-                            columns(F_(), T_(), F_());
-                        else
-                            columns(F_(), F_(), F_());
-                    }
-                }
-            }
-        }
-    }
+    if constexpr (AXIS)
+        splat_columns<KIND, WAVES, KM, CH>(a, g, code, vol, scale * scalev, acc, band, u0, cs, W, v0, vb);
+    else
+        splat_tilted<KIND, WAVES, KM>(a, g, code, scale, acc, u0, cs, W, v0, vb);
     __syncthreads();
 
     double lsum = 0.0, l2sum = 0.0;  // sum |y - p|, sum (y - p)^2 (OUT_RESIDUAL_L2)
@@ -1030,8 +1009,9 @@ __device__ __forceinline__ int view_grouped(const FwdArgs& a, int oi) {
     return jj * a.n_slots + sl;
 }
 
-template <int KIND, bool AXIS, int KM = kMaxBasis, int WAVES = kFwdWaves>
-__global__ __launch_bounds__(64 * WAVES) void k_forward(const FwdArgs a) {
+// two blocks per CU: at most 80 VGPRs in 12-wave blocks, 128 in 8-wave ones
+template <int KIND, bool AXIS, int KM, int WAVES, int CH>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 12 ? 6 : 4) void k_forward(const FwdArgs a) {
     extern __shared__ unsigned long long acc_raw[];
     const int per_chunk = a.n_bands * max(a.n_sub, 1) * a.n_slots;
     const int nblk = per_chunk * a.n_chunks;
@@ -1047,7 +1027,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_forward(const FwdArgs a) {
     const int chunk = o / per_chunk;
     const int v0 = a.v0 + chunk * a.vb;
     const int vb = min(a.vb, a.d.V - v0);
-    forward_item<KIND, AXIS, WAVES, KM>(a, view_grouped(a, o - chunk * per_chunk), 0, a.loss, acc_raw, v0, vb);
+    forward_item<KIND, AXIS, WAVES, KM, CH>(a, view_grouped(a, o - chunk * per_chunk), 0, a.loss, acc_raw, v0, vb);
 }
 
 // Work queue of a persistent launch: q[0] hands out tickets 0, 1, 2, ...; a
@@ -1086,7 +1066,7 @@ __device__ __forceinline__ int find_item(const int* __restrict__ item_end, int n
 // so the long items listed first are started first and the short ones fill
 // the tail.  ticket_slot: index of a free 8-byte LDS word past every item's
 // band accumulator.
-template <int KIND, int AXES, int WAVES, int KM = kMaxBasis>
+template <int KIND, int AXES, int WAVES, int KM = 1>
 __device__ __forceinline__ void forward_batch_loop(const FwdArgs* __restrict__ items,
                                                    const int* __restrict__ item_end, int n_items, unsigned* queue,
                                                    int ticket_slot, int step, int loss_shift) {
@@ -1105,16 +1085,16 @@ __device__ __forceinline__ void forward_batch_loop(const FwdArgs* __restrict__ i
         const int o = view_grouped(a, t - (i ? item_end[i - 1] : 0));
         double* loss = a.loss ? a.loss + loss_shift : nullptr;
         if (AXES == 1 || a.axis)
-            forward_item<KIND, true, WAVES, KM>(a, o, step, loss, acc_raw, a.v0, a.vb);
+            forward_item<KIND, true, WAVES, KM, KIND == FWD_XTT ? kXttChunks : 8>(a, o, step, loss, acc_raw, a.v0, a.vb);
         else
-            forward_item<KIND, false, WAVES, KM>(a, o, step, loss, acc_raw, a.v0, a.vb);
+            forward_item<KIND, false, WAVES, KM, 8>(a, o, step, loss, acc_raw, a.v0, a.vb);
     }
 }
 
 // Persistent forward of XTT problems (forwardProjXTT, ir.cu:1753-1804): the
 // same loop with the directional splat, KM >= every item's basis count.
 template <int KM>
-__global__ __launch_bounds__(64 * kFwdXttWaves) void k_forward_batch_xtt(const FwdArgs* __restrict__ items,
+__global__ __launch_bounds__(64 * kFwdXttWaves, 4) void k_forward_batch_xtt(const FwdArgs* __restrict__ items,
                                                                        const int* __restrict__ item_end,
                                                                        int n_items, unsigned* queue, int ticket_slot,
                                                                        int step, int loss_shift) {
@@ -2621,39 +2601,44 @@ inline unsigned grid1(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs);
 
 }  // namespace
 
+static int forward_waves(int kind) { return kind == FWD_XTT ? kFwdXttWaves : kFwdWaves; }
+
+// Standalone forward kernel: chunks per column and step by the volume's depth
+// (see splat_columns), XTT by the basis count rounded up to a compiled size (the
+// registers of a voxel's coefficients).
+template <int KIND>
+static const void* forward_kernel_of(bool axis, int nz) {
+    if (!axis) return (const void*)k_forward<KIND, false, 1, kFwdWaves, 1>;
+    if (nz <= 64) return (const void*)k_forward<KIND, true, 1, kFwdWaves, 1>;
+    if (nz <= 128) return (const void*)k_forward<KIND, true, 1, kFwdWaves, 2>;
+    if (nz <= 256) return (const void*)k_forward<KIND, true, 1, kFwdWaves, 4>;
+    return (const void*)k_forward<KIND, true, 1, kFwdWaves, 8>;
+}
+template <int KM>
+static const void* forward_kernel_xtt(bool axis) {
+    return axis ? (const void*)k_forward<FWD_XTT, true, KM, kFwdXttWaves, kXttChunks>
+                : (const void*)k_forward<FWD_XTT, false, KM, kFwdXttWaves, 1>;
+}
+static const void* forward_kernel(int kind, bool axis, const Dims& d) {
+    if (kind == FWD_WEIGHT) return forward_kernel_of<FWD_WEIGHT>(axis, d.nz);
+    if (kind == FWD_PLAIN) return forward_kernel_of<FWD_PLAIN>(axis, d.nz);
+    if (d.K <= 4) return forward_kernel_xtt<4>(axis);
+    if (d.K <= 8) return forward_kernel_xtt<8>(axis);
+    if (d.K <= 13) return forward_kernel_xtt<13>(axis);
+    return forward_kernel_xtt<16>(axis);
+}
+
 hipError_t launch_forward(const FwdArgs& a, int kind, bool axis, hipStream_t stream) {
     const int nblk = a.n_bands * std::max(a.n_sub, 1) * a.n_slots * a.n_chunks;
     if (nblk == 0) return hipSuccess;
     const unsigned grid = (unsigned)(8 * ((nblk + 7) / 8));
     const size_t lds = forward_lds_bytes(kind, a.vb);
-#define XR_FWD(KD, A) hipLaunchKernelGGL((k_forward<KD, A>), dim3(grid), dim3(64 * kFwdWaves), lds, stream, a)
-    if (kind == FWD_WEIGHT) {
-        if (axis) XR_FWD(FWD_WEIGHT, true); else XR_FWD(FWD_WEIGHT, false);
-    } else if (kind == FWD_PLAIN) {
-        if (axis) XR_FWD(FWD_PLAIN, true); else XR_FWD(FWD_PLAIN, false);
-    } else {
-        // basis count rounded up to a compiled size (the registers of a voxel's coefficients)
-#define XR_FWD_K(KM)                                                                                             \
-    do {                                                                                                         \
-        if (axis)                                                                                                \
-            hipLaunchKernelGGL((k_forward<FWD_XTT, true, KM, kFwdXttWaves>), dim3(grid), dim3(64 * kFwdXttWaves), \
-                               lds, stream, a);                                                                  \
-        else                                                                                                     \
-            hipLaunchKernelGGL((k_forward<FWD_XTT, false, KM, kFwdXttWaves>), dim3(grid), dim3(64 * kFwdXttWaves), \
-                               lds, stream, a);                                                                  \
-    } while (0)
-        if (a.d.K <= 4)
-            XR_FWD_K(4);
-        else if (a.d.K <= 8)
-            XR_FWD_K(8);
-        else if (a.d.K <= 13)
-            XR_FWD_K(13);
-        else
-            XR_FWD_K(16);
-#undef XR_FWD_K
-    }
-#undef XR_FWD
-    return hipGetLastError();
+    FwdArgs arg = a;
+    void* args[] = {&arg};
+    return (kind == FWD_PLAIN || kind == FWD_WEIGHT || kind == FWD_XTT)
+               ? hipLaunchKernel(forward_kernel(kind, axis, a.d), dim3(grid), dim3(64 * forward_waves(kind)),
+                                 args, lds, stream)
+               : hipErrorInvalidValue;
 }
 
 int default_zpl(int N) { return N > 128 ? 4 : (N > 64 ? 2 : 1); }
@@ -2928,15 +2913,10 @@ size_t forward_lds_bytes(int kind, int vb) {
     return ((size_t)fwd_red_slot(vb + 2, acc_bytes) + 2 * kFwdWaves) * sizeof(unsigned long long);
 }
 
-int forward_blocks_per_cu(int kind, bool axis, size_t lds_bytes) {
+int forward_blocks_per_cu(int kind, bool axis, const Dims& d, size_t lds_bytes) {
     int n = 0;
-    const void* k = nullptr;
-    if (kind == FWD_WEIGHT) k = axis ? (const void*)k_forward<FWD_WEIGHT, true> : (const void*)k_forward<FWD_WEIGHT, false>;
-    else if (kind == FWD_PLAIN) k = axis ? (const void*)k_forward<FWD_PLAIN, true> : (const void*)k_forward<FWD_PLAIN, false>;
-    else k = axis ? (const void*)k_forward<FWD_XTT, true, 13, kFwdXttWaves>
-                  : (const void*)k_forward<FWD_XTT, false, 13, kFwdXttWaves>;
-    const int threads = kind == FWD_XTT ? 64 * kFwdXttWaves : 64 * kFwdWaves;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, threads, lds_bytes);
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, forward_kernel(kind, axis, d),
+                                                                      64 * forward_waves(kind), lds_bytes);
     return e == hipSuccess ? n : 0;
 }
 

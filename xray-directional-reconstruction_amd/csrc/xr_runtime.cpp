@@ -364,8 +364,8 @@ int forward_launch(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stri
     if (a.n_sub == 0 && items < 4096) {
         if (ctx->n_cu == 0)
             XR_HIP(ctx, hipDeviceGetAttribute(&ctx->n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device));
-        const int64_t slots = (int64_t)forward_blocks_per_cu(kind, axis, forward_lds_bytes(kind, rows)) * ctx->n_cu;
-        a.n_sub = forward_split(items, slots, 0);
+        const int64_t slots = (int64_t)forward_blocks_per_cu(kind, axis, a.d, forward_lds_bytes(kind, rows)) * ctx->n_cu;
+        a.n_sub = forward_split_alone(items, slots, p->g.n_vox);
     }
     a.n_sub = std::max(a.n_sub, 1);
     if (no_alloc) {
