@@ -29,36 +29,40 @@ void subset_views(int sub, int batch, int P, std::vector<int>& out) {
     for (int j = 0; j < ss; j++) out[j] = (sub + batch * j) % P;
 }
 
+// Workspace of xr_poisson_solve that a context keeps: 512^3 in one piece.
+constexpr int64_t kPoissonBytes = 1200ll << 20;
+
 }  // namespace
 
 int xr_poisson_solve(xr_context* ctx, int n, const float* gx, const float* gy, float* vol) {
     if (!ctx || !gx || !gy || !vol) return fail(ctx, XR_ERR_INVALID, "bad args");
     if (n < 3 || n > 4096) return fail(ctx, XR_ERR_INVALID, "poisson solve needs 3 <= n <= 4096 (got %d)", n);
-    const int M = n - 2;
-    const double h = (double)(M + 1);
-    // S[j][k] = sin(pi (j+1)(k+1) / h), with the product reduced mod 2h so the
-    // argument stays in [0, 2 pi)
-    std::vector<double> S((size_t)M * M), e(M);
-    for (int j = 0; j < M; j++) {
-        for (int k = 0; k < M; k++) {
-            const int64_t m = ((int64_t)(j + 1) * (k + 1)) % (2 * (int64_t)(M + 1));
-            S[(size_t)j * M + k] = std::sin(M_PI * (double)m / h);
-        }
-        e[j] = 2.0 - 2.0 * std::cos(M_PI * (double)(j + 1) / h);
+    const int64_t M = n - 2, He = (M + 1) / 2, Ho = M / 2;
+    // Tables, then the modes of as many slices as fit the workspace.  The
+    // context keeps the buffer (allocating and freeing a gigabyte costs as much
+    // as a solve): at most kPoissonBytes, or one slice where that is larger.
+    const int64_t tables = He * He + He * Ho + M * M;
+    const int64_t slices = std::max<int64_t>(1, std::min<int64_t>(n, (kPoissonBytes / 8 - tables) / (M * M)));
+    const size_t need = (size_t)(tables + slices * M * M);
+    if (ctx->poisson_len < need) {
+        if (ctx->d_poisson) (void)hipFree(ctx->d_poisson);
+        ctx->d_poisson = nullptr;
+        ctx->poisson_len = 0;
+        XR_HIP(ctx, device_malloc((void**)&ctx->d_poisson, need * sizeof(double)));
+        ctx->poisson_len = need;
     }
-    const int64_t slab = (int64_t)n * M * M;
-    DevBuf<double> dS, de, dB, dT;
-    XR_HIP(ctx, dS.alloc(S.size()));
-    XR_HIP(ctx, de.alloc(e.size()));
-    XR_HIP(ctx, dB.alloc(slab));
-    XR_HIP(ctx, dT.alloc(slab));
-    XR_HIP(ctx, hipMemcpyAsync(dS.p, S.data(), S.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    XR_HIP(ctx, hipMemcpyAsync(de.p, e.data(), e.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    // the slice borders are the identity rows with zero right side: zero
-    XR_TRY(timed(ctx, 3, [&] { return launch_fill(vol, (int64_t)n * n * n, 0.0f, ctx->stream); }));
-    XR_TRY(timed(ctx, 3, [&] { return launch_poisson_rhs(gx, gy, dB.p, n, ctx->stream); }));
-    XR_TRY(timed(ctx, 3, [&] { return launch_poisson_dst(dS.p, de.p, dB.p, dT.p, vol, n, ctx->stream); }));
-    // the workspace is freed on return: wait for the kernels that read it
+    double* const Se = ctx->d_poisson;
+    double* const So = Se + He * He;
+    double* const G = So + He * Ho;
+    double* const T = G + M * M;
+    XR_TRY(timed(ctx, 3, [&] { return launch_poisson_tables(Se, So, G, n, ctx->stream); }));
+    XR_TRY(timed(ctx, 3, [&] { return launch_poisson_border(vol, n, ctx->stream); }));
+    for (int64_t z0 = 0; z0 < n; z0 += slices)
+        XR_TRY(timed(ctx, 3, [&] {
+            return launch_poisson_slices(gx, gy, Se, So, G, T, vol, n, (int)z0, (int)std::min<int64_t>(slices, n - z0),
+                                         ctx->stream);
+        }));
+    // the next call, perhaps on another stream, overwrites the workspace
     XR_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return XR_OK;
 }

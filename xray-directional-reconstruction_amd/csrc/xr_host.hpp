@@ -24,6 +24,8 @@ struct xr_context {
     size_t flags_cap = 0;
     double* d_loss = nullptr;
     float* d_scal = nullptr;  // [0] = 1.0f, [1] = max |voxel value| of the last forward launch
+    double* d_poisson = nullptr;  // workspace of xr_poisson_solve (bounded, freed with the context)
+    size_t poisson_len = 0;
     bool timing = false;
     struct Ev {
         int kind;

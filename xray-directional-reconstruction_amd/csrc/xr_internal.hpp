@@ -250,9 +250,10 @@ hipError_t launch_fill(float* p, int64_t n, float value, hipStream_t stream);
 hipError_t launch_scale_views(const float* src, float* dst, const float* coef, int64_t len_view, int n_views,
                               hipStream_t stream);
 hipError_t launch_grad_faces(float* vol, int N1, int ext, float value, hipStream_t stream);
-hipError_t launch_poisson_rhs(const float* g0, const float* g1, double* B, int n, hipStream_t stream);
-hipError_t launch_poisson_dst(const double* S, const double* e, double* B, double* T, float* vol, int n,
-                              hipStream_t stream);
+hipError_t launch_poisson_tables(double* Se, double* So, double* G, int n, hipStream_t stream);
+hipError_t launch_poisson_slices(const float* g0, const float* g1, const double* Se, const double* So, const double* G,
+                                 double* T, float* vol, int n, int z0, int slices, hipStream_t stream);
+hipError_t launch_poisson_border(float* vol, int n, hipStream_t stream);
 // Direction post-processing on 3 channels of n floats (pca.cu:67-106).
 hipError_t launch_md_angles(const float* md, float* angle, int64_t n, hipStream_t stream);
 hipError_t launch_md_normalise(float* md, int64_t n, float eps, hipStream_t stream);

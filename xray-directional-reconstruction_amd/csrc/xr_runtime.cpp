@@ -691,6 +691,7 @@ void xr_context_destroy(xr_context* ctx) {
     if (ctx->d_flags) (void)hipFree(ctx->d_flags);
     if (ctx->d_loss) (void)hipFree(ctx->d_loss);
     if (ctx->d_scal) (void)hipFree(ctx->d_scal);
+    if (ctx->d_poisson) (void)hipFree(ctx->d_poisson);
     delete ctx;
 }
 
