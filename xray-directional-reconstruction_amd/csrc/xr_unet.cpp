@@ -236,12 +236,11 @@ int conv_bwd(xr_unet* n, int i, const __bf16* in, int in_ld, int in_off, const _
     w.Cout = l.Cout;
     w.dw = n->d_g + l.w_off;
     w.ldw = 27 * l.Cin;
+    w.db = n->d_g + l.b_off;
     w.D0 = D0;
     w.D1 = D1;
     w.D2 = D2;
     XR_K(ctx, launch_conv3_wgrad(w, ctx->stream));
-    const int64_t V = (int64_t)D0 * D1 * D2;
-    XR_K(ctx, launch_bias_grad(gout, g_ld, g_off, l.Cout, V, n->d_g + l.b_off, ctx->stream));
     if (!gin) return XR_OK;
     ConvArgs a{};
     a.in = gout;

@@ -41,7 +41,8 @@ struct ConvArgs {
 // takes a fused upsampling source).
 bool conv3_tiled_ok(const ConvArgs& a);
 
-// dw[co * ldw + k] += sum_v gout[v][g_off + co] im2col(in)[v][k]  (k < 27*Cin).
+// dw[co * ldw + k] += sum_v gout[v][g_off + co] im2col(in)[v][k]  (k < 27*Cin),
+// db[co] += sum_v gout[v][g_off + co].
 struct WgradArgs {
     const __bf16* in;
     int in_ld, in_off, Cin;
@@ -49,13 +50,12 @@ struct WgradArgs {
     int g_ld, g_off, Cout;
     float* dw;
     int ldw;
+    float* db;
     int D0, D1, D2;
-    int64_t vox_per_block;  // set by the launcher
 };
 
 hipError_t launch_conv3(const ConvArgs& a, hipStream_t s);
-hipError_t launch_conv3_wgrad(WgradArgs a, hipStream_t s);
-hipError_t launch_bias_grad(const __bf16* g, int ld, int off, int C, int64_t V, float* db, hipStream_t s);
+hipError_t launch_conv3_wgrad(const WgradArgs& a, hipStream_t s);
 hipError_t launch_pool(const __bf16* in, int in_ld, int in_off, int C, int D0, int D1, int D2, __bf16* out,
                        hipStream_t s);
 hipError_t launch_pool_bwd(const __bf16* gp, int C, int D0, int D1, int D2, __bf16* gin, int g_ld, int g_off,

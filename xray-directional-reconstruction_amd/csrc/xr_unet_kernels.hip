@@ -11,11 +11,12 @@
 // (v_mfma_f32_16x16x32_bf16): M = voxels, N = output channels, K = 27*Cin with
 // k = tap*Cin + ci, tap = (d0+1)*9 + (d1+1)*3 + (d2+1).  Cin is a multiple of
 // 8 so the 8 consecutive k of one MFMA lane lie in one tap: one 16-byte load
-// of 8 channels of one neighbour voxel.  Weights are [Cout16][Kpad] BF16 (k
-// fastest, zero padded).  The data gradient is the same kernel on the output
+// of 8 channels of one neighbour voxel.  Weights are [Cout16][Kpad] BF16, zero
+// padded, in the order in which a wave reads them (weight_index): each MFMA
+// operand is one contiguous KB.  The data gradient is the same kernel on the output
 // gradient with mirrored taps and transposed channels (weights [Cin16][K'pad],
 // k' = (26 - tap)*Cout + co); the weight gradient contracts over voxels with
-// both operands transposed through LDS.
+// both operands read transposed from LDS.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -43,6 +44,24 @@ __device__ __forceinline__ bf16x8 zero8() {
     return z;
 }
 
+// Packed position of weight (co, k): operand (k / 32, co / 16) of cout16 / 16 per
+// step, lane (k % 32 / 8) * 16 + co % 16, element k % 8.
+__device__ __forceinline__ int64_t weight_index(int co, int k, int cout16) {
+    return ((int64_t)(k >> 5) * (cout16 >> 4) + (co >> 4)) * 512 + ((k & 31) >> 3) * 128 + (co & 15) * 8 + (k & 7);
+}
+
+// 16 bytes per lane from global memory straight to LDS: lane l's go to lds + 16 l.
+// The caller waits (lds_wait) before the barrier that publishes them.
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) void global_void;
+__device__ __align__(16) __bf16 g_zero8[8];  // source of the padding
+
+__device__ __forceinline__ void lds_load16(const __bf16* src, lds_bf16x8* lds) {
+    __builtin_amdgcn_global_load_lds((global_void*)src, (lds_void*)lds, 16, 0, 0);
+}
+
+__device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // Tap t -> offsets (d0, d1, d2) in {-1, 0, 1}.
 __device__ __forceinline__ void tap_offsets(int t, int& d0, int& d1, int& d2) {
     d0 = t / 9 - 1;
@@ -51,70 +70,116 @@ __device__ __forceinline__ void tap_offsets(int t, int& d0, int& d1, int& d2) {
 }
 
 // ---------------------------------------------------------------------------
-// Forward / data-gradient convolution.  Block: 4 waves, 128 consecutive
-// voxels (32 per wave as two 16-row MFMA tiles) x all output channels (NT
-// tiles of 16).
+// Data-gradient convolution, and the forward one for dims that the chunked
+// kernel below does not take.  K runs in the order k = tap*Cin + ci, so every
+// channel of the input halo is staged in LDS before the first step and read by
+// all 27 taps; the four lane groups of a step look up their (tap, chunk of 8
+// channels) in a table of LDS offsets.  Block: 4 waves with MT 16-voxel MFMA
+// tiles each: 2 x 4 x 32, 2 x 4 x 16 or 2 x 2 x 16 voxels (MT = 4, 2, 1; the last
+// ones reach past the volume), the largest whose halo leaves room for two blocks
+// per CU.  blockIdx.y: pieces of NT 16-channel tiles of the output.
+// Bound by the LDS reads and, at the start of a block, the staging (the other
+// blocks of the CU hide part of it); the weights are prefetched one step ahead.
+// Measured: 24 -> 72 channels at 96^3 335 -> 245 us, 48 -> 144 at 48^3 246 -> 158,
+// 48 -> 48 at 48^3 94 -> 58, 96 -> 96 at 24^3 116 -> 62, against loading every
+// operand from global memory (one 16-byte load per lane, tap and 8 channels);
+// weights as plain rows instead of whole operands: 346 us for the first.
 // ---------------------------------------------------------------------------
-template <int NT>
-__global__ __launch_bounds__(256) void k_conv3(const ConvArgs a) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t V = (int64_t)a.D0 * a.D1 * a.D2;
-    const int64_t vbase = (int64_t)blockIdx.x * 128 + wave * 32;
-    if (vbase >= V) return;
+template <int MT>
+struct ConvTile {
+    static constexpr int T0 = 2, T1 = MT == 1 ? 2 : 4, T2 = MT == 4 ? 32 : 16;
+    static constexpr int H1 = T1 + 2, H2 = T2 + 2, halo = (T0 + 2) * H1 * H2;
+    static constexpr int stride = halo + 4;  // LDS distance of two chunks, 16-byte units
+    static constexpr int64_t lds(int nchunk) { return 16 * (int64_t)stride * nchunk + 4 * 28 * nchunk; }
+};
+
+template <int MT, int NT>
+__global__ __launch_bounds__(256, 2) void k_conv3(const ConvArgs a) {
+    using T = ConvTile<MT>;
+    extern __shared__ bf16x8 conv_lds[];
+    const int nch = a.Cin / 8, nq = 27 * nch;
+    bf16x8* const halo = conv_lds;
+    int* const off = (int*)(conv_lds + T::stride * nch);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 15, kg = lane >> 4;
-    int p0[2], p1[2], p2[2];
-    bool vin[2];
-#pragma unroll
-    for (int ms = 0; ms < 2; ms++) {
-        const int64_t v = vbase + ms * 16 + row;
-        vin[ms] = v < V;
-        const int64_t vv = vin[ms] ? v : 0;
-        p2[ms] = (int)(vv % a.D2);
-        p1[ms] = (int)((vv / a.D2) % a.D1);
-        p0[ms] = (int)(vv / ((int64_t)a.D2 * a.D1));
+    const int nb2 = (a.D2 + T::T2 - 1) / T::T2, nb1 = (a.D1 + T::T1 - 1) / T::T1;
+    const int o2 = blockIdx.x % nb2 * T::T2, o1 = blockIdx.x / nb2 % nb1 * T::T1, o0 = blockIdx.x / (nb2 * nb1) * T::T0;
+    const int co0 = blockIdx.y * (16 * NT), tiles = (a.Cout + 15) / 16;
+    for (int q = threadIdx.x; q < nq; q += 256) {
+        const int tap = q / nch;
+        off[q] = (q - tap * nch) * T::stride + (tap / 9 * T::H1 + tap / 3 % 3) * T::H2 + tap % 3;
     }
-    f32x4 acc[2][NT];
+    for (int v0 = 0; v0 < T::halo; v0 += 256) {
+        const int v = v0 + threadIdx.x;
+        const int g0 = o0 + v / (T::H2 * T::H1) - 1, g1 = o1 + v / T::H2 % T::H1 - 1, g2 = o2 + v % T::H2 - 1;
+        const bool ok = (unsigned)g0 < (unsigned)a.D0 && (unsigned)g1 < (unsigned)a.D1 && (unsigned)g2 < (unsigned)a.D2;
+        const __bf16* const src =
+            ok ? a.in + (((int64_t)g0 * a.D1 + g1) * a.D2 + g2) * a.in_ld + a.in_off : g_zero8;
+        const int step = ok ? 8 : 0;
+        if (v < T::halo)
+            for (int c = 0; c < nch; c++)
+                lds_load16(src + step * c, (lds_bf16x8*)halo + c * T::stride + v0 + 64 * wave);
+    }
+    lds_wait();
+    __syncthreads();
+    const lds_bf16x8* base[MT];
 #pragma unroll
-    for (int ms = 0; ms < 2; ms++)
+    for (int m = 0; m < MT; m++) {
+        const int g = (wave * MT + m) / (T::T2 / 16), half = (wave * MT + m) % (T::T2 / 16);
+        base[m] = (const lds_bf16x8*)halo + (g / T::T1 * T::H1 + g % T::T1) * T::H2 + 16 * half + row;
+    }
+    const __bf16* wop[NT];
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++) acc[ms][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int K = 27 * a.Cin;
-    const __bf16* __restrict__ in = a.in + a.in_off;
-    for (int kc = 0; kc < a.Kpad; kc += 32) {
-        const int k0 = kc + 8 * kg;
-        const int tap = k0 / a.Cin;
-        const int ci = k0 - tap * a.Cin;
-        int d0, d1, d2;
-        tap_offsets(tap, d0, d1, d2);
-        bf16x8 A[2];
+    for (int nt = 0; nt < NT; nt++) wop[nt] = a.w + min((int)blockIdx.y * NT + nt, tiles - 1) * 512 + lane * 8;
+    f32x4 acc[MT][NT];
+    bf16x8 B[NT];
 #pragma unroll
-        for (int ms = 0; ms < 2; ms++) {
-            const int n0 = p0[ms] + d0, n1 = p1[ms] + d1, n2 = p2[ms] + d2;
-            const bool ok = vin[ms] && k0 < K && (unsigned)n0 < (unsigned)a.D0 && (unsigned)n1 < (unsigned)a.D1 &&
-                            (unsigned)n2 < (unsigned)a.D2;
-            const int64_t nv = ((int64_t)n0 * a.D1 + n1) * a.D2 + n2;
-            A[ms] = ok ? *(const bf16x8*)(in + nv * a.in_ld + ci) : zero8();
-        }
+    for (int nt = 0; nt < NT; nt++) {
+#pragma unroll
+        for (int m = 0; m < MT; m++) acc[m][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        B[nt] = *(const bf16x8*)wop[nt];
+    }
+    // one step ahead: the weights and the halo values; two: the LDS offsets
+    const int last = a.Kpad - 32;
+    bf16x8 A[MT];
+    int o = off[min(kg, nq - 1)];
+#pragma unroll
+    for (int m = 0; m < MT; m++) A[m] = kg < nq ? base[m][o] : zero8();
+    o = off[min(4 + kg, nq - 1)];
+    for (int kc = 0; kc <= last; kc += 32) {
+        bf16x8 nextB[NT], nextA[MT];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) nextB[nt] = *(const bf16x8*)(wop[nt] + min(kc + 32, last) * 16 * tiles);
+        const int q = kc / 8 + 4 + kg;
+#pragma unroll
+        for (int m = 0; m < MT; m++) nextA[m] = q < nq ? base[m][o] : zero8();
+        o = off[min(q + 4, nq - 1)];
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
-            const bf16x8 B = *(const bf16x8*)(a.w + (int64_t)(nt * 16 + row) * a.Kpad + k0);
 #pragma unroll
-            for (int ms = 0; ms < 2; ms++) acc[ms][nt] = mfma(A[ms], B, acc[ms][nt]);
+            for (int m = 0; m < MT; m++) acc[m][nt] = mfma(A[m], B[nt], acc[m][nt]);
+            B[nt] = nextB[nt];
         }
+#pragma unroll
+        for (int m = 0; m < MT; m++) A[m] = nextA[m];
     }
     // D layout of the 16x16 MFMA: lane holds column (lane & 15), rows 4*kg + i.
 #pragma unroll
-    for (int ms = 0; ms < 2; ms++) {
+    for (int m = 0; m < MT; m++) {
+        const int g = (wave * MT + m) / (T::T2 / 16), half = (wave * MT + m) % (T::T2 / 16);
+        const int v0 = o0 + g / T::T1, v1 = o1 + g % T::T1;
+        if (v0 >= a.D0 || v1 >= a.D1) continue;
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
-            const int co = nt * 16 + row;
+            const int co = co0 + nt * 16 + row;
             if (co >= a.Cout) continue;
             const float b = a.bias ? a.bias[co] : 0.f;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int64_t v = vbase + ms * 16 + 4 * kg + i;
-                if (v >= V) continue;
-                float val = acc[ms][nt][i] + b;
+                const int v2 = o2 + 16 * half + 4 * kg + i;
+                if (v2 >= a.D2) continue;
+                const int64_t v = ((int64_t)v0 * a.D1 + v1) * a.D2 + v2;
+                float val = acc[m][nt][i] + b;
                 if (a.relu) val = fmaxf(val, 0.f);
                 if (a.mask && !((float)a.mask[v * a.mask_ld + a.mask_off + co] > 0.f)) val = 0.f;
                 __bf16* o = a.out + v * a.out_ld + a.out_off + co;
@@ -220,7 +285,7 @@ __global__ __launch_bounds__(256) void k_conv3_tiled(const ConvArgs a) {
         for (int c = 0; c < CPS; c++) {
             const int cc = st * CPS + c;
             if (cc >= nchunk) break;
-            const __bf16* __restrict__ wc = a.wt + cc * (kTapsPad * 8);
+            const __bf16* __restrict__ wc = a.wt + (int64_t)cc * (kTapsPad / 4 * NT * 512) + lane * 8;
             const lds_bf16x8* const hc = hl + c * kCHalo;
 #pragma unroll
             for (int s = 0; s < kTapsPad / 4; s++) {
@@ -232,7 +297,7 @@ __global__ __launch_bounds__(256) void k_conv3_tiled(const ConvArgs a) {
                 for (int m = 0; m < 4; m++) A[m] = hc[((h0 + d0) * kCH1 + h1[m] + d1) * kCH2 + h2[m] + d2];
 #pragma unroll
                 for (int nt = 0; nt < NT; nt++) {
-                    const bf16x8 B = *(const bf16x8*)(wc + (int64_t)(nt * 16 + row) * a.Ktpad + tap * 8);
+                    const bf16x8 B = *(const bf16x8*)(wc + (s * NT + nt) * 512);
 #pragma unroll
                     for (int m = 0; m < 4; m++) acc[m][nt] = mfma(A[m], B, acc[m][nt]);
                 }
@@ -269,101 +334,150 @@ __global__ void k_pack_tiled(const float* __restrict__ W, int Cin, int Cout, __b
     const int co = (int)(i / Ktpad), k = (int)(i % Ktpad);
     const int cc = k / (kTapsPad * 8), tap = (k / 8) % kTapsPad, c = k % 8;
     const int ci = cc * 8 + c;
-    wt[i] = (__bf16)((co < Cout && tap < 27 && ci < Cin) ? W[((int64_t)co * 27 + tap) * Cin + ci] : 0.f);
+    wt[weight_index(co, k, cout16)] = (__bf16)((co < Cout && tap < 27 && ci < Cin) ? W[((int64_t)co * 27 + tap) * Cin + ci] : 0.f);
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient: dw[co][k] += sum_v gout[v][co] * im2col(in)[v][k].
-// Block: 4 waves; all output channels (MT tiles of 16) x 64 k columns (16 per
-// wave) over a slab of voxels, 32 voxels per step.  Both operands are staged
-// transposed in LDS ([channel][voxel]) so that each MFMA lane reads 8
-// consecutive voxels with one 16-byte LDS load.  Partial sums are added to dw
-// with FP32 atomics (the summation order of the slabs is not fixed).
+// Weight and bias gradient: dw[co][tap][ci] += sum_v gout[v][co] in[v + tap][ci],
+// db[co] += sum_v gout[v][co].  A contraction over voxels: both MFMA operands
+// need 8 consecutive voxels of one channel per lane, while the tensors (and
+// their LDS copies) are channels-last.  The transposed LDS read
+// ds_read_b64_tr_b16 gives them: of the 4 voxels x 16 channels that 16 lanes
+// point at, lane l receives channel l of the 4 voxels.  A tap is an offset of
+// the row address.
+// Block: 4 waves, 32 output x 32 input channels (blockIdx.y), tiles of 2 (D0) x
+// 4 (D1) x 32 (D2) voxels, a stride of gridDim.x tiles; a tile's input halo (4
+// x 6 x 34 voxels) and output gradient are staged once for all 27 taps.  Wave w
+// accumulates taps 7 w .. 7 w + 6 (2 x 2 tiles each) over all its tiles; the
+// 28th tap is a row of ones, whose sums are the bias gradient.  Partial sums are
+// added with FP32 atomics (their order is not fixed).
+// Bound by LDS reads (one b64 per MFMA) and staging, which goes from global
+// memory straight to LDS (through registers, with a branch per load: twice the
+// time).  Measured: 72 -> 24 channels at 96^3 1340 + 185 (bias) -> 296 us, 144 ->
+// 48 at 48^3 398 + 20 -> 142, against a block per output tile that built both
+// transposed operands in LDS for every tap.
 // ---------------------------------------------------------------------------
-constexpr int kWgVox = 32;          // voxels per step
-constexpr int kWgRow = kWgVox + 8;  // LDS row stride (bf16), padded
+constexpr int kWgCh = 32;  // channels per block, both sides; LDS row of one voxel
+constexpr int kWgTaps = 7;  // per wave
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
-template <int MT>
-__global__ __launch_bounds__(256) void k_conv3_wgrad(const WgradArgs a) {
-    extern __shared__ __bf16 wg_smem[];
-    lds_bf16* const gT = (lds_bf16*)wg_smem;                    // [MT*16][kWgRow]
-    lds_bf16* const iT = (lds_bf16*)wg_smem + MT * 16 * kWgRow;  // [64][kWgRow]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int row = lane & 15, kg = lane >> 4;
-    const int kbase = blockIdx.x * 64;
-    const int64_t V = (int64_t)a.D0 * a.D1 * a.D2;
-    const int64_t v_beg = (int64_t)blockIdx.y * a.vox_per_block;
-    const int64_t v_end = v_beg + a.vox_per_block < V ? v_beg + a.vox_per_block : V;
-    const int K = 27 * a.Cin;
-    const int cg_out = a.Cout / 8;  // 8-channel groups of gout
-    // rows of gT beyond Cout stay zero
-    for (int i = tid; i < MT * 16 * kWgRow; i += 256) gT[i] = (__bf16)0.0f;
-    f32x4 acc[MT];
+// LDS voxel records of 4 16-byte pieces; the halves of a record are swapped for
+// odd groups of 8 voxels, so that the 32 lanes of one read (4 voxels of each of
+// two groups) cover all banks.
+__device__ __forceinline__ int wg_piece(int v, int piece) { return piece ^ ((v >> 2) & 2); }
+
+// Eight consecutive voxels of channel 16 half + (lane & 15), for the lane's
+// voxel group 8 (lane >> 4) from voxel v0 on; lv, lc: lane's part of the address.
+__device__ __forceinline__ bf16x8 voxels8(const lds_bf16* p, int v, int half, int lc) {
+    const lds_bf16* const q0 = p + v * kWgCh + ((((v >> 3) & 1) ^ half) << 4) + lc;
+    const lds_bf16* const q1 = p + (v + 4) * kWgCh + (((((v + 4) >> 3) & 1) ^ half) << 4) + lc;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)q0);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)q1);
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// One tile: taps of this wave over its 8 rows of 32 voxels; NM x NN used 16-channel tiles.
+template <int NM, int NN>
+__device__ __forceinline__ void wgrad_tile(f32x4 (&acc)[kWgTaps][2][2], const lds_bf16* halo, const lds_bf16* grad,
+                                           int wave, int lane) {
+    const int li = lane & 15, lv = 8 * (lane >> 4) + (li >> 2), lc = 4 * (li & 3);
+    bf16x8 ones;
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // this thread's im2col column group (fixed over the slab): 32 voxels x 8 groups
-    const int iv = tid >> 3, ig = tid & 7;
-    const int k0 = kbase + 8 * ig;
-    const bool kin = k0 < K;
-    const int tap = kin ? k0 / a.Cin : 0;
-    const int ci = kin ? k0 - tap * a.Cin : 0;
-    int d0, d1, d2;
-    tap_offsets(tap, d0, d1, d2);
-    for (int64_t v0 = v_beg; v0 < v_end; v0 += kWgVox) {
-        __syncthreads();
-        // stage gout[v0 .. v0+31][0 .. Cout) transposed
-        for (int i = tid; i < kWgVox * cg_out; i += 256) {
-            const int vv = i / cg_out, g = i - vv * cg_out;
-            const int64_t v = v0 + vv;
-            const bf16x8 x = (v < v_end) ? *(const bf16x8*)(a.gout + v * a.g_ld + a.g_off + 8 * g) : zero8();
+    for (int j = 0; j < 8; j++) ones[j] = (__bf16)1.0f;
+#pragma unroll 1
+    for (int r = 0; r < kCT0 * kCT1; r++) {
+        bf16x8 A[NM];
 #pragma unroll
-            for (int j = 0; j < 8; j++) gT[(8 * g + j) * kWgRow + vv] = x[j];
+        for (int m = 0; m < NM; m++) A[m] = voxels8(grad, r * kCT2 + lv, m, lc);
+        const int h = (r / kCT1 * kCH1 + r % kCT1) * kCH2 + lv;
+#pragma unroll
+        for (int t = 0; t < kWgTaps; t++) {
+            const int tap = min(kWgTaps * wave + t, 26);
+            const int v = h + (tap / 9 * kCH1 + tap / 3 % 3) * kCH2 + tap % 3;
+#pragma unroll
+            for (int n = 0; n < NN; n++) {
+                bf16x8 B = voxels8(halo, v, n, lc);
+                if (n == 0 && t == kWgTaps - 1) B = wave == 3 ? ones : B;
+#pragma unroll
+                for (int m = 0; m < NM; m++) acc[t][m][n] = mfma(A[m], B, acc[t][m][n]);
+            }
         }
-        // stage im2col[v0 .. v0+31][kbase .. kbase+63] transposed
-        {
-            const int64_t v = v0 + iv;
-            bf16x8 x = zero8();
-            if (kin && v < v_end) {
-                const int p2 = (int)(v % a.D2), p1 = (int)((v / a.D2) % a.D1), p0 = (int)(v / ((int64_t)a.D2 * a.D1));
-                const int n0 = p0 + d0, n1 = p1 + d1, n2 = p2 + d2;
-                if ((unsigned)n0 < (unsigned)a.D0 && (unsigned)n1 < (unsigned)a.D1 && (unsigned)n2 < (unsigned)a.D2) {
-                    const int64_t nv = ((int64_t)n0 * a.D1 + n1) * a.D2 + n2;
-                    x = *(const bf16x8*)(a.in + nv * a.in_ld + a.in_off + ci);
+    }
+}
+
+__global__ __launch_bounds__(256, 2) void k_conv3_wgrad(const WgradArgs a) {
+    __shared__ __align__(16) __bf16 halo[kCHalo * kWgCh];
+    __shared__ __align__(16) __bf16 grad[kCT0 * kCT1 * kCT2 * kWgCh];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nci = (a.Cin + kWgCh - 1) / kWgCh;
+    const int ci0 = (blockIdx.y % nci) * kWgCh, co0 = (blockIdx.y / nci) * kWgCh;
+    const int n1 = (a.D1 + kCT1 - 1) / kCT1, n2 = (a.D2 + kCT2 - 1) / kCT2;
+    const int tiles = (a.D0 + kCT0 - 1) / kCT0 * n1 * n2;
+    const bool two_ci = ci0 + 16 < a.Cin, two_co = co0 + 16 < a.Cout;
+    f32x4 acc[kWgTaps][2][2];
+#pragma unroll
+    for (int t = 0; t < kWgTaps; t++)
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) acc[t][m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const lds_bf16* const hl = (const lds_bf16*)halo;
+    const lds_bf16* const gl = (const lds_bf16*)grad;
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int o2 = tile % n2 * kCT2, o1 = tile / n2 % n1 * kCT1, o0 = tile / (n2 * n1) * kCT0;
+        __syncthreads();  // the previous tile's reads are done
+        // four pieces of 8 channels per voxel; zero outside the volume and past the channels
+        for (int i0 = 0; i0 < kCHalo * 4; i0 += 256) {
+            const int i = i0 + threadIdx.x, v = i >> 2, c = ci0 + 8 * wg_piece(v, i & 3);
+            const int g0 = o0 + v / (kCH2 * kCH1) - 1, g1 = o1 + v / kCH2 % kCH1 - 1, g2 = o2 + v % kCH2 - 1;
+            const bool ok = c < a.Cin && (unsigned)g0 < (unsigned)a.D0 && (unsigned)g1 < (unsigned)a.D1 &&
+                            (unsigned)g2 < (unsigned)a.D2;
+            const __bf16* const src =
+                ok ? a.in + (((int64_t)g0 * a.D1 + g1) * a.D2 + g2) * a.in_ld + a.in_off + c : g_zero8;
+            if (i < kCHalo * 4) lds_load16(src, (lds_bf16x8*)halo + i0 + 64 * wave);
+        }
+#pragma unroll
+        for (int i0 = 0; i0 < kCT0 * kCT1 * kCT2 * 4; i0 += 256) {
+            const int i = i0 + threadIdx.x, v = i >> 2, c = co0 + 8 * wg_piece(v, i & 3);
+            const int g0 = o0 + v / (kCT2 * kCT1), g1 = o1 + v / kCT2 % kCT1, g2 = o2 + v % kCT2;
+            const bool ok = c < a.Cout && g0 < a.D0 && g1 < a.D1 && g2 < a.D2;
+            const __bf16* const src =
+                ok ? a.gout + (((int64_t)g0 * a.D1 + g1) * a.D2 + g2) * a.g_ld + a.g_off + c : g_zero8;
+            lds_load16(src, (lds_bf16x8*)grad + i0 + 64 * wave);
+        }
+        lds_wait();
+        __syncthreads();
+        if (two_ci) {
+            if (two_co) wgrad_tile<2, 2>(acc, hl, gl, wave, lane);
+            else wgrad_tile<1, 2>(acc, hl, gl, wave, lane);
+        } else {
+            if (two_co) wgrad_tile<2, 1>(acc, hl, gl, wave, lane);
+            else wgrad_tile<1, 1>(acc, hl, gl, wave, lane);
+        }
+    }
+    // D layout of the 16x16 MFMA: lane holds column (lane & 15), rows 4*kg + i
+    const int li = lane & 15, kg = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < kWgTaps; t++) {
+        const int tap = kWgTaps * wave + t;
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int co = co0 + m * 16 + 4 * kg + i;
+                if (co >= a.Cout) continue;
+                if (tap < 27) {
+#pragma unroll
+                    for (int n = 0; n < 2; n++) {
+                        const int ci = ci0 + n * 16 + li;
+                        if (ci < a.Cin) atomicAdd(a.dw + (int64_t)co * a.ldw + tap * a.Cin + ci, acc[t][m][n][i]);
+                    }
+                } else if (ci0 == 0 && li == 0) {
+                    atomicAdd(a.db + co, acc[t][m][0][i]);
                 }
             }
-#pragma unroll
-            for (int j = 0; j < 8; j++) iT[(8 * ig + j) * kWgRow + iv] = x[j];
-        }
-        __syncthreads();
-        const bf16x8 B = *(const lds_bf16x8*)(iT + (16 * wave + row) * kWgRow + 8 * kg);
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            const bf16x8 A = *(const lds_bf16x8*)(gT + (mt * 16 + row) * kWgRow + 8 * kg);
-            acc[mt] = mfma(A, B, acc[mt]);
-        }
     }
-    const int k = kbase + 16 * wave + row;
-    if (k >= K) return;
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int co = mt * 16 + 4 * kg + i;
-            if (co < a.Cout) atomicAdd(a.dw + (int64_t)co * a.ldw + k, acc[mt][i]);
-        }
-    }
-}
-
-// db[c] += sum_v g[v][c]; block = C threads (one per channel) over a voxel slab.
-__global__ void k_bias_grad(const __bf16* __restrict__ g, int ld, int off, int C, int64_t V, int64_t per_block,
-                            float* db) {
-    const int c = threadIdx.x;
-    if (c >= C) return;
-    const int64_t v0 = (int64_t)blockIdx.x * per_block;
-    const int64_t v1 = v0 + per_block < V ? v0 + per_block : V;
-    float s = 0.f;
-    for (int64_t v = v0; v < v1; v++) s += (float)g[v * ld + off + c];
-    atomicAdd(db + c, s);
 }
 
 // 2x2x2 average pooling: out[p][c] = mean of the 8 children (dims halve).
@@ -469,6 +583,16 @@ __global__ void k_input8(const float* __restrict__ x, int64_t V, float inv_scale
     *(bf16x8*)(x8 + v * 8) = o;
 }
 
+// Sum of l over a block of 256 threads, added to *out by one atomic (FP64 atomics
+// to one address serialise: one per wave of a 128^3 volume took 100 us).
+__device__ __forceinline__ void block_add(double l, double* out) {
+    __shared__ double part[4];
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = l;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(out, (part[0] + part[1]) + (part[2] + part[3]));
+}
+
 // Output head (1x1x1 conv, C -> 1) with the residual: y = x + scale*(w.e[v] + b),
 // w[C] = b.  Loss mode (t != null): r = (x/scale + w.e + b) - t/scale,
 // loss += r^2, g[v] = 2 r / V (normalised units).
@@ -476,9 +600,8 @@ template <int C>
 __global__ __launch_bounds__(256) void k_head(const __bf16* __restrict__ e, int64_t V, const float* __restrict__ w,
                                               const float* __restrict__ x, float scale, float* __restrict__ y,
                                               const float* __restrict__ t, float* g, double* loss) {
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     double l = 0.0;
-    if (v < V) {
+    for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < V; v += (int64_t)gridDim.x * 256) {
         float f = w[C];
 #pragma unroll
         for (int c = 0; c < C; c += 8) {
@@ -490,14 +613,11 @@ __global__ __launch_bounds__(256) void k_head(const __bf16* __restrict__ e, int6
         if (y) y[v] = x[v] + scale * f;
         if (t) {
             const float r = (x[v] * inv + f) - t[v] * inv;
-            l = (double)r * (double)r;
+            l += (double)r * (double)r;
             g[v] = 2.0f * r / (float)V;
         }
     }
-    if (loss) {
-        for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
-        if ((threadIdx.x & 63) == 0) atomicAdd(loss, l);
-    }
+    if (loss) block_add(l, loss);
 }
 
 // Head backward: ge[v][c] = g[v] w[c] (e[v][c] > 0); dw[c] += sum_v g[v] e[v][c];
@@ -549,7 +669,7 @@ __global__ void k_pack(const float* __restrict__ W, int Cin, int Cout, __bf16* w
     const int K = 27 * Cin, Kd = 27 * Cout;
     if (i < nf) {
         const int co = (int)(i / Kpad), k = (int)(i % Kpad);
-        wf[i] = (__bf16)((co < Cout && k < K) ? W[(int64_t)co * K + k] : 0.f);
+        wf[weight_index(co, k, cout16)] = (__bf16)((co < Cout && k < K) ? W[(int64_t)co * K + k] : 0.f);
     } else if (wd && i < nf + nd) {
         const int64_t j = i - nf;
         const int ci = (int)(j / Kdpad), kd = (int)(j % Kdpad);
@@ -558,7 +678,7 @@ __global__ void k_pack(const float* __restrict__ W, int Cin, int Cout, __bf16* w
             const int tp = kd / Cout, co = kd % Cout;
             val = W[(int64_t)co * K + (26 - tp) * Cin + ci];
         }
-        wd[j] = (__bf16)val;
+        wd[weight_index(ci, kd, cin16)] = (__bf16)val;
     }
 }
 
@@ -579,8 +699,7 @@ __global__ void k_adam(float* p, const float* g, float* m, float* v, int64_t n, 
 __global__ __launch_bounds__(256) void k_sum(const float* __restrict__ x, int64_t n, double* out) {
     double s = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) s += x[i];
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-    if ((threadIdx.x & 63) == 0) atomicAdd(out, s);
+    block_add(s, out);
 }
 
 inline unsigned blocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -591,6 +710,31 @@ bool conv3_tiled_ok(const ConvArgs& a) {
     const int nt = (a.Cout + 15) / 16;
     return a.wt && a.D0 % kCT0 == 0 && a.D1 % kCT1 == 0 && a.D2 % kCT2 == 0 &&
            a.Ktpad == a.Cin / 8 * kTapsPad * 8 && nt <= 6;
+}
+
+template <int MT, int NT>
+hipError_t conv3_run(const ConvArgs& a, unsigned tiles, int pieces, hipStream_t s) {
+    hipLaunchKernelGGL((k_conv3<MT, NT>), dim3(tiles, pieces), dim3(256), ConvTile<MT>::lds(a.Cin / 8), s, a);
+    return hipGetLastError();
+}
+
+template <int MT>
+hipError_t conv3_pieces(const ConvArgs& a, int nt, hipStream_t s) {
+    using T = ConvTile<MT>;
+    const int64_t tiles = (int64_t)((a.D0 + T::T0 - 1) / T::T0) * ((a.D1 + T::T1 - 1) / T::T1) * ((a.D2 + T::T2 - 1) / T::T2);
+    if (tiles > INT32_MAX) return hipErrorInvalidValue;
+    // at most 6 output tiles per block (accumulators in registers), fewer where
+    // the volume alone gives less than two blocks per CU
+    const int want = (int)std::max<int64_t>((nt + 5) / 6, std::min<int64_t>(nt, (512 + tiles - 1) / tiles));
+    const int per = (nt + want - 1) / want, pieces = (nt + per - 1) / per;
+    switch (per) {
+        case 1: return conv3_run<MT, 1>(a, (unsigned)tiles, pieces, s);
+        case 2: return conv3_run<MT, 2>(a, (unsigned)tiles, pieces, s);
+        case 3: return conv3_run<MT, 3>(a, (unsigned)tiles, pieces, s);
+        case 4: return conv3_run<MT, 4>(a, (unsigned)tiles, pieces, s);
+        case 5: return conv3_run<MT, 5>(a, (unsigned)tiles, pieces, s);
+        default: return conv3_run<MT, 6>(a, (unsigned)tiles, pieces, s);
+    }
 }
 
 hipError_t launch_conv3(const ConvArgs& a, hipStream_t s) {
@@ -632,66 +776,27 @@ hipError_t launch_conv3(const ConvArgs& a, hipStream_t s) {
         }
         return hipGetLastError();
     }
-    const dim3 grid(blocks(V, 128));
-    switch (nt) {
-#define XR_CONV(N) \
-    case N: hipLaunchKernelGGL(k_conv3<N>, grid, dim3(256), 0, s, a); break;
-        XR_CONV(1)
-        XR_CONV(2)
-        XR_CONV(3)
-        XR_CONV(4)
-        XR_CONV(5)
-        XR_CONV(6)
-        XR_CONV(7)
-        XR_CONV(8)
-        XR_CONV(9)
-#undef XR_CONV
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    if (nt > 9 || a.Cin / 8 > 24) return hipErrorInvalidValue;
+    // the largest tile whose halo of all channels leaves room for two blocks in
+    // a CU's 160 KB; the smallest tile takes 24 chunks in 110 KB
+    const int nch = a.Cin / 8;
+    if (ConvTile<4>::lds(nch) <= 80 * 1024) return conv3_pieces<4>(a, nt, s);
+    if (ConvTile<2>::lds(nch) <= 80 * 1024) return conv3_pieces<2>(a, nt, s);
+    return conv3_pieces<1>(a, nt, s);
 }
 
-hipError_t launch_conv3_wgrad(WgradArgs a, hipStream_t s) {
+hipError_t launch_conv3_wgrad(const WgradArgs& a, hipStream_t s) {
     const int64_t V = (int64_t)a.D0 * a.D1 * a.D2;
     if (V == 0) return hipSuccess;
     if (a.Cin % 8 != 0 || a.Cout % 8 != 0 || a.in_ld % 8 != 0 || a.in_off % 8 != 0 || a.g_ld % 8 != 0 ||
         a.g_off % 8 != 0 || a.ldw < 27 * a.Cin)
         return hipErrorInvalidValue;
-    const int mt = (a.Cout + 15) / 16;
-    const int kblocks = (27 * a.Cin + 63) / 64;
-    // slabs: about 2048 blocks in all, whole 32-voxel steps
-    int64_t slabs = std::max<int64_t>(1, std::min<int64_t>((V + kWgVox - 1) / kWgVox, 2048 / kblocks + 1));
-    int64_t per = (V + slabs - 1) / slabs;
-    per = ((per + kWgVox - 1) / kWgVox) * kWgVox;
-    slabs = (V + per - 1) / per;
-    a.vox_per_block = per;
-    const dim3 grid((unsigned)kblocks, (unsigned)slabs);
-    const size_t lds = (size_t)(mt * 16 + 64) * kWgRow * sizeof(__bf16);
-    switch (mt) {
-#define XR_WG(M) \
-    case M: hipLaunchKernelGGL(k_conv3_wgrad<M>, grid, dim3(256), lds, s, a); break;
-        XR_WG(1)
-        XR_WG(2)
-        XR_WG(3)
-        XR_WG(4)
-        XR_WG(5)
-        XR_WG(6)
-        XR_WG(7)
-        XR_WG(8)
-        XR_WG(9)
-#undef XR_WG
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_bias_grad(const __bf16* g, int ld, int off, int C, int64_t V, float* db, hipStream_t s) {
-    if (V == 0) return hipSuccess;
-    if (C > 1024) return hipErrorInvalidValue;
-    const int64_t nb = std::min<int64_t>(1024, (V + 255) / 256);
-    const int64_t per = (V + nb - 1) / nb;
-    hipLaunchKernelGGL(k_bias_grad, dim3(blocks(V, (int)per)), dim3(((C + 63) / 64) * 64), 0, s, g, ld, off, C, V,
-                       per, db);
+    const int64_t tiles = (int64_t)((a.D0 + kCT0 - 1) / kCT0) * ((a.D1 + kCT1 - 1) / kCT1) * ((a.D2 + kCT2 - 1) / kCT2);
+    if (tiles > INT32_MAX) return hipErrorInvalidValue;
+    const int pairs = ((a.Cin + kWgCh - 1) / kWgCh) * ((a.Cout + kWgCh - 1) / kWgCh);
+    // two blocks per CU in all: more would add more partial sums than they save
+    const int64_t slabs = std::max<int64_t>(1, std::min<int64_t>(tiles, (512 + pairs - 1) / pairs));
+    hipLaunchKernelGGL(k_conv3_wgrad, dim3((unsigned)slabs, pairs), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -760,9 +865,11 @@ hipError_t launch_input8(const float* x, int64_t V, float inv_scale, __bf16* x8,
 hipError_t launch_head(const __bf16* e, int C, int64_t V, const float* w, const float* x, float scale, float* y,
                        const float* t, float* g, double* loss, hipStream_t s) {
     if (V == 0) return hipSuccess;
+    // with a loss, a few blocks per CU (each adds to it once)
+    const unsigned nb = (unsigned)std::min<int64_t>((V + 255) / 256, loss ? 1024 : INT32_MAX);
     switch (C) {
 #define XR_HEAD(N) \
-    case N: hipLaunchKernelGGL(k_head<N>, dim3(blocks(V, 256)), dim3(256), 0, s, e, V, w, x, scale, y, t, g, loss); break;
+    case N: hipLaunchKernelGGL(k_head<N>, dim3(nb), dim3(256), 0, s, e, V, w, x, scale, y, t, g, loss); break;
         XR_HEAD(8)
         XR_HEAD(16)
         XR_HEAD(24)
@@ -814,7 +921,7 @@ hipError_t launch_adam(float* p, const float* g, float* m, float* v, int64_t n, 
 
 hipError_t launch_sum(const float* x, int64_t n, double* out, hipStream_t s) {
     if (n == 0) return hipSuccess;
-    const int64_t nb = std::min<int64_t>(2048, (n + 255) / 256);
+    const int64_t nb = std::min<int64_t>(512, (n + 1023) / 1024);
     hipLaunchKernelGGL(k_sum, dim3((unsigned)nb), dim3(256), 0, s, x, n, out);
     return hipGetLastError();
 }
