@@ -1971,81 +1971,103 @@ __global__ __launch_bounds__(256) void k_absmax_seg(const float* const* __restri
 // matrix cores: C[row][u] = sum_j A[row][j] T[j][u], A the weighted rows and
 // T[j][u] = h(u - j) taken from a tap window in LDS (the Toeplitz operand is
 // never stored).  h(m) = taps[|m|] (a linear convolution) or taps[m mod U]
-// (circular), zero for |m| >= U.  Block tile 64 rows x 128 columns, four
-// waves of 32 x 64, K steps of 32 samples.  v_mfma_f32_16x16x4f32 operands:
-// A from lane (row lane&15, k lane>>4), B from lane (k lane>>4, column
-// lane&15); the result lane holds column lane&15, rows 4*(lane>>4) + r.
+// (circular), zero for |m| >= U.  v_mfma_f32_16x16x4f32 operands: A from lane
+// (row lane&15, k lane>>4), B from lane (k lane>>4, column lane&15); the result
+// lane holds column lane&15, rows 4*(lane>>4) + r.
+// Block: 64 rows x 64 NT columns, four waves of 64 rows x 16 NT columns, K steps
+// of 32 samples; the next step's samples are loaded during this step's products
+// (rows contiguous over 32 lanes).  The wider the block, the fewer times a row is
+// staged: with NT = 8 and U <= 512, once.
+// Bound by the FP32 matrix rate.  Measured, 401 x 451 rows of 487: 1662 -> 903 us
+// (95 TFLOP/s of 153 without the padding) against 64 x 128 tiles that staged
+// eight strided samples per lane between two barriers, four times per row.
 // ---------------------------------------------------------------------------
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-constexpr int kFiltBM = 64, kFiltBN = 128, kFiltBK = 32, kFiltAStride = kFiltBK + 1;
-constexpr int kFiltWin = kFiltBN + kFiltBK - 1;  // taps one K step of one block touches
+constexpr int kFiltBM = 64, kFiltBK = 32, kFiltAStride = kFiltBK + 1;
 
-__global__ __launch_bounds__(256) void k_fdk_filter(const float* __restrict__ src, float* __restrict__ dst,
-                                                   const float* __restrict__ weight, const float* __restrict__ taps,
-                                                   int U, int V, const int32_t* __restrict__ views, int n_rows,
-                                                   int row_base, int code_base, int circular) {
+template <int NT>
+__global__ __launch_bounds__(256, 2) void k_fdk_filter(const float* __restrict__ src, float* __restrict__ dst,
+                                                       const float* __restrict__ weight,
+                                                       const float* __restrict__ taps, int U, int V,
+                                                       const int32_t* __restrict__ views, int n_rows, int row_base,
+                                                       int code_base, int circular) {
+    constexpr int BN = 64 * NT, win = BN + kFiltBK - 1;  // win: taps one K step of the block touches
+    constexpr int nr = kFiltBM / 8, nh = (win + 255) / 256;
     __shared__ float As[kFiltBM * kFiltAStride];
-    __shared__ float Hs[kFiltWin + 1];
+    __shared__ float Hs[nh * 256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int row0 = row_base + blockIdx.y * kFiltBM, col0 = blockIdx.x * kFiltBN;
-    // this thread loads row lr, samples lj .. lj+7 of each K step
-    const int lr = tid >> 2, lj = (tid & 3) * 8;
-    int64_t roff = -1;
-    int wv = 0;
-    if (row0 + lr < n_rows) {
-        const int slot = (row0 + lr) / V;
-        wv = row0 + lr - slot * V;
-        roff = ((int64_t)(views[slot] - code_base) * V + wv) * U;
+    const int row0 = row_base + blockIdx.y * kFiltBM, col0 = blockIdx.x * BN;
+    // this thread loads sample sj of rows sr + 8 i of each K step
+    const int sj = tid & 31, sr = tid >> 5;
+    int64_t roff[nr];
+    int woff[nr];
+#pragma unroll
+    for (int i = 0; i < nr; i++) {
+        const int row = min(row0 + sr + 8 * i, n_rows - 1);  // rows past the last are computed and not stored
+        const int slot = row / V, v = row - slot * V;
+        roff[i] = ((int64_t)(views[slot] - code_base) * V + v) * U;
+        woff[i] = v;
     }
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;  // the wave's 32 x 64 sub-tile
+    const int wn = wave * (16 * NT);  // the wave's columns
     const int li = lane & 15, lk = lane >> 4;
-    f32x4_t acc[2][4];
+    f32x4_t acc[4][NT];
 #pragma unroll
-    for (int mt = 0; mt < 2; mt++)
+    for (int mt = 0; mt < 4; mt++)
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int nt = 0; nt < NT; nt++) acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float x[nr], w[nr], h[nh];
+    auto fetch = [&](int j0) XR_INLINE {
+        const int j = j0 + sj, jj = min(j, U - 1);
+#pragma unroll
+        for (int i = 0; i < nr; i++) x[i] = src[roff[i] + jj];
+        if (weight) {
+#pragma unroll
+            for (int i = 0; i < nr; i++) w[i] = weight[(int64_t)woff[i] * U + jj];
+        }
+        // Hs[t] = h(m), m = col0 - j0 - (BK - 1) + t
+#pragma unroll
+        for (int i = 0; i < nh; i++) {
+            const int m = col0 - j0 - (kFiltBK - 1) + tid + 256 * i, am = abs(m);
+            const float tap = taps[min(circular && m < 0 ? max(m + U, 0) : am, U - 1)];
+            h[i] = am < U ? tap : 0.f;
+        }
+    };
+    fetch(0);
     for (int j0 = 0; j0 < U; j0 += kFiltBK) {
         __syncthreads();  // the previous K step is done with As and Hs
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const int j = j0 + lj + q;
-            float x = 0.f;
-            if (roff >= 0 && j < U) {
-                x = src[roff + j];
-                if (weight) x *= weight[(int64_t)wv * U + j];
-            }
-            As[lr * kFiltAStride + lj + q] = x;
+        for (int i = 0; i < nr; i++) {
+            const float xw = weight ? x[i] * w[i] : x[i];
+            As[(sr + 8 * i) * kFiltAStride + sj] = j0 + sj < U ? xw : 0.f;
         }
-        // Hs[t] = h(m), m = col0 - j0 - (BK - 1) + t
-        if (tid < kFiltWin) {
-            const int m = col0 - j0 - (kFiltBK - 1) + tid, am = abs(m);
-            Hs[tid] = (am < U) ? taps[circular ? ((m % U) + U) % U : am] : 0.f;
-        }
+#pragma unroll
+        for (int i = 0; i < nh; i++) Hs[tid + 256 * i] = h[i];
         __syncthreads();
+        if (j0 + kFiltBK < U) fetch(j0 + kFiltBK);
 #pragma unroll
         for (int kk = 0; kk < kFiltBK; kk += 4) {
-            float a[2], b[4];
+            float a[4], b[NT];
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++) a[mt] = As[(wm + mt * 16 + li) * kFiltAStride + kk + lk];
+            for (int mt = 0; mt < 4; mt++) a[mt] = As[(mt * 16 + li) * kFiltAStride + kk + lk];
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) b[nt] = Hs[wn + nt * 16 + li - kk - lk + (kFiltBK - 1)];
+            for (int nt = 0; nt < NT; nt++) b[nt] = Hs[wn + nt * 16 + li - kk - lk + (kFiltBK - 1)];
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++)
+            for (int mt = 0; mt < 4; mt++)
 #pragma unroll
-                for (int nt = 0; nt < 4; nt++)
+                for (int nt = 0; nt < NT; nt++)
                     acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
         }
     }
 #pragma unroll
-    for (int mt = 0; mt < 2; mt++)
+    for (int mt = 0; mt < 4; mt++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int row = row0 + wm + mt * 16 + 4 * lk + r;
+            const int row = row0 + mt * 16 + 4 * lk + r;
             if (row >= n_rows) continue;
             const int slot = row / V, v = row - slot * V;
             const int64_t off = ((int64_t)(views[slot] - code_base) * V + v) * U;
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) {
+            for (int nt = 0; nt < NT; nt++) {
                 const int col = col0 + wn + nt * 16 + li;
                 if (col < U) dst[off + col] = acc[mt][nt][r];
             }
@@ -2987,12 +3009,20 @@ hipError_t launch_fdk_filter(const float* src, float* dst, const float* weight, 
                              const int32_t* views, int n_views, int code_base, int circular, hipStream_t stream) {
     const int64_t n_rows = (int64_t)n_views * V;
     if (n_rows > INT32_MAX - kFiltBM) return hipErrorInvalidValue;
+    // the widest block that pads the columns no more than a narrower one does and
+    // leaves two blocks per CU (512 of 64 rows)
+    int nt = 2;
+    for (int t = 4; t <= 8; t *= 2) {
+        const int64_t cols = (U + 64 * t - 1) / (64 * t), narrow = (U + 64 * nt - 1) / (64 * nt);
+        if (cols * t <= narrow * nt && cols * ((n_rows + kFiltBM - 1) / kFiltBM) >= 512) nt = t;
+    }
+    const auto kernel = nt == 8 ? k_fdk_filter<8> : nt == 4 ? k_fdk_filter<4> : k_fdk_filter<2>;
     // row tiles in launches of at most 65535 tiles (the grid's y limit)
     const int64_t per_launch = (int64_t)65535 * kFiltBM;
     for (int64_t base = 0; base < n_rows; base += per_launch) {
         const int64_t rows = std::min(per_launch, n_rows - base);
-        const dim3 grid((U + kFiltBN - 1) / kFiltBN, (unsigned)((rows + kFiltBM - 1) / kFiltBM));
-        hipLaunchKernelGGL(k_fdk_filter, grid, dim3(256), 0, stream, src, dst, weight, taps, U, V, views, (int)n_rows,
+        const dim3 grid((U + 64 * nt - 1) / (64 * nt), (unsigned)((rows + kFiltBM - 1) / kFiltBM));
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, src, dst, weight, taps, U, V, views, (int)n_rows,
                            (int)base, code_base, circular);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
