@@ -93,7 +93,7 @@ int xr_grad_reconstruct(xr_context* ctx, const xr_geometry* g, const xr_scan* s,
     const int64_t V1 = (int64_t)N1 * N1 * N1, lenP = (int64_t)g->n_det_u * g->n_det_v, lenD = lenP * P;
     const int ss = (P + batch - 1) / batch;
     const size_t per_epoch = (size_t)batch * ss;
-    DevBuf<float> dref, dvol, dsino0, dsino, dproj, dvmax, dcoef, dgx, dgy, dout;
+    DevBuf<float> dref, dvol, dsino0, dsino, dproj, dcoef, dgx, dgy, dout;
     DevBuf<int32_t> dcodes;
     DevBuf<uint8_t> dflags;
     XR_HIP(ctx, dref.alloc(V1));
@@ -101,7 +101,8 @@ int xr_grad_reconstruct(xr_context* ctx, const xr_geometry* g, const xr_scan* s,
     XR_HIP(ctx, dsino0.alloc(lenD));
     XR_HIP(ctx, dsino.alloc(lenD));
     XR_HIP(ctx, dproj.alloc(lenD));
-    XR_HIP(ctx, dvmax.alloc(1));
+    SolveSums sums;
+    XR_HIP(ctx, sums.alloc(epochs, batch));
     XR_HIP(ctx, dcoef.alloc(P));
     XR_HIP(ctx, dgx.alloc(V1));
     XR_HIP(ctx, dgy.alloc(V1));
@@ -153,25 +154,22 @@ int xr_grad_reconstruct(xr_context* ctx, const xr_geometry* g, const xr_scan* s,
             // at zero while projecting and get their 0.01 back at the end
             XR_HIP(ctx, launch_fill(dvol.p, V1, 0.01f, ctx->stream));
             XR_HIP(ctx, launch_grad_faces(dvol.p, N1, ext, 0.0f, ctx->stream));
-            bool vmax_known = false;
-            for (int ep = 0; ep < epochs; ep++) {
-                XR_HIP(ctx, hipMemsetAsync(ctx->d_loss, 0, sizeof(double), ctx->stream));
+            XR_HIP(ctx, sums.clear(ctx->stream));
+            for (int ep = 0; ep < epochs; ep++)
                 for (int pos = 0; pos < batch; pos++) {
                     const size_t off = (size_t)ep * per_epoch + (size_t)pos * ss;
+                    float* const vmax = sums.vmax(ep, pos);
                     XR_TRY(forward_launch(plan, FWD_PLAIN, dvol.p, 0, dproj.p, dsino.p, c * P, dcodes.p + off,
-                                          dflags.p + off, ss, out_mode, ctx->d_loss, vmax_known ? dvmax.p : nullptr));
-                    XR_HIP(ctx, launch_fill(dvmax.p, 1, 0.0f, ctx->stream));
+                                          dflags.p + off, ss, out_mode, sums.loss(ep), ep + pos ? vmax - 1 : nullptr));
                     XR_TRY(backward_launch(plan, kind, dproj.p, c * P, dcodes.p + off, ss, dvol.p, nullptr, nullptr,
-                                           alpha, 0, reinterpret_cast<unsigned*>(dvmax.p)));
+                                           alpha, 0, reinterpret_cast<unsigned*>(vmax)));
                     // the update touched the skipped layers too: back to zero (the
-                    // max left in dvmax may count them, a bound that stays safe)
+                    // max left in vmax may count them, a bound that stays safe)
                     XR_HIP(ctx, launch_grad_faces(dvol.p, N1, ext, 0.0f, ctx->stream));
-                    vmax_known = true;
                 }
-                if (stats && stats->losses)
-                    XR_HIP(ctx, hipMemcpyAsync(&stats->losses[(size_t)slot * epochs + ep], ctx->d_loss,
-                                               sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-            }
+            if (stats && stats->losses && epochs > 0)
+                XR_HIP(ctx, hipMemcpyAsync(&stats->losses[(size_t)slot * epochs], sums.loss(0),
+                                           sizeof(double) * epochs, hipMemcpyDeviceToHost, ctx->stream));
             XR_HIP(ctx, launch_grad_faces(dvol.p, N1, ext, 0.01f, ctx->stream));
             float* dst = (c == 0 && d == 0) ? dgx.p : (c == 0 && d == 1) ? dgy.p : dref.p;
             XR_TRY(xr_volume_from_columns(ctx, dvol.p, dst, N1, 1));

@@ -334,7 +334,7 @@ int forward_launch(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stri
                 XR_HIP(ctx, launch_fill(vb, 1, 0.0f, ctx->stream));
                 XR_HIP(ctx, launch_absmax(vol, nvals, vb, ctx->stream));
             } else {
-                XR_HIP(ctx, hipMemsetAsync(vb, 0, sizeof(float), ctx->stream));
+                if (!vmax_buf) XR_HIP(ctx, hipMemsetAsync(vb, 0, sizeof(float), ctx->stream));
                 XR_TRY(timed(ctx, 3, [&] { return launch_absmax(vol, nvals, vb, ctx->stream); }));
             }
             a.vmax = vb;
@@ -661,7 +661,7 @@ int xr_context_create(xr_context** out, int device) {
     auto* c = new (std::nothrow) xr_context();
     if (!c) return XR_ERR_ALLOC;
     c->device = device;
-    if (device_malloc((void**)&c->d_loss, 2 * sizeof(double)) != hipSuccess ||
+    if (device_malloc((void**)&c->d_loss, 3 * sizeof(double)) != hipSuccess ||
         device_malloc((void**)&c->d_scal, 2 * sizeof(float)) != hipSuccess) {
         if (c->d_loss) (void)hipFree(c->d_loss);
         delete c;
@@ -995,10 +995,11 @@ int xr_project(xr_context* ctx, xr_plan* plan, const float* vol, float* proj, co
     }
     XR_TRY(upload_views(plan, views, n_views, accumulate));
     if (out_mode != XR_OUT_RAW) XR_TRY(ensure_norm(plan));
-    if (loss) XR_HIP(ctx, hipMemsetAsync(ctx->d_loss, 0, sizeof(double), ctx->stream));
+    XR_HIP(ctx, hipMemsetAsync(ctx->d_loss, 0, 3 * sizeof(double), ctx->stream));
     const int64_t N3 = (int64_t)plan->g.n_vox * plan->g.n_vox * plan->g.n_vox;
     XR_TRY(forward_launch(plan, xtt ? FWD_XTT : FWD_PLAIN, vol, N3, proj, sino, 0, ctx->d_codes,
-                          accumulate ? ctx->d_flags : nullptr, n_views, out_mode, ctx->d_loss));
+                          accumulate ? ctx->d_flags : nullptr, n_views, out_mode, ctx->d_loss, nullptr,
+                          reinterpret_cast<float*>(ctx->d_loss + 2)));
     if (loss) {
         XR_HIP(ctx, hipMemcpyAsync(loss, ctx->d_loss, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         XR_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1057,10 +1058,10 @@ int xr_residual(xr_context* ctx, xr_plan* plan, const float* vol, float* resid, 
     if (n_views == 0) return XR_OK;
     XR_TRY(upload_views(plan, views, n_views, nullptr));
     XR_TRY(ensure_norm(plan));
-    XR_HIP(ctx, hipMemsetAsync(ctx->d_loss, 0, 2 * sizeof(double), ctx->stream));
+    XR_HIP(ctx, hipMemsetAsync(ctx->d_loss, 0, 3 * sizeof(double), ctx->stream));
     const int64_t N3 = (int64_t)plan->g.n_vox * plan->g.n_vox * plan->g.n_vox;
     XR_TRY(forward_launch(plan, xtt ? FWD_XTT : FWD_PLAIN, vol, N3, resid, sino, 0, ctx->d_codes, nullptr, n_views,
-                          OUT_RESIDUAL_L2, ctx->d_loss));
+                          OUT_RESIDUAL_L2, ctx->d_loss, nullptr, reinterpret_cast<float*>(ctx->d_loss + 2)));
     double sums[2] = {0, 0};
     XR_HIP(ctx, hipMemcpyAsync(sums, ctx->d_loss, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     XR_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1276,9 +1277,9 @@ int xr_ir_reconstruct(xr_context* ctx, const xr_geometry* g, const xr_scan* s, f
     XR_HIP(ctx, dvol.alloc(N3));
     XR_HIP(ctx, dsino.alloc(lenD));
     XR_HIP(ctx, dproj.alloc(lenD));
-    DevBuf<float> dvmax;
-    XR_HIP(ctx, dvmax.alloc(1));
     const size_t per_epoch = (size_t)batch * ss;
+    SolveSums sums;
+    XR_HIP(ctx, sums.alloc(epochs, batch));
     XR_HIP(ctx, dcodes.alloc(per_epoch * std::max(epochs, 1)));
     XR_HIP(ctx, dflags.alloc(per_epoch * std::max(epochs, 1)));
     // One engine per call, continuing across conditions (reconstruct.cu:75-81).
@@ -1319,23 +1320,19 @@ int xr_ir_reconstruct(xr_context* ctx, const xr_geometry* g, const xr_scan* s, f
         // max |voxel| for the forward's fixed-point scale: measured from the
         // uploaded volume, then left by each backprojection for the next
         // subset (the update writes every voxel once)
-        bool vmax_known = false;
-        for (int ep = 0; ep < epochs; ep++) {
-            XR_HIP(ctx, hipMemsetAsync(ctx->d_loss, 0, sizeof(double), ctx->stream));
+        XR_HIP(ctx, sums.clear(ctx->stream));
+        for (int ep = 0; ep < epochs; ep++)
             for (int pos = 0; pos < batch; pos++) {
                 const size_t off = (size_t)ep * per_epoch + (size_t)pos * ss;
+                float* const vmax = sums.vmax(ep, pos);
                 XR_TRY(forward_launch(plan, FWD_PLAIN, dvol.p, 0, dproj.p, dsino.p, c * P, dcodes.p + off,
-                                      dflags.p + off, ss, out_mode, ctx->d_loss, vmax_known ? dvmax.p : nullptr));
-                XR_HIP(ctx, launch_fill(dvmax.p, 1, 0.0f, ctx->stream));
+                                      dflags.p + off, ss, out_mode, sums.loss(ep), ep + pos ? vmax - 1 : nullptr));
                 XR_TRY(backward_launch(plan, kind, dproj.p, c * P, dcodes.p + off, ss, dvol.p, nullptr, nullptr, alpha,
-                                       0, reinterpret_cast<unsigned*>(dvmax.p)));
-                vmax_known = true;
+                                       0, reinterpret_cast<unsigned*>(vmax)));
             }
-            if (stats && stats->losses) {
-                XR_HIP(ctx, hipMemcpyAsync(&stats->losses[(size_t)c * epochs + ep], ctx->d_loss, sizeof(double),
-                                           hipMemcpyDeviceToHost, ctx->stream));
-            }
-        }
+        if (stats && stats->losses && epochs > 0)
+            XR_HIP(ctx, hipMemcpyAsync(&stats->losses[(size_t)c * epochs], sums.loss(0), sizeof(double) * epochs,
+                                       hipMemcpyDeviceToHost, ctx->stream));
         XR_TRY(xr_volume_from_columns(ctx, dvol.p, dref.p, N, 1));
         XR_HIP(ctx, hipMemcpyAsync(vol[c], dref.p, sizeof(float) * N3, hipMemcpyDeviceToHost, ctx->stream));
         XR_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1370,6 +1367,8 @@ int xr_xtt_reconstruct(xr_context* ctx, const xr_geometry* g, const xr_scan* s, 
     const size_t per_epoch = (size_t)batch * C * ss;
     XR_HIP(ctx, dcodes.alloc(per_epoch * std::max(epochs, 1)));
     XR_HIP(ctx, dflags.alloc(per_epoch * std::max(epochs, 1)));
+    SolveSums sums;
+    XR_HIP(ctx, sums.alloc(epochs, 0));
     std::vector<int> order(batch);
     for (int i = 0; i < batch; i++) order[i] = i;
     std::vector<int32_t> codes(per_epoch * std::max(epochs, 1));
@@ -1406,18 +1405,17 @@ int xr_xtt_reconstruct(xr_context* ctx, const xr_geometry* g, const xr_scan* s, 
     const float alpha = (method == XR_METHOD_ART) ? lambda / (float)ss : 0.f;
     const int kind = (method == XR_METHOD_MLEM) ? BWD_XTT_MLEM : BWD_XTT_ART;
     const int out_mode = (method == XR_METHOD_MLEM) ? OUT_RATIO : OUT_RESIDUAL;
-    for (int ep = 0; ep < epochs; ep++) {
-        XR_HIP(ctx, hipMemsetAsync(ctx->d_loss, 0, sizeof(double), ctx->stream));
+    XR_HIP(ctx, sums.clear(ctx->stream));
+    for (int ep = 0; ep < epochs; ep++)
         for (int pos = 0; pos < batch; pos++) {
             const size_t off = (size_t)ep * per_epoch + (size_t)pos * C * ss;
             XR_TRY(forward_launch(plan, FWD_XTT, dvol.p, 0, dproj.p, dsino.p, 0, dcodes.p + off, dflags.p + off,
-                                  C * ss, out_mode, ctx->d_loss));
+                                  C * ss, out_mode, sums.loss(ep)));
             XR_TRY(backward_launch(plan, kind, dproj.p, 0, dcodes.p + off, C * ss, dvol.p, nullptr, nullptr, alpha, 0));
         }
-        if (stats && stats->losses)
-            XR_HIP(ctx, hipMemcpyAsync(&stats->losses[ep], ctx->d_loss, sizeof(double), hipMemcpyDeviceToHost,
-                                       ctx->stream));
-    }
+    if (stats && stats->losses && epochs > 0)
+        XR_HIP(ctx, hipMemcpyAsync(stats->losses, sums.loss(0), sizeof(double) * epochs, hipMemcpyDeviceToHost,
+                                   ctx->stream));
     // voxelSqrt (reconstruct.cu:919-922), sinogram overwrite (:924-925), volumes (:926-927).
     XR_TRY(xr_volume_sqrt(ctx, dvol.p, N3 * K));
     for (int c = 0; c < C; c++)
