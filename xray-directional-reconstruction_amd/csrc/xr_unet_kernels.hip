@@ -205,10 +205,15 @@ constexpr int kCH0 = kCT0 + 2, kCH1 = kCT1 + 2, kCH2 = kCT2 + 2;
 constexpr int kCHalo = kCH0 * kCH1 * kCH2;
 constexpr int kTapsPad = 28;
 
-// CPS: input-channel chunks staged per barrier.  Wide inputs (the decoder's
-// concatenations, 96-byte voxel records) stage two chunks at once, so that
-// both 16-byte pieces of a record are fetched together while its cache line
-// is resident, instead of the line being fetched again for the next chunk.
+// CPS: input-channel chunks staged per barrier, up to three: they go from global
+// memory straight to LDS and are waited for there, so few stages of long loads
+// are better than many short ones (24 -> 24 channels at 128^3: three chunks 125,
+// one 150 us), and the 16-byte pieces of a voxel record are fetched while its
+// cache line is resident.  Staging through registers a stage ahead took 48 of
+// them and did not overlap: the weights' loads, issued later, return in order.
+// Bound by LDS reads (narrow outputs) and the stage's latency, hidden by three or
+// four blocks per CU.  Measured at 128^3, 72 -> 24 channels with fused upsampling:
+// 421 (row-major weights) -> 457 (packed) -> 258 us.
 // UP: the first a.up_chunks chunks come from the half-resolution tensor a.up
 // at the halo voxel's parent (nearest x2 upsampling), the rest from a.in, so
 // the decoder's concatenation is never written; the halo in LDS, and hence
@@ -217,7 +222,7 @@ template <int NT, int CPS, bool UP>
 __global__ __launch_bounds__(256) void k_conv3_tiled(const ConvArgs a) {
     __shared__ bf16x8 halo[CPS * kCHalo];
     const lds_bf16x8* const hl = (const lds_bf16x8*)halo;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 15, kg = lane >> 4;
     const int nb2 = a.D2 / kCT2, nb1 = a.D1 / kCT1;
     const int b2 = blockIdx.x % nb2, b1 = (blockIdx.x / nb2) % nb1, b0 = blockIdx.x / (nb2 * nb1);
@@ -237,50 +242,47 @@ __global__ __launch_bounds__(256) void k_conv3_tiled(const ConvArgs a) {
         for (int nt = 0; nt < NT; nt++) acc[m][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
     const __bf16* __restrict__ in = a.in + a.in_off;
     const int nchunk = a.Cin / 8;
-    // halo voxels of this thread: i = threadIdx.x + 256 j; their global offsets
-    // (-1: outside the volume, zero padding) are the same for every chunk
+    // halo voxels of this thread: i = threadIdx.x + 256 j; their sources (outside the
+    // volume: zeros, for every chunk) are the same records for every chunk
     constexpr int kPer = (kCHalo + 255) / 256;
-    int64_t hoff[kPer], uoff[kPer];
+    const __bf16* hsrc[kPer];
+    const __bf16* usrc[kPer];
+    int hstep[kPer];
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
         const int i = threadIdx.x + 256 * j;
         const int q2 = i % kCH2, q1 = (i / kCH2) % kCH1, q0 = i / (kCH2 * kCH1);
         const int g0 = o0 + q0 - 1, g1 = o1 + q1 - 1, g2 = o2 + q2 - 1;
-        const bool ok = i < kCHalo && (unsigned)g0 < (unsigned)a.D0 && (unsigned)g1 < (unsigned)a.D1 &&
-                        (unsigned)g2 < (unsigned)a.D2;
-        hoff[j] = ok ? (((int64_t)g0 * a.D1 + g1) * a.D2 + g2) * a.in_ld : -1;
+        const bool ok = (unsigned)g0 < (unsigned)a.D0 && (unsigned)g1 < (unsigned)a.D1 && (unsigned)g2 < (unsigned)a.D2;
+        hstep[j] = ok ? 8 : 0;
+        hsrc[j] = ok ? in + (((int64_t)g0 * a.D1 + g1) * a.D2 + g2) * a.in_ld : g_zero8;
         if (UP)
-            uoff[j] = ok ? (((int64_t)(g0 >> 1) * (a.D1 >> 1) + (g1 >> 1)) * (a.D2 >> 1) + (g2 >> 1)) * a.up_ld : -1;
+            usrc[j] = ok ? a.up + a.up_off +
+                               (((int64_t)(g0 >> 1) * (a.D1 >> 1) + (g1 >> 1)) * (a.D2 >> 1) + (g2 >> 1)) * a.up_ld
+                         : g_zero8;
     }
-    const __bf16* __restrict__ up = UP ? a.up + a.up_off : nullptr;
-    // stage st holds chunks st*CPS .. st*CPS + CPS-1 (chunks past the last are zero)
-    bf16x8 pre[CPS][kPer];
-    auto fetch = [&](int st) {
+    const int up_chunks = UP ? a.up_chunks : 0;
+    // stage st holds chunks st*CPS .. st*CPS + CPS-1
+    auto stage = [&](int st) {
 #pragma unroll
         for (int c = 0; c < CPS; c++) {
             const int cc = st * CPS + c;
+            if (cc >= nchunk) break;
 #pragma unroll
             for (int j = 0; j < kPer; j++) {
-                const __bf16* src = (UP && cc < a.up_chunks) ? up + uoff[j] + cc * 8
-                                                             : in + hoff[j] + (cc - (UP ? a.up_chunks : 0)) * 8;
-                pre[c][j] = (cc < nchunk && hoff[j] >= 0) ? *(const bf16x8*)src : zero8();
+                const __bf16* const src =
+                    (UP && cc < up_chunks) ? usrc[j] + cc * hstep[j] : hsrc[j] + (cc - up_chunks) * hstep[j];
+                if (256 * j + 255 < kCHalo || threadIdx.x + 256 * j < kCHalo)
+                    lds_load16(src, (lds_bf16x8*)halo + c * kCHalo + 256 * j + 64 * wave);
             }
         }
-    };
-    auto store = [&] {
-#pragma unroll
-        for (int c = 0; c < CPS; c++)
-#pragma unroll
-            for (int j = 0; j < kPer; j++)
-                if (threadIdx.x + 256 * j < kCHalo) halo[c * kCHalo + threadIdx.x + 256 * j] = pre[c][j];
+        lds_wait();
     };
     const int nstage = (nchunk + CPS - 1) / CPS;
-    fetch(0);
     for (int st = 0; st < nstage; st++) {
         __syncthreads();  // the previous stage's reads are done
-        store();
+        stage(st);
         __syncthreads();
-        if (st + 1 < nstage) fetch(st + 1);  // in flight during this stage's MFMAs
 #pragma unroll 1
         for (int c = 0; c < CPS; c++) {
             const int cc = st * CPS + c;
@@ -749,8 +751,8 @@ hipError_t launch_conv3(const ConvArgs& a, hipStream_t s) {
         return hipErrorInvalidValue;
     if (conv3_tiled_ok(a)) {
         const dim3 tgrid((unsigned)(V / (kCT0 * kCT1 * kCT2)));
-        // several chunks per stage for inputs of 32 or more channels
-        const int cps = (a.Cin >= 32 && nt <= 3) ? (nt <= 2 ? 3 : 2) : 1;
+        // three chunks per stage where there are as many: a stage's loads are waited for
+        const int cps = std::min(3, a.Cin / 8);
         switch (nt) {
 #define XR_CONVT_UP(N, C)                                                                  \
     if (up) hipLaunchKernelGGL((k_conv3_tiled<N, C, true>), tgrid, dim3(256), 0, s, a); \
