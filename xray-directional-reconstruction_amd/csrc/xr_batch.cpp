@@ -325,7 +325,6 @@ int build_tables(xr_batch* b) {
             a.sino = p.sino;
             a.norm = pl->d_norm;
             a.bands = pl->tiles.fwd_scan ? nullptr : pl->d_bands;
-            a.g2 = pl->d_g2;
             a.xw = pl->d_xw;
             a.loss = b->d_loss + k;
             // max |voxel| of problem oi: measured by k_absmax_seg at the first
@@ -367,7 +366,6 @@ int build_tables(xr_batch* b) {
             w.code_base = 0;
             w.vol = p.vol;
             w.chan_stride = N3;
-            w.g2 = pl->d_g2;
             w.xw = pl->d_xw;
             w.alpha = mlem ? 0.f : b->lambda / (float)p.ss;  // reconstruct.cu:124, 911
             w.axis = a.axis;

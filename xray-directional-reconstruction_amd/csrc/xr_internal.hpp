@@ -114,7 +114,6 @@ struct FwdArgs {
     float* proj;             // [n_cond][P][V][U]
     const float* sino;       // measured data, same layout (RATIO / RESIDUAL)
     const float* norm;       // L/(factor+1e-5), same layout (NORMALISED / RATIO / RESIDUAL)
-    const float* g2;         // XTT [n_cond*P][K]: (S_k.G)^2
     const float* xw;         // untilted XTT [n_cond*P][5][kXwStride]: weight constants (see BwdArgs::xw)
     double* loss;            // accumulated sum |y - p| (RATIO / RESIDUAL)
     const float* vmax;       // device scalar: max |voxel value| of vol (1 for the weight pass)
@@ -149,7 +148,6 @@ struct BwdArgs {
     float* tmp;              // BWD_RAW / BWD_XTT_RAW accumulators (internal layout)
     float* factor;
     int64_t chan_stride;
-    const float* g2;         // XTT [n_cond*P][K]: (S_k.G)^2
     // untilted XTT [n_cond*P][5][kXwStride], with sig_k = |S_k.G|: sig_k S_k,z,
     // (S_k.G)^2 |S_k|^2, sig_k vs S_k,x, sig_k vs S_k,y, sig_k (d0_x S_k,x + d0_y S_k,y);
     // entries k >= K are zero

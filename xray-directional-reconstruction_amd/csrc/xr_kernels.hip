@@ -16,7 +16,7 @@
 // No global atomics; the sinogram is written exactly once per view.  The LDS
 // accumulation is fixed point: each contribution is rounded to a 32-bit integer
 // on a per-launch power-of-two scale (from max |voxel value|) and summed with
-// 64-bit integer LDS atomics (ds_add_u64).  On gfx950 these run at bank rate
+// integer LDS atomics (ds_add_u32; the weight pass: ds_add_u64).  On gfx950 these run at bank rate
 // while FP32 LDS atomics (ds_add_f32) serialise per lane (~20x slower here), and
 // integer sums are exact and order independent: the forward projection is
 // bitwise deterministic.

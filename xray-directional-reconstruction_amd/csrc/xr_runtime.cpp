@@ -303,7 +303,6 @@ int forward_launch(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stri
     a.norm = p->d_norm;
     a.bands = p->tiles.fwd_scan ? nullptr : p->d_bands;
     a.code_base = code_base;
-    a.g2 = p->d_g2;
     a.xw = p->d_xw;
     a.loss = d_loss;
     a.out_mode = out_mode;
@@ -405,7 +404,6 @@ int backward_launch(xr_plan* p, int kind, const float* proj, int code_base, cons
     a.tmp = tmp;
     a.factor = factor;
     a.chan_stride = (int64_t)p->g.n_vox * p->g.n_vox * p->g.n_vox;
-    a.g2 = p->d_g2;
     a.xw = p->d_xw;
     a.alpha = alpha;
     a.overwrite = overwrite;
@@ -864,12 +862,10 @@ int xr_plan_create(xr_context* ctx, const xr_geometry* g, const xr_scan* s, int 
     XR_HIP(ctx, hipSetDevice(ctx->device));
     XR_HIP(ctx, device_malloc((void**)&p->d_vg, vg.size() * sizeof(ViewGeom)));
     XR_HIP(ctx, device_malloc((void**)&p->d_cg, cg.size() * sizeof(ChordGeom)));
-    XR_HIP(ctx, device_malloc((void**)&p->d_g2, g2.size() * sizeof(float)));
     XR_HIP(ctx, device_malloc((void**)&p->d_xw, xw.size() * sizeof(float)));
     XR_HIP(ctx, hipMemcpy(p->d_xw, xw.data(), xw.size() * sizeof(float), hipMemcpyHostToDevice));
     XR_HIP(ctx, hipMemcpy(p->d_vg, vg.data(), vg.size() * sizeof(ViewGeom), hipMemcpyHostToDevice));
     XR_HIP(ctx, hipMemcpy(p->d_cg, cg.data(), cg.size() * sizeof(ChordGeom), hipMemcpyHostToDevice));
-    XR_HIP(ctx, hipMemcpy(p->d_g2, g2.data(), g2.size() * sizeof(float), hipMemcpyHostToDevice));
     *out = p.release();
     return XR_OK;
 }
@@ -879,7 +875,6 @@ void xr_plan_destroy(xr_plan* p) {
     (void)hipStreamSynchronize(p->ctx->stream);
     if (p->d_vg) (void)hipFree(p->d_vg);
     if (p->d_cg) (void)hipFree(p->d_cg);
-    if (p->d_g2) (void)hipFree(p->d_g2);
     if (p->d_xw) (void)hipFree(p->d_xw);
     if (p->d_norm) (void)hipFree(p->d_norm);
     if (p->d_bands) (void)hipFree(p->d_bands);
