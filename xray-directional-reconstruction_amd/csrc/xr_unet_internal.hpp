@@ -14,7 +14,7 @@ namespace nn {
 struct ConvArgs {
     const __bf16* in;
     int in_ld, in_off, Cin;
-    const __bf16* w;  // [round16(Cout)][Kpad], k = tap*Cin + ci
+    const __bf16* w;  // [round16(Cout)][Kpad], k = tap*Cin + ci, in the operand order of launch_pack
     int Kpad;
     const float* bias;  // [Cout] or null
     __bf16* out;
@@ -23,7 +23,7 @@ struct ConvArgs {
     int mask_ld, mask_off;
     int D0, D1, D2;  // spatial dims, D2 fastest
     int relu, accumulate;
-    // optional: the same weights as [round16(Cout)][Ktpad] with k = chunk*224 +
+    // optional: the same weights (and order) as [round16(Cout)][Ktpad] with k = chunk*224 +
     // tap*8 + c (chunk of 8 input channels, 28 taps with tap 27 zero), for the
     // LDS-tiled kernel (used when the dims are multiples of its tile)
     const __bf16* wt;
