@@ -1514,7 +1514,9 @@ __device__ __forceinline__ float backward_item(const BwdArgs& a, int o, int step
     };
     unsigned long long wholes = 0;
     // column terms of views b0 .. b0+15 for this wave's columns: lane = 4 x view
-    // + column (plain) or channel quarter (XTT)
+    // + column (plain) or channel quarter (XTT).  A column past the volume repeats
+    // the last one (its sums are never stored): the tile's box, hence its footprint
+    // and FOOT_INSIDE, ends at N - 1, and so must everything a column reads.
     auto term_batch = [&](int b0) XR_INLINE {
         const int j = lane >> 2, p = lane & 3;
         const lds_int* fp = foot_of(b0 + j);
@@ -1522,7 +1524,8 @@ __device__ __forceinline__ float backward_item(const BwdArgs& a, int o, int step
         const ViewGeom g = vg[code];
         const int iu_lo = fp[0], iv_lo = fp[1], W = fp[2], Ws = fp[3] & 0xffff, fl = fp[4];
         const int cidx = XTT ? 0 : (p & (NC - 1));
-        const float xp = (float)(xb + cidx % C::CX) - d.xc, yp = (float)(yb + cidx / C::CX) - d.xc;
+        const float xp = (float)min(xb + cidx % C::CX, d.N - 1) - d.xc;
+        const float yp = (float)min(yb + cidx / C::CX, d.N - 1) - d.xc;
         const ColForms c = col_forms(g, xp, yp);
         lds_float* tp = term + (j * NC + cidx) * TW;
         lds_int* ti = (lds_int*)tp;
@@ -1625,15 +1628,16 @@ __device__ __forceinline__ float backward_item(const BwdArgs& a, int o, int step
             const int code = uniformi(foot_of(s)[5]);
             const float cxy = tp[7], d0z = vgc[code].d0[2];
             if (TILT && a.coef) {
-                // backwardOrth: the basis rotated per voxel
+                // backwardOrth: the basis rotated per voxel (of the column the terms are of)
                 const ViewGeom& g = a.vg[code];
-                const float dx = fmaf(d.vs, (float)xb - d.xc, g.d0[0]), dy = fmaf(d.vs, (float)yb - d.xc, g.d0[1]);
+                const int x = min(xb, d.N - 1), y = min(yb, d.N - 1);
+                const float dx = fmaf(d.vs, (float)x - d.xc, g.d0[0]), dy = fmaf(d.vs, (float)y - d.xc, g.d0[1]);
 #pragma unroll
                 for (int q = 0; q < ZPL; q++) {
                     if (!all && !ok[q]) continue;
                     const float dz = fmaf(d.vs, zpq[q], d0z);
                     const float id2 = rcpf(fmaf(dz, dz, cxy));
-                    const int64_t vi = ((int64_t)yb * d.N + xb) * d.N + (int)(zpq[q] + d.xc);
+                    const int64_t vi = ((int64_t)y * d.N + x) * d.N + (int)(zpq[q] + d.xc);
                     float R[9];
                     orth_rotation(a.coef[vi], a.coef[vi + a.chan_stride], R);
 #pragma unroll
