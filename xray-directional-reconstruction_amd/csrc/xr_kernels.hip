@@ -551,7 +551,9 @@ __device__ __forceinline__ void splat_tilted(const FwdArgs& a, const ViewGeom& g
                     lp[w] = (e & 0xffff) + (i - s * L);
                     cc[w] = e >> 16;
                     in[w] = i < total && lp[w] < n_lane;
-                    const unsigned at = in[w] ? (unsigned)cc[w] * s_col + (unsigned)lp[w] * s_lane : 0u;
+                    // 64 bits: without a copy one stride is N^2, and from N = 1626 on the sum passes 2^32
+                    const int64_t at =
+                        in[w] ? (int64_t)((uint64_t)(unsigned)cc[w] * s_col + (uint64_t)(unsigned)lp[w] * s_lane) : 0;
                     if (KIND == FWD_WEIGHT) {
                         mu[w][0] = 1.f;
                     } else if (KIND == FWD_PLAIN) {
@@ -559,7 +561,7 @@ __device__ __forceinline__ void splat_tilted(const FwdArgs& a, const ViewGeom& g
                     } else {
 #pragma unroll
                         for (int k = 0; k < (KIND == FWD_XTT ? KM : 1); k++)
-                            mu[w][k] = k < d.K ? vrow[at + (int64_t)k * a.chan_stride] : 0.f;
+                            mu[w][k] = k < d.K ? vrow[at + k * a.chan_stride] : 0.f;
                     }
                 }
 #pragma unroll
