@@ -1387,6 +1387,20 @@ __device__ __forceinline__ float backward_update(const BwdArgs& a, const float (
     return vmx;
 }
 
+// Bilinear sample of texels (iu, iv), (iu + 1, iv), (iu, iv + 1), (iu + 1, iv + 1).
+// Tilted: four weighted terms and no difference of texels, so that an infinite
+// texel (a pixel without a count) beside a finite one gives infinity, not NaN.
+template <bool TILT>
+__device__ __forceinline__ float blend(float fu, float fv, float r00, float r01, float r10, float r11) {
+    const float gu = 1.0f - fu;
+    if (TILT) {
+        const float gv = 1.0f - fv;
+        return fmaf(gu * gv, r00, fmaf(fu * gv, r01, fmaf(fu * fv, r11, gu * fv * r10)));
+    }
+    const float top = fmaf(fu, r01, gu * r00), bot = fmaf(fu, r11, gu * r10);
+    return fmaf(fv, bot - top, top);
+}
+
 // One voxel tile o of a backprojection launch; step selects the view list
 // views + step*n_views (a solver's subset step).  stage: the block's LDS.
 // Returns the lane's max |updated voxel| (MLEM / ART kinds).
@@ -1716,12 +1730,9 @@ __device__ __forceinline__ float backward_item(const BwdArgs& a, int o, int step
             r[q][2] = p1[0];
             r[q][3] = p1[1];
         }
-        const float a0 = 1.0f - fu[0];
 #pragma unroll
         for (int q = 0; q < ZPL; q++) {
-            const float top = TILT ? fmaf(fu[q], r[q][1] - r[q][0], r[q][0]) : fmaf(fu[q], r[q][1], a0 * r[q][0]);
-            const float bot = TILT ? fmaf(fu[q], r[q][3] - r[q][2], r[q][2]) : fmaf(fu[q], r[q][3], a0 * r[q][2]);
-            nb[q] = fmaf(fv[q], bot - top, top);
+            nb[q] = blend<TILT>(fu[q], fv[q], r[q][0], r[q][1], r[q][2], r[q][3]);
             ok[q] = true;
         }
         accumulate(s, cidx, tp, nb, ok, std::true_type(), 0.0f);
@@ -1780,9 +1791,7 @@ __device__ __forceinline__ float backward_item(const BwdArgs& a, int o, int step
                 r10 = __builtin_nontemporal_load(img + qi + d.U);
                 r11 = __builtin_nontemporal_load(img + qi + d.U + 1);
             }
-            const float top = TILT ? fmaf(fu, r01 - r00, r00) : fmaf(fu, r01, (1.0f - fu) * r00);
-            const float bot = TILT ? fmaf(fu, r11 - r10, r10) : fmaf(fu, r11, (1.0f - fu) * r10);
-            nb[q] = ok[q] ? fmaf(fv, bot - top, top) : 0.0f;
+            nb[q] = ok[q] ? blend<TILT>(fu, fv, r00, r01, r10, r11) : 0.0f;
         }
         accumulate(s, cidx, tp, nb, ok, std::false_type(), counted ? 0.0f : 1.0f);
     };
