@@ -428,7 +428,8 @@ __global__ void k_band_rows(const ViewGeom* __restrict__ vg, const Dims d, int n
 // ---------------------------------------------------------------------------
 
 // XTT voxel value sum_k mu_k (S_k.G)^2 |B x S_k|^2 vs ratio (ir.cu:1780-1794)
-// from the view's row of the weight table (BwdArgs::xw), as the untilted path.
+// from the view's row of the weight table (BwdArgs::xw), as the untilted path;
+// a weight that rounding leaves below zero (a ray along S_k) is zero.
 template <int KM>
 __device__ __forceinline__ float xtt_value(const FwdArgs& a, const ViewGeom& g, cptr<float> row, float xp, float yp,
                                            float zp, const float (&mu)[KM]) {
@@ -440,7 +441,7 @@ __device__ __forceinline__ float xtt_value(const FwdArgs& a, const ViewGeom& g, 
     for (int k = 0; k < KM; k++) {
         const float ck = fmaf(xp, row[2 * kXwStride + k], fmaf(yp, row[3 * kXwStride + k], row[4 * kXwStride + k]));
         const float q = fmaf(dz, row[k], ck);
-        s = fmaf(fmaf(-q * q, id2, row[kXwStride + k]), mu[k], s);
+        s = fmaf(fmaxf(fmaf(-q * q, id2, row[kXwStride + k]), 0.f), mu[k], s);
     }
     return s * (d.vs * d.ratio);
 }
@@ -1682,7 +1683,8 @@ __device__ __forceinline__ float backward_item(const BwdArgs& a, int o, int step
 #pragma unroll
                 for (int k = 0; k < KM; k++) {
                     const float qk = fmaf(dz, sz[k], ca[k]);
-                    const float w = fmaf(-qk * qk, id2, g2s[k]);
+                    float w = fmaf(-qk * qk, id2, g2s[k]);
+                    if (TILT) w = fmaxf(w, 0.f);  // see xtt_value
                     tmp[cidx][q][k] = fmaf(w, nb[q], tmp[cidx][q][k]);
                     fac[cidx][q][k] += w;
                 }
