@@ -57,10 +57,9 @@ struct xr_plan {
     xr_tiles tiles{};      // projector tile shape (zeros: defaults)
     float max_factor = 0.f;     // largest per-pixel splat weight sum (set with d_norm)
     // tilted forward projections: copies of the volume with axis 0 or 1 contiguous (FwdArgs::vol_axis), their
-    // lengths, the stream of the last launch that reads them and the event after it
+    // lengths and the event after the last launch that reads them
     float* d_lane[2] = {nullptr, nullptr};
     size_t lane_len[2] = {0, 0};
-    hipStream_t lane_stream = nullptr;
     hipEvent_t lane_done = nullptr;
     float* d_fmax = nullptr;    // device scalar receiving it during the weight pass
 };

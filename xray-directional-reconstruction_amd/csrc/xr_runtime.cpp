@@ -256,8 +256,9 @@ static int lane_copies(xr_plan* p, int kind, const float* vol, int64_t vol_cond_
             }
             p->lane_len[la] = len;
         }
-        // the previous launch that reads the buffer may be on another stream
-        if (p->lane_stream != ctx->stream) XR_HIP(ctx, hipStreamWaitEvent(ctx->stream, p->lane_done, 0));
+        // the previous launch that reads the buffer may be on another stream (whose handle may even be
+        // this one's, if it was destroyed since): its event says, not the handle
+        XR_HIP(ctx, hipStreamWaitEvent(ctx->stream, p->lane_done, 0));
         float* dst = p->d_lane[la];
         if (kind == FWD_PLAIN && vol_cond_stride) {
             // only the volumes of the conditions with these lanes
@@ -273,7 +274,6 @@ static int lane_copies(xr_plan* p, int kind, const float* vol, int64_t vol_cond_
         a.vol_axis[la] = dst;
         used = true;
     }
-    p->lane_stream = ctx->stream;
     return XR_OK;
 }
 
