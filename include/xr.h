@@ -127,7 +127,11 @@ int xr_timing_read(xr_context* ctx, int kind, double* total_ms, int64_t* count);
  * scan, convention and direction; the L/(factor+1e-5) normalisation table is
  * built on first use (forward projection's correlationProjByLength,
  * ir.cu:1533-1603).  Replaces init_params' constant-memory upload
- * (params.cu:80-95) and the per-thread geometry of rayCasting. */
+ * (params.cu:80-95) and the per-thread geometry of rayCasting.
+ * Forward projections of conditions tilted by more than 45 degrees keep up to
+ * two copies of the volume (with another axis contiguous) in the plan, until it
+ * is destroyed; where they cannot be allocated the volume is read strided, with
+ * the same result. */
 int xr_plan_create(xr_context* ctx, const xr_geometry* g, const xr_scan* s, int convention, int direction,
                    xr_plan** out);
 void xr_plan_destroy(xr_plan* plan);

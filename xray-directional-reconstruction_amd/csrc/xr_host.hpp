@@ -153,10 +153,11 @@ int timed(xr_context* ctx, int kind, F&& launch) {
 // no_alloc: the call makes no allocation of any kind (the plan's tables must
 // already exist; max |voxel| goes to vmax_buf, cleared by a fill kernel; no
 // timing events).  Otherwise a vmax_buf is one that the caller has cleared.
+// views: the launch's codes on the host where the caller has them (see lane_copies).
 int forward_launch(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stride, float* proj, const float* sino,
                    int code_base, const int32_t* d_codes, const uint8_t* d_flags, int n_slots, int out_mode,
                    double* d_loss, const float* vmax_known = nullptr, float* vmax_buf = nullptr,
-                   bool no_alloc = false);
+                   bool no_alloc = false, const int32_t* views = nullptr);
 // vmax_out (MLEM / ART kinds): receives the atomic max of |updated voxel| as
 // float bits; the caller clears it first.
 int backward_launch(xr_plan* p, int kind, const float* proj, int code_base, const int32_t* d_codes, int n_views,

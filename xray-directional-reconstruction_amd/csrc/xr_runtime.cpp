@@ -220,28 +220,49 @@ hipEvent_t get_event(xr_context* ctx) {
 }
 
 
-// Copies of the volume for the conditions whose lanes run along x or y (see
+// Copies of the volume for the launched views whose lanes run along x or y (see
 // splat_tilted), in buffers of the plan: reading the column layout strided
-// costs one cache line per lane.  A launch of one view would read what it
-// copies only once and goes without, and so does one that may not allocate: a
-// stream under capture, a failed allocation.  The images are the same.
-static int lane_copies(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stride, int code_base, int n_slots,
-                       FwdArgs& a, bool& used) {
+// costs one cache line per lane.  Only of volumes that such a view projects
+// (views: the launch's codes on the host, or null for all conditions alike), and
+// where the views read it often enough to pay for the copy: at least two, and
+// channels^2 N^3 views >= kLaneCopyWork (each channel is read strided by itself,
+// and their lines evict each other).  Measured at 60 degrees, strided against
+// copied, us: 64^3 8 views 69, 83; 128^3 4 views 159, 166, 6 views 180, 165;
+// 64^3 x 3 8 views 110, 110; 48^3 x 13 2 views 216, 133.  A launch that may not
+// allocate (a stream under capture, a failed allocation) goes without.  The
+// images are the same.
+constexpr double kLaneCopyWork = 1.2e7;
+static int lane_copies(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stride, int code_base,
+                       const int32_t* views, int n_slots, FwdArgs& a, bool& used) {
     xr_context* ctx = p->ctx;
     used = false;
-    if (n_slots < 2) return XR_OK;
+    const int N = p->g.n_vox, C = p->n_cond, P = p->g.n_proj;
     // a solver's launch over one condition's single volume (vol_cond_stride 0) has that condition's codes alone
-    const int c0 = kind == FWD_PLAIN && vol_cond_stride == 0 ? code_base / p->g.n_proj : 0;
-    const int c1 = kind == FWD_PLAIN && vol_cond_stride == 0 ? c0 + 1 : p->n_cond;
-    bool want[2] = {false, false};
-    for (int c = c0; c < c1; c++)
-        if (p->lane_cond[c] < 2) want[(int)p->lane_cond[c]] = true;
+    const bool single = kind == FWD_PLAIN && vol_cond_stride == 0;
+    std::vector<int> count(C, 0);
+    if (single)
+        count[code_base / P] = n_slots;
+    else if (views)
+        for (int i = 0; i < n_slots; i++) count[views[i] / P]++;
+    else
+        for (int c = 0; c < C; c++) count[c] = n_slots / C;
+    // each condition has its own volume, or all share the K coefficients
+    const bool apart = kind == FWD_PLAIN && !single;
+    int most[2] = {0, 0};
+    for (int c = 0; c < C; c++)
+        if (p->lane_cond[c] < 2) {
+            int& m = most[(int)p->lane_cond[c]];
+            m = apart ? std::max(m, count[c]) : m + count[c];
+        }
+    const int K = kind == FWD_XTT ? p->n_basis : 1;
+    const double work = (double)K * K * N * N * N;
+    bool want[2];
+    for (int la = 0; la < 2; la++) want[la] = most[la] >= 2 && work * most[la] >= kLaneCopyWork;
     if (!want[0] && !want[1]) return XR_OK;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     XR_HIP(ctx, hipStreamIsCapturing(ctx->stream, &st));
     if (st != hipStreamCaptureStatusNone) return XR_OK;
-    const int N = p->g.n_vox;
-    const int channels = kind == FWD_XTT ? p->n_basis : (vol_cond_stride ? p->n_cond : 1);
+    const int channels = kind == FWD_XTT ? K : (apart ? C : 1);
     const size_t len = (size_t)N * N * N * channels;
     if (!p->lane_done) XR_HIP(ctx, hipEventCreateWithFlags(&p->lane_done, hipEventDisableTiming));
     for (int la = 0; la < 2; la++) {
@@ -260,11 +281,11 @@ static int lane_copies(xr_plan* p, int kind, const float* vol, int64_t vol_cond_
         // this one's, if it was destroyed since): its event says, not the handle
         XR_HIP(ctx, hipStreamWaitEvent(ctx->stream, p->lane_done, 0));
         float* dst = p->d_lane[la];
-        if (kind == FWD_PLAIN && vol_cond_stride) {
-            // only the volumes of the conditions with these lanes
+        if (apart) {
+            // the volume of every launched condition with these lanes: all of them read the copy
             const int64_t N3 = (int64_t)N * N * N;
-            for (int c = c0; c < c1; c++)
-                if (p->lane_cond[c] == la)
+            for (int c = 0; c < C; c++)
+                if (p->lane_cond[c] == la && count[c] > 0)
                     XR_TRY(timed(ctx, 3, [&] {
                         return launch_lane_copy(vol + c * N3, dst + c * N3, N, 1, la, ctx->stream);
                     }));
@@ -281,7 +302,8 @@ static int lane_copies(xr_plan* p, int kind, const float* vol, int64_t vol_cond_
 // for a single volume; code_base: proj/sino hold the images of codes >= code_base.
 int forward_launch(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stride, float* proj, const float* sino,
                    int code_base, const int32_t* d_codes, const uint8_t* d_flags, int n_slots, int out_mode,
-                   double* d_loss, const float* vmax_known, float* vmax_buf, bool no_alloc) {
+                   double* d_loss, const float* vmax_known, float* vmax_buf, bool no_alloc,
+                   const int32_t* views) {
     xr_context* ctx = p->ctx;
     FwdArgs a{};
     a.d = p->dims;
@@ -349,7 +371,8 @@ int forward_launch(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stri
         axis = false;
     }
     bool copies = false;
-    if (!axis && kind != FWD_WEIGHT && !no_alloc) XR_TRY(lane_copies(p, kind, vol, vol_cond_stride, code_base, n_slots, a, copies));
+    if (!axis && kind != FWD_WEIGHT && !no_alloc)
+        XR_TRY(lane_copies(p, kind, vol, vol_cond_stride, code_base, views, n_slots, a, copies));
     // Detector rows in equal chunks, all in one launch (untilted scans walk
     // only the z range that reaches a chunk's rows).
     const int V = p->g.n_det_v;
@@ -994,7 +1017,7 @@ int xr_project(xr_context* ctx, xr_plan* plan, const float* vol, float* proj, co
     const int64_t N3 = (int64_t)plan->g.n_vox * plan->g.n_vox * plan->g.n_vox;
     XR_TRY(forward_launch(plan, xtt ? FWD_XTT : FWD_PLAIN, vol, N3, proj, sino, 0, ctx->d_codes,
                           accumulate ? ctx->d_flags : nullptr, n_views, out_mode, ctx->d_loss, nullptr,
-                          reinterpret_cast<float*>(ctx->d_loss + 2)));
+                          reinterpret_cast<float*>(ctx->d_loss + 2), false, views));
     if (loss) {
         XR_HIP(ctx, hipMemcpyAsync(loss, ctx->d_loss, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         XR_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1056,7 +1079,7 @@ int xr_residual(xr_context* ctx, xr_plan* plan, const float* vol, float* resid, 
     XR_HIP(ctx, hipMemsetAsync(ctx->d_loss, 0, 3 * sizeof(double), ctx->stream));
     const int64_t N3 = (int64_t)plan->g.n_vox * plan->g.n_vox * plan->g.n_vox;
     XR_TRY(forward_launch(plan, xtt ? FWD_XTT : FWD_PLAIN, vol, N3, resid, sino, 0, ctx->d_codes, nullptr, n_views,
-                          OUT_RESIDUAL_L2, ctx->d_loss, nullptr, reinterpret_cast<float*>(ctx->d_loss + 2)));
+                          OUT_RESIDUAL_L2, ctx->d_loss, nullptr, reinterpret_cast<float*>(ctx->d_loss + 2), false, views));
     double sums[2] = {0, 0};
     XR_HIP(ctx, hipMemcpyAsync(sums, ctx->d_loss, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     XR_HIP(ctx, hipStreamSynchronize(ctx->stream));
