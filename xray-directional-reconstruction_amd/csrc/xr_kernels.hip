@@ -730,7 +730,7 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                         // whole chunks (XTT: and K the compiled count); 1: the last chunk partial; 0: any.
                         auto step = [&](int zg, auto mode_c) XR_INLINE {
                             constexpr int MODE = decltype(mode_c)::value;
-                            constexpr bool FULL = MODE > 0;
+                            constexpr bool FULL = XTT ? MODE >= 2 : MODE > 0, EXACT = MODE == 1 || MODE == 2;
                             // t = B (z - xc) + A: z - xc is exact in FP32 (half-integers below
                             // 2^23), so t depends on z alone and not on where the step starts
                             const float zoff = (float)zg - d.xc;
@@ -738,7 +738,7 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                             const auto there = [&](int c) XR_INLINE { return FULL || zg + c * 64 < ze; };
                             // a chunk that ends past the volume masks its lanes
                             auto in_chunk = [&](int c) XR_INLINE {
-                                return MODE == 2 || (MODE == 1 && c < CH - 1) || c * 64 + 64 <= rem || lane < rem - c * 64;
+                                return MODE >= 2 || (!XTT && MODE == 1 && c < CH - 1) || c * 64 + 64 <= rem || lane < rem - c * 64;
                             };
                             auto splat = [&](int c, float val, float B, float A, unsigned row0, lds_ptr<AccT> spare,
                                              float w0, float w1) XR_INLINE {
@@ -782,7 +782,7 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                                 // pair, so only one k's constants are live at a time.
                                 const float cxy = lane_f(xcxy, b[0]);
                                 float mu[CH][KM];
-                                if (MODE == 2) {
+                                if (MODE >= 2) {
                                     // one address per channel walked from the previous one (the chunks
                                     // are immediate offsets); opaque, or the compiler keeps all K
                                     // channels' lane addresses in registers across the columns
@@ -790,21 +790,20 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                                     asm volatile("" : "+v"(col));
 #pragma unroll
                                     for (int k = 0; k < KM; k++) {
+                                        if (!EXACT && k >= d.K) break;
 #pragma unroll
                                         for (int c = 0; c < CH; c++) mu[c][k] = col[c * 64];
                                         col += a.chan_stride;
                                     }
                                 } else {
-                                    // lanes past the end read the last layer (one offset for all channels)
-                                    const auto col = row + (int64_t)b[0] * d.N + zg;
-                                    unsigned zl[CH];
+                                    const auto col = row + (int64_t)b[0] * d.N + (zg + lane);
 #pragma unroll
-                                    for (int c = 0; c < CH; c++) zl[c] = (unsigned)min(c * 64 + lane, rem - 1);
+                                    for (int c = 0; c < CH; c++) {
+                                        const bool in = there(c) && in_chunk(c);
 #pragma unroll
-                                    for (int k = 0; k < KM; k++)
-#pragma unroll
-                                        for (int c = 0; c < CH; c++)
-                                            if (k < d.K) mu[c][k] = col[zl[c] + (int64_t)k * a.chan_stride];
+                                        for (int k = 0; k < KM; k++)
+                                            mu[c][k] = in && (EXACT || k < d.K) ? col[c * 64 + (int64_t)k * a.chan_stride] : 0.f;
+                                    }
                                 }
                                 float dz[CH], id2[CH], val[CH];
 #pragma unroll
@@ -815,7 +814,7 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                                 }
 #pragma unroll
                                 for (int k = 0; k < KM; k++) {
-                                    if (MODE == 2 || k < d.K) {
+                                    if (EXACT || k < d.K) {
                                         const float ck = lane_f(xck[k], b[0]), sS2 = xrow[k], g2s = xrow[xws + k];
 #pragma unroll
                                         for (int c = 0; c < CH; c++) {
@@ -839,7 +838,9 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                             const int left = ze - zg;
                             if (n == NCOL && left >= 64 * CH && (!XTT || d.K == KM))
                                 step(zg, std::integral_constant<int, 2>());
-                            else if (!XTT && INSIDE && n == NCOL && left > 64 * (CH - 1))
+                            else if (XTT && left >= 64 * CH)
+                                step(zg, std::integral_constant<int, 3>());
+                            else if (XTT ? d.K == KM : INSIDE && n == NCOL && left > 64 * (CH - 1))
                                 step(zg, std::integral_constant<int, 1>());
                             else
                                 step(zg, std::integral_constant<int, 0>());
