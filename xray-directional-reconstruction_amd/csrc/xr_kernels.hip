@@ -796,13 +796,21 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                                         col += a.chan_stride;
                                     }
                                 } else {
-                                    const auto col = row + (int64_t)b[0] * d.N + (zg + lane);
+                                    // lanes past the end read the last layer; a chunk that is not there reads nothing
 #pragma unroll
                                     for (int c = 0; c < CH; c++) {
-                                        const bool in = there(c) && in_chunk(c);
 #pragma unroll
-                                        for (int k = 0; k < KM; k++)
-                                            mu[c][k] = in && (EXACT || k < d.K) ? col[c * 64 + (int64_t)k * a.chan_stride] : 0.f;
+                                        for (int k = 0; k < KM; k++) mu[c][k] = 0.f;
+                                        if (there(c)) {
+                                            auto col = row + (int64_t)b[0] * d.N + (zg + min(c * 64 + lane, rem - 1));
+                                            asm volatile("" : "+v"(col));
+#pragma unroll
+                                            for (int k = 0; k < KM; k++) {
+                                                if (!EXACT && k >= d.K) break;
+                                                mu[c][k] = *col;
+                                                col += a.chan_stride;
+                                            }
+                                        }
                                     }
                                 }
                                 float dz[CH], id2[CH], val[CH];
