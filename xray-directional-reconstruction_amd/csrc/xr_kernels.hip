@@ -622,8 +622,9 @@ __device__ __forceinline__ void splat_tilted(const FwdArgs& a, const ViewGeom& g
 // Columns whose z extent lies inside the window (t is monotone in z) run
 // without tests; a partial last chunk only masks its lanes (such depths used to
 // take masked loads and tests throughout).
-// Measured, before -> now: 64^3 / 90 views 94 -> 64 us; 203^3 / 20 views 321 ->
-// 226 us; 512^3 / 720 views, bound by VALU issue, 58.8 -> 57.2 ms.
+// Measured, column pairs of eight chunks -> now: 64^3 / 90 views 94 -> 64 us;
+// 203^3 / 20 views 321 -> 226 us; 512^3 / 720 views, bound by VALU issue, 58.8 ->
+// 57.2 ms.
 // ---------------------------------------------------------------------------
 template <int KIND, int WAVES, int KM, int CH>
 __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& g, int code, gptr<const float> vol,
@@ -633,6 +634,10 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
     typedef typename FwdAcc<KIND>::S AccS;
     constexpr bool XTT = KIND == FWD_XTT;
     constexpr int NCOL = XTT ? 1 : (CH >= 2 ? 16 / CH : 8);
+    // Few columns are left for a step where a band is split or narrow.  With many columns a step the
+    // missing ones repeat the first one's loads, unmasked (128^3, 4 views 110 against 94 us); with four
+    // or less the step of any shape takes them (256^3, 4 views 173 against 197 us).
+    constexpr bool ANY_N = NCOL > 4;
     constexpr int xws = kXwStride;
     const Dims& d = a.d;
     const int lane = threadIdx.x & 63, wave = uniformi(threadIdx.x >> 6);
@@ -764,7 +769,7 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                                 }
 #pragma unroll
                                 for (int k = 0; k < NCOL; k++) {
-                                    if (!FULL && k >= n) break;
+                                    if ((ANY_N || !FULL) && k >= n) break;
                                     const float B = lane_f(sB, b[k]), A = lane_f(sA, b[k]);
                                     const float w0 = lane_f(sw0, b[k]), w1 = lane_f(sw1, b[k]);
                                     const unsigned row0 = row0_of(b[k]);
@@ -844,11 +849,12 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                         };
                         for (int zg = zb & ~63; zg < ze; zg += 64 * CH) {
                             const int left = ze - zg;
-                            if (n == NCOL && left >= 64 * CH && (!XTT || d.K == KM))
+                            const bool cols = ANY_N || n == NCOL;
+                            if (cols && left >= 64 * CH && (!XTT || d.K == KM))
                                 step(zg, std::integral_constant<int, 2>());
                             else if (XTT && left >= 64 * CH)
                                 step(zg, std::integral_constant<int, 3>());
-                            else if (XTT ? d.K == KM : INSIDE && n == NCOL && left > 64 * (CH - 1))
+                            else if (XTT ? d.K == KM : INSIDE && cols && left > 64 * (CH - 1))
                                 step(zg, std::integral_constant<int, 1>());
                             else
                                 step(zg, std::integral_constant<int, 0>());
@@ -2690,15 +2696,26 @@ inline unsigned grid1(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs);
 static int forward_waves(int kind) { return kind == FWD_XTT ? kFwdXttWaves : kFwdWaves; }
 
 // Standalone forward kernel: chunks per column and step by the volume's depth
-// (see splat_columns), XTT by the basis count rounded up to a compiled size (the
+// (see splat_columns), one step for a column of up to eight, so that no step of a
+// whole column is partial but for its last lanes (steps of 8 for every depth above
+// 256, of 4 for three chunks: 288^3 608 against 509 us, 384^3 1121 against 1044,
+// 160^3 203 against 183, 20 views each; ten chunks in two steps of five: 5 %
+// slower than 8 + 2).  XTT by the basis count rounded up to a compiled size (the
 // registers of a voxel's coefficients).
 template <int KIND>
 static const void* forward_kernel_of(bool axis, int nz) {
     if (!axis) return (const void*)k_forward<KIND, false, 1, kFwdWaves, 1>;
-    if (nz <= 64) return (const void*)k_forward<KIND, true, 1, kFwdWaves, 1>;
-    if (nz <= 128) return (const void*)k_forward<KIND, true, 1, kFwdWaves, 2>;
-    if (nz <= 256) return (const void*)k_forward<KIND, true, 1, kFwdWaves, 4>;
-    return (const void*)k_forward<KIND, true, 1, kFwdWaves, 8>;
+    const int ch = std::min((nz + 63) / 64, 8);
+    switch (ch) {
+        case 1: return (const void*)k_forward<KIND, true, 1, kFwdWaves, 1>;
+        case 2: return (const void*)k_forward<KIND, true, 1, kFwdWaves, 2>;
+        case 3: return (const void*)k_forward<KIND, true, 1, kFwdWaves, 3>;
+        case 4: return (const void*)k_forward<KIND, true, 1, kFwdWaves, 4>;
+        case 5: return (const void*)k_forward<KIND, true, 1, kFwdWaves, 5>;
+        case 6: return (const void*)k_forward<KIND, true, 1, kFwdWaves, 6>;
+        case 7: return (const void*)k_forward<KIND, true, 1, kFwdWaves, 7>;
+        default: return (const void*)k_forward<KIND, true, 1, kFwdWaves, 8>;
+    }
 }
 template <int KM>
 static const void* forward_kernel_xtt(bool axis) {
