@@ -927,9 +927,12 @@ __device__ __forceinline__ void forward_item(const FwdArgs& a, int o, int step, 
     // value scale folded into the untilted splat weights: ratio (ir.cu:1513-1518),
     // XTT vs * ratio (ir.cu:1791)
     const float scalev = (KIND == FWD_PLAIN) ? d.ratio : (KIND == FWD_XTT ? d.vs * d.ratio : 1.f);
-    if constexpr (AXIS)
+    // A launch with tilted views (AXIS false) may hold untilted ones of other conditions, which need
+    // not pay for the tilt (unless the basis is rotated per voxel): 384^3, eight such views 1854 us as
+    // tilted ones, 705 as untilted.
+    if (AXIS || (g.axis != 0.f && !a.coef))
         splat_columns<KIND, WAVES, KM, CH>(a, g, code, vol, scale * scalev, acc, band, u0, cs, W, v0, vb);
-    else
+    else if constexpr (!AXIS)
         splat_tilted<KIND, WAVES, KM>(a, g, code, scale, acc, u0, cs, W, v0, vb);
     __syncthreads();
 
@@ -1102,10 +1105,7 @@ __device__ __forceinline__ void forward_batch_loop(const FwdArgs* __restrict__ i
         const FwdArgs& a = items[i];
         const int o = view_grouped(a, t - (i ? item_end[i - 1] : 0));
         double* loss = a.loss ? a.loss + loss_shift : nullptr;
-        if (AXES == 1 || a.axis)
-            forward_item<KIND, true, WAVES, KM, KIND == FWD_XTT ? kXttChunks : 8>(a, o, step, loss, acc_raw, a.v0, a.vb);
-        else
-            forward_item<KIND, false, WAVES, KM, 8>(a, o, step, loss, acc_raw, a.v0, a.vb);
+        forward_item<KIND, AXES == 1, WAVES, KM, KIND == FWD_XTT ? kXttChunks : 8>(a, o, step, loss, acc_raw, a.v0, a.vb);
     }
 }
 
@@ -2700,11 +2700,12 @@ static int forward_waves(int kind) { return kind == FWD_XTT ? kFwdXttWaves : kFw
 // whole column is partial but for its last lanes (steps of 8 for every depth above
 // 256, of 4 for three chunks: 288^3 608 against 509 us, 384^3 1121 against 1044,
 // 160^3 203 against 183, 20 views each; ten chunks in two steps of five: 5 %
-// slower than 8 + 2).  XTT by the basis count rounded up to a compiled size (the
+// slower than 8 + 2); of four for the untilted views of a launch that also holds
+// tilted ones.  XTT by the basis count rounded up to a compiled size (the
 // registers of a voxel's coefficients).
 template <int KIND>
 static const void* forward_kernel_of(bool axis, int nz) {
-    if (!axis) return (const void*)k_forward<KIND, false, 1, kFwdWaves, 1>;
+    if (!axis) return (const void*)k_forward<KIND, false, 1, kFwdWaves, 4>;
     const int ch = std::min((nz + 63) / 64, 8);
     switch (ch) {
         case 1: return (const void*)k_forward<KIND, true, 1, kFwdWaves, 1>;
@@ -2720,7 +2721,7 @@ static const void* forward_kernel_of(bool axis, int nz) {
 template <int KM>
 static const void* forward_kernel_xtt(bool axis) {
     return axis ? (const void*)k_forward<FWD_XTT, true, KM, kFwdXttWaves, kXttChunks>
-                : (const void*)k_forward<FWD_XTT, false, KM, kFwdXttWaves, 1>;
+                : (const void*)k_forward<FWD_XTT, false, KM, kFwdXttWaves, kXttChunks>;
 }
 static const void* forward_kernel(int kind, bool axis, const Dims& d) {
     if (kind == FWD_WEIGHT) return forward_kernel_of<FWD_WEIGHT>(axis, d.nz);
