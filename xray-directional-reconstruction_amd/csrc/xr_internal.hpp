@@ -133,6 +133,7 @@ struct FwdArgs {
     float out_scale = 1.0f;  // factor on each new pixel sum before it joins proj's contents (gradient grid: vs)
     // tilted views: vol with axis 0 (x + N y + N^2 z) or 1 (y + N x + N^2 z) contiguous, or null (read vol strided)
     const float* vol_axis[2] = {nullptr, nullptr};
+    int lanes_z = 0;  // tilted views without such a copy: lanes along z all the same (see lanes_along_z)
     int view_group = 0;      // item order: 0 band-major; G > 0: groups of G views, all bands of a group together
 };
 
@@ -191,6 +192,17 @@ int batch_blocks_per_cu_forward(int kind, size_t lds_bytes, bool axis_all, int k
 size_t forward_lds_bytes(int kind, int vb);
 // Resident blocks per CU of the standalone forward kernel.
 int forward_blocks_per_cu(int kind, bool axis, const Dims& d, size_t lds_bytes);
+// Tilted views whose lanes would run along x or y, without a copy of the volume
+// that has that axis contiguous: read strided (a cache line per lane and
+// channel), or with the lanes along z.  Strided pays while neighbouring waves find
+// each other's lines: few channels, and few views or a small volume.  Measured,
+// strided against z, us (x60 / x90: tilt): 128^3, 24 views 470 315 / 368 524, one
+// view 130 138 / 99 247; 256^3, 4 views 993 673 / 1141 1062; 64^3 x 3, 24 views 202
+// 115 / 146 146; 160^3 x 4, one view 665 457 / 436 627; 64^3 x 13, one view 188 123
+// / 169 146; two problems of 64^3 x 13 in a batch 15159 3148 / 11738 3121.
+inline bool lanes_along_z(int K, int N, int views) {
+    return K > 8 || (views > 3 && (double)K * K * N * N * N * views >= 6e7);
+}
 // Sub-bands per detector band (1, 2, 4) of a standalone launch of `items` band
 // items on `slots` resident blocks, volume edge N: the least of (rounds of the
 // chip, and three quarters of one for the last items) x (work of an item).  An

@@ -501,7 +501,8 @@ __device__ __forceinline__ void splat_tilted(const FwdArgs& a, const ViewGeom& g
     const int lane = threadIdx.x & 63, wave = uniformi(threadIdx.x >> 6);
     const int cond = code / d.P;
     // axes: lanes along la, columns side by side along ca, one row per wave along ra
-    const int la = (int)g.lane_axis;
+    const int own = (int)g.lane_axis;
+    const int la = a.lanes_z && own < 2 && !a.vol_axis[own] ? 2 : own;
     const int ca = la == 0 ? 1 : 0, ra = la == 2 ? 1 : 2;
     const int n_lane = la == 2 ? d.nz : d.N, n_row = ra == 2 ? d.nz : d.N;
     auto pick = [](const float (&v)[4], int i) { return i == 0 ? v[0] : (i == 1 ? v[1] : v[2]); };
