@@ -86,7 +86,7 @@ struct Dims {
     float ratio;     // (vs*vs)/(det*(sod/sdd)*det*(sod/sdd))
     float sod;
     float cfdk;      // 2 pi / P (FP32, fdk.cu:161)
-    float px;        // detector pixels per voxel where the magnification is largest (launch shapes)
+    float px, px_mid;  // detector pixels per voxel where the magnification is largest; 0.4 edges off the centre (launch shapes)
     float tilt_cos, tilt_sin;  // largest z extent of a unit z step on the detector along v, along u (launch shapes)
 };
 

@@ -2755,13 +2755,14 @@ int backward_threads(int kind) {
 }
 
 // Estimated footprint of a tile of cx x cy columns and 64 zpl voxels: its
-// diagonal and, along z, its extent at the tilt, at the largest magnification
-// in the volume.  Launch shapes only: a footprint that turns out larger is read
-// from the image directly.
-static void backward_footprint(const Dims& d, int cx, int cy, int zpl, float& w, float& h) {
+// diagonal and, along z, its extent at the tilt, at px detector pixels per voxel
+// (0: at the largest magnification in the volume).  Launch shapes only: a
+// footprint that turns out larger is read from the image directly.
+static void backward_footprint(const Dims& d, int cx, int cy, int zpl, float& w, float& h, float px = 0.0f) {
     const float diag = std::sqrt((float)((cx - 1) * (cx - 1) + (cy - 1) * (cy - 1))), z = 64.0f * zpl - 1.0f;
-    w = (diag + z * d.tilt_sin) * d.px + 2.02f;
-    h = (z * d.tilt_cos + diag * d.tilt_sin) * d.px + 2.02f;
+    if (px == 0.0f) px = d.px;
+    w = (diag + z * d.tilt_sin) * px + 2.02f;
+    h = (z * d.tilt_cos + diag * d.tilt_sin) * px + 2.02f;
 }
 
 // Tile counts of a grid of `waves` waves, gx along x, each of cpw x cpw columns
@@ -2807,13 +2808,22 @@ bool backward_shape(BwdArgs& a, int zpl, int gx, bool xtt) {
 // footprint's edges cost about as much per view as two chunks (three chunks,
 // 160^3 / 180 views: zpl 3 615, 4 724, 2 971 us; five chunks, 320^3 / 60 views:
 // zpl 5 1171, 2 1605, 4 1759 us).
+// Footprints of any width (w > 16 where the magnification is largest): the depth
+// whose footprint fits the staging buffer 0.4 edges off the centre; the few tiles
+// nearer the source read the image directly.  (By the nearest voxel 512^3
+// 0.4, 400^3 0.4 mm at 300 mm and 512^3 0.5 mm at 1000 mm took zpl 1, 2, 2: 6557,
+// 2464, 4128 against 4073, 1802, 3226 us for 32 views; at the centre 512^3 0.5 mm at
+// 500 mm would take 4: 9500 against 4123 us.)
 // Fewer than kSmallTiles such tiles leave most of the chip idle: BwdSmall
 // (64^3 / 90 views, 64 tiles: 41 against 95 us; but at 96^3 / 90 views, 144
 // tiles: 177 against 125 us).
 // Tilted: the largest depth whose footprint fits the staging buffer.
 // XTT: two voxels per lane halve the per-view overhead of a column (35.1
 // against 23.0 ms for ART at 256^3 x 13, 4 x 90 views) where the volume has
-// more than 64 layers, the footprint fits and the accumulators do.
+// more than 64 layers, the footprint fits and the accumulators do.  Where the
+// footprint is of any width, it fits as above (256^3 x 3 0.6 mm at 300 mm, 16
+// views: 1410 against 817 us); a fixed width with one voxel is better than any width
+// with two (400^3 x 3 0.4 mm at 300 mm: 2725 against 3900 us).
 constexpr int kSmallTiles = 96;
 static bool backward_choose(BwdArgs& a, int kind, bool axis) {
     const Dims& d = a.d;
@@ -2821,7 +2831,11 @@ static bool backward_choose(BwdArgs& a, int kind, bool axis) {
     float w, h;
     if (bwd_xtt(kind)) {
         backward_footprint(d, 2, 4, 2, w, h);
-        const bool fits = axis ? h <= 192.0f : w * h <= 0.9f * 3584.0f;
+        bool fits = axis ? h <= 192.0f : w * h <= 0.9f * 3584.0f;
+        if (axis && w > 8.0f) {
+            backward_footprint(d, 2, 4, 2, w, h, d.px_mid);
+            fits = w * h <= 0.9f * 3584.0f;
+        }
         // (26 accumulators per voxel of 13 coefficients: two voxels spill where both sums are kept)
         const bool regs = a.d.K <= 8 || (kind == BWD_XTT_ART && (axis || a.d.K <= 13));
         backward_tiles(a, 8, 1, chunks > 1 && fits && regs ? 2 : 1, 2);
@@ -2832,7 +2846,13 @@ static bool backward_choose(BwdArgs& a, int kind, bool axis) {
         int best = 0;
         for (int z = 5; z >= 1; z--) {
             backward_footprint(d, 8, 8, z, w, h);
-            if (z > 1 && (w <= 16.0f ? h > 448.0f : (z % 2 == 1 || w * h > 0.9f * 7168.0f))) continue;
+            if (w > 16.0f) {
+                float wm, hm;
+                backward_footprint(d, 8, 8, z, wm, hm, d.px_mid);
+                if (z > 1 && (z % 2 == 1 || wm * hm > 0.9f * 7168.0f)) continue;
+            } else if (z > 1 && h > 448.0f) {
+                continue;
+            }
             const int cost = (chunks + z - 1) / z * (z + 2);
             if (best == 0 || cost < best) {
                 best = cost;

@@ -857,8 +857,9 @@ int xr_plan_create(xr_context* ctx, const xr_geometry* g, const xr_scan* s, int 
     d.cfdk = 2.0f * (float)M_PI / (float)P;
     {
         // launch shapes only: no result depends on these
-        const double near_den = 1.0 - 0.5 * std::sqrt(3.0) * g->n_vox * (double)g->vox_size / g->sod;
-        d.px = (float)((double)g->sdd / g->det_size / g->sod * g->vox_size / std::max(near_den, 0.05));
+        const double edge = g->n_vox * (double)g->vox_size / g->sod, centre = (double)g->sdd / g->det_size / g->sod * g->vox_size;
+        d.px = (float)(centre / std::max(1.0 - 0.5 * std::sqrt(3.0) * edge, 0.05));
+        d.px_mid = (float)(centre / std::max(1.0 - 0.4 * edge, 0.05));
         d.tilt_cos = d.tilt_sin = 0.0f;
         for (int c = 0; c < C; c++) {
             const float zz = std::min(std::fabs(p->cond_R[9 * c + 8]), 1.0f);
