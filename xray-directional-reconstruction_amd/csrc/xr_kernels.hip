@@ -1340,7 +1340,7 @@ struct FootStageAny {
                 pre[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff + k * step, 0, 0));
     }
     __device__ __forceinline__ void store(lds_float* buf, const FootSrc& f) const {
-        if (f.H == 0 || r0 >= f.R) return;  // H 0: not staged (and R has no meaning)
+        if (r0 >= f.R) return;
         const int rs = f.R * f.Ws;
 #pragma unroll
         for (int k = 0; k < C::NP; k++) {
@@ -1539,7 +1539,9 @@ __device__ __forceinline__ float backward_item(const BwdArgs& a, int o, int step
         f.W = f.Ws = f.R = 0;
         if (C::WF == 0) {
             const int w = uniformi(p[3]);
-            f.W = max(uniformi(p[2]), 1);  // a footprint that is not staged may have none
+            // a footprint that is not staged may have no width: of one, every thread's row is R = 0 or more
+            // or H = 0 ends the passes (tests of either in the store cost 3 %)
+            f.W = max(uniformi(p[2]), 1);
             f.Ws = w & 0xffff;
             f.R = w >> 16;
         }
