@@ -56,7 +56,7 @@ def test_copies_follow_the_views(xr, ctx, torch_dev, K):
 @pytest.mark.parametrize("N,U,V,K", [(20, 34, 30, 0), (65, 90, 100, 0), (150, 190, 240, 0), (270, 200, 180, 0), (64, 90, 80, 3),
                                      (130, 190, 150, 4)])
 def test_untilted_views_of_a_mixed_plan(orc, xr, ctx, torch_dev, N, U, V, K):
-    """They take the untilted splat: against the FP64 oracle (1e-5 relative L2,
+    """They are splat by whole columns: against the FP64 oracle (1e-5 relative L2,
     without the two outermost rows and columns, as the tilted ones)."""
     import torch
 

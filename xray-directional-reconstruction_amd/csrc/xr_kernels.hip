@@ -288,6 +288,16 @@ __device__ __forceinline__ void splat_inside(float t, float val, unsigned row0, 
     __hip_atomic_fetch_add(p + kBandStride + 1, (AccT)(AccS)q2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// Terms of pixels (iu, iv), (iu + 1, iv), (iu, iv + 1), (iu + 1, iv + 1) added at p, rounded to nearest.
+template <class AccT, class AccS>
+__device__ __forceinline__ void splat_rounded(lds_ptr<AccT> p, float t4, float t3, float t1, float t2) {
+    const int q4 = __float2int_rn(t4), q3 = __float2int_rn(t3), q1 = __float2int_rn(t1), q2 = __float2int_rn(t2);
+    __hip_atomic_fetch_add(p, (AccT)(AccS)q4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_add(p + 1, (AccT)(AccS)q3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_add(p + kBandStride, (AccT)(AccS)q1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_add(p + kBandStride + 1, (AccT)(AccS)q2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // The per-voxel basis rotation of forwardOrth / backwardOrth (ir.cu:316-328,
 // 390-400): rodriguesRotation (ir.cu:597-621) about the axis (cos phi, sin phi,
 // 0) with cosine cc and sine sqrt(1 - cc^2), (1 - cc) n n^T + [[cc, -n_z s,
@@ -597,15 +607,7 @@ __device__ __forceinline__ void splat_tilted(const FwdArgs& a, const ViewGeom& g
                     const float vs = val * scale;
                     const float c1 = (1.0f - fu) * fv, c2 = fu * fv;
                     const float c3 = fu * (1.0f - fv), c4 = (1.0f - fu) * (1.0f - fv);
-                    lds_ptr<AccT> p = acc + (iv - v0 + 1) * kBandStride + (iu - u0 + 1);
-                    const int q4 = __float2int_rn(c4 * vs), q3 = __float2int_rn(c3 * vs);
-                    const int q1 = __float2int_rn(c1 * vs), q2 = __float2int_rn(c2 * vs);
-                    __hip_atomic_fetch_add(p, (AccT)(AccS)q4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    __hip_atomic_fetch_add(p + 1, (AccT)(AccS)q3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    __hip_atomic_fetch_add(p + kBandStride, (AccT)(AccS)q1, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                    __hip_atomic_fetch_add(p + kBandStride + 1, (AccT)(AccS)q2, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                    splat_rounded<AccT, AccS>(acc + (iv - v0 + 1) * kBandStride + (iu - u0 + 1), c4 * vs, c3 * vs, c1 * vs, c2 * vs);
                 }
             }
         }
@@ -627,7 +629,11 @@ __device__ __forceinline__ void splat_tilted(const FwdArgs& a, const ViewGeom& g
 // 203^3 / 20 views 321 -> 226 us; 512^3 / 720 views, bound by VALU issue, 58.8 ->
 // 57.2 ms.
 // ---------------------------------------------------------------------------
-template <int KIND, int WAVES, int KM, int CH>
+// MIXED: the untilted views of a launch that also holds tilted ones.  Their images
+// keep the bits of splat_tilted (v by voxel_uv, four weighted terms rounded to
+// nearest, XTT weights not below zero): the column's terms are then 1/den and the
+// form of v at z = xc in place of B and A, and the u weights without the scale.
+template <int KIND, int WAVES, int KM, int CH, bool MIXED>
 __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& g, int code, gptr<const float> vol,
                                               float wscale, lds_ptr<typename FwdAcc<KIND>::T> acc, int band, int u0,
                                               int cs, int W, int v0, int vb) {
@@ -680,15 +686,25 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                         float fu;
                         split(u, iu, fu);
                         cand = (unsigned)(iu - (u0 + cs - 1)) <= (unsigned)W;
-                        sB = g.av[2] * inv;
-                        sA = fmaf(c.nv, inv, d.hv - 0.5f);
-                        sw0 = (1.0f - fu) * wscale;
-                        sw1 = fu * wscale;
                         scp = iu - u0 + 1;
-                        // t at the first and last z bounds every lane's t: z - xc is exact and
-                        // fmaf is monotone in it
-                        const float ta = fmaf(sB, z_first, sA), tb = fmaf(sB, z_end, sA);
-                        in = rows_all && fminf(ta, tb) > t_lo && fmaxf(ta, tb) < t_hi;
+                        // t (MIXED: v) at the first and last z bounds every lane's: z - xc is exact
+                        // and fmaf is monotone in it
+                        if (MIXED) {
+                            sB = inv;
+                            sA = c.nv;
+                            sw0 = 1.0f - fu;
+                            sw1 = fu;
+                            const float va = fmaf(fmaf(g.av[2], z_first, c.nv), inv, d.hv);
+                            const float ve = fmaf(fmaf(g.av[2], z_end, c.nv), inv, d.hv);
+                            in = rows_all && accept_v(va, d) && accept_v(ve, d);
+                        } else {
+                            sB = g.av[2] * inv;
+                            sA = fmaf(c.nv, inv, d.hv - 0.5f);
+                            sw0 = (1.0f - fu) * wscale;
+                            sw1 = fu * wscale;
+                            const float ta = fmaf(sB, z_first, sA), tb = fmaf(sB, z_end, sA);
+                            in = rows_all && fminf(ta, tb) > t_lo && fmaxf(ta, tb) < t_hi;
+                        }
                     }
                 }
                 // XTT: |d|^2 - dz^2 of the column's source->voxel vector d and
@@ -727,7 +743,12 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
 #pragma unroll
                             for (int k = 0; k < NCOL; k++) {
                                 int zb_k, ze_k;
-                                col_zrange_t(lane_f(sB, b[k]), lane_f(sA, b[k]), d, v0, vb, zb_k, ze_k);
+                                float B = lane_f(sB, b[k]), A = lane_f(sA, b[k]);
+                                if (MIXED) {
+                                    A = fmaf(A, B, d.hv - 0.5f);
+                                    B *= g.av[2];
+                                }
+                                col_zrange_t(B, A, d, v0, vb, zb_k, ze_k);
                                 zb = min(zb, zb_k);
                                 ze = max(ze, ze_k);
                             }
@@ -748,6 +769,19 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
                             };
                             auto splat = [&](int c, float val, float B, float A, unsigned row0, lds_ptr<AccT> spare,
                                              float w0, float w1) XR_INLINE {
+                                if constexpr (MIXED) {
+                                    const float v = fmaf(fmaf(g.av[2], lanef[c] + zoff, A), B, d.hv);
+                                    int iv;
+                                    float fv;
+                                    split(v, iv, fv);
+                                    if (in_chunk(c) && (INSIDE || (accept_v(v, d) && (unsigned)(iv - (v0 - 1)) <= (unsigned)vb))) {
+                                        const float vs = val * (KIND == FWD_PLAIN ? d.ratio : (XTT ? d.vs * d.ratio : 1.f)) * wscale;
+                                        const float gv = 1.0f - fv;
+                                        const lds_ptr<AccT> p = (lds_ptr<AccT>)(uintptr_t)row0 + iv * kBandStride;
+                                        splat_rounded<AccT, AccS>(p, w0 * gv * vs, w1 * gv * vs, w0 * fv * vs, w1 * fv * vs);
+                                    }
+                                    return;
+                                }
                                 const float t = fmaf(B, lanef[c] + zoff, A);
                                 if (in_chunk(c)) {
                                     if (XTT ? (mi >> b[0] & 1) != 0 : INSIDE)
@@ -833,7 +867,9 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
 #pragma unroll
                                         for (int c = 0; c < CH; c++) {
                                             const float q = fmaf(dz[c], sS2, ck);
-                                            val[c] = fmaf(fmaf(-q * q, id2[c], g2s), mu[c][k], val[c]);
+                                            float w = fmaf(-q * q, id2[c], g2s);
+                                            if (MIXED) w = fmaxf(w, 0.f);
+                                            val[c] = fmaf(w, mu[c][k], val[c]);
                                         }
                                     }
                                 }
@@ -873,7 +909,9 @@ __device__ __forceinline__ void splat_columns(const FwdArgs& a, const ViewGeom& 
 // One (band, view) work item o = band * n_slots + slot of a forward launch.
 // step selects the view list views + step*n_slots (a solver's subset step);
 // loss receives the item's share of sum |y - p|.
-template <int KIND, bool AXIS, int WAVES, int KM, int CH>
+// AXIS: every view of the launch is untilted.  MIXED: otherwise, those that are
+// take splat_columns (with the bits of splat_tilted).
+template <int KIND, bool AXIS, int WAVES, int KM, int CH, bool MIXED>
 __device__ __forceinline__ void forward_item(const FwdArgs& a, int o, int step, double* loss,
                                              unsigned long long* acc_raw, int v0, int vb) {
     typedef typename FwdAcc<KIND>::T AccT;
@@ -928,13 +966,18 @@ __device__ __forceinline__ void forward_item(const FwdArgs& a, int o, int step, 
     // value scale folded into the untilted splat weights: ratio (ir.cu:1513-1518),
     // XTT vs * ratio (ir.cu:1791)
     const float scalev = (KIND == FWD_PLAIN) ? d.ratio : (KIND == FWD_XTT ? d.vs * d.ratio : 1.f);
-    // A launch with tilted views (AXIS false) may hold untilted ones of other conditions, which need
-    // not pay for the tilt (unless the basis is rotated per voxel): 384^3, eight such views 1854 us as
-    // tilted ones, 705 as untilted.
-    if (AXIS || (g.axis != 0.f && !a.coef))
-        splat_columns<KIND, WAVES, KM, CH>(a, g, code, vol, scale * scalev, acc, band, u0, cs, W, v0, vb);
-    else if constexpr (!AXIS)
-        splat_tilted<KIND, WAVES, KM>(a, g, code, scale, acc, u0, cs, W, v0, vb);
+    // The untilted views of a launch that also holds tilted ones need not pay for the tilt (unless the
+    // basis is rotated per voxel): 384^3, eight such views 1854 us as tilted ones, 800 as columns.
+    bool columns = AXIS;
+    if constexpr (AXIS || MIXED) {
+        columns = AXIS || (g.axis != 0.f && !a.coef);
+        if (columns)
+            splat_columns<KIND, WAVES, KM, CH, MIXED>(a, g, code, vol, AXIS ? scale * scalev : scale, acc, band, u0, cs, W,
+                                                      v0, vb);
+    }
+    if constexpr (!AXIS) {
+        if (!columns) splat_tilted<KIND, WAVES, KM>(a, g, code, scale, acc, u0, cs, W, v0, vb);
+    }
     __syncthreads();
 
     double lsum = 0.0, l2sum = 0.0;  // sum |y - p|, sum (y - p)^2 (OUT_RESIDUAL_L2)
@@ -1049,7 +1092,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 12 ? 6 : 4) void k_forward(con
     const int chunk = o / per_chunk;
     const int v0 = a.v0 + chunk * a.vb;
     const int vb = min(a.vb, a.d.V - v0);
-    forward_item<KIND, AXIS, WAVES, KM, CH>(a, view_grouped(a, o - chunk * per_chunk), 0, a.loss, acc_raw, v0, vb);
+    forward_item<KIND, AXIS, WAVES, KM, CH, !AXIS>(a, view_grouped(a, o - chunk * per_chunk), 0, a.loss, acc_raw, v0, vb);
 }
 
 // Work queue of a persistent launch: q[0] hands out tickets 0, 1, 2, ...; a
@@ -1106,7 +1149,11 @@ __device__ __forceinline__ void forward_batch_loop(const FwdArgs* __restrict__ i
         const FwdArgs& a = items[i];
         const int o = view_grouped(a, t - (i ? item_end[i - 1] : 0));
         double* loss = a.loss ? a.loss + loss_shift : nullptr;
-        forward_item<KIND, AXES == 1, WAVES, KM, KIND == FWD_XTT ? kXttChunks : 8>(a, o, step, loss, acc_raw, a.v0, a.vb);
+        if (AXES == 1 || a.axis)
+            forward_item<KIND, true, WAVES, KM, KIND == FWD_XTT ? kXttChunks : 8, false>(a, o, step, loss, acc_raw, a.v0,
+                                                                                       a.vb);
+        else
+            forward_item<KIND, false, WAVES, KM, 8, false>(a, o, step, loss, acc_raw, a.v0, a.vb);
     }
 }
 
