@@ -144,10 +144,15 @@ float xr_default_vox_size(float sdd, float sod, float det_size);
  * only the work split, never the arithmetic: every voxel still sums the views
  * of a subset in order and the forward accumulation is exact fixed point, so
  * results are bitwise identical for every setting.
- *   bwd_zpl:  z voxels per lane in the backprojection (1, 2, 4; default by N)
+ *   bwd_zpl:  z voxels per lane in the backprojection (1, 2, 4)
  *   bwd_gx:   column groups along x in a backprojection block of 16 waves
- *             (1, 2, 4, 8, 16; gy = 16/gx; default 4); XTT kinds run 8-wave
- *             blocks, where a gx of 16 is taken as 8 (gy = 8/gx; default 2)
+ *             (1, 2, 4, 8, 16; gy = 16/gx); XTT kinds run 8-wave blocks, where
+ *             a gx of 16 is taken as 8 (gy = 8/gx; default 2)
+ *             Both zero: the shape by the volume, the footprint and the kind,
+ *             which need not be one of these (3 or 5 voxels per lane, one
+ *             column per wave in small volumes).  For the plain kinds the pair
+ *             that xr_plan_get_tiles reports for such a plan, (1 up to 64^3, 2
+ *             up to 128^3, 4 above; 4), means the same
  *   fwd_rows: cap on the detector rows of one forward launch (default: the
  *             most that fit 64 KB of LDS)
  *   fwd_scan: 0 (default): the forward of an untilted view scans, per volume
@@ -165,6 +170,8 @@ typedef struct xr_tiles {
 } xr_tiles;
 
 int xr_plan_set_tiles(xr_plan* plan, const xr_tiles* tiles);
+/* The plan's settings with those left open filled in; set on a plan they run what
+ * this one runs. */
 int xr_plan_get_tiles(const xr_plan* plan, xr_tiles* tiles);
 
 /* Autotuner: times every candidate tile shape of the plan's forward projection

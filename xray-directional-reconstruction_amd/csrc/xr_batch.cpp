@@ -46,8 +46,9 @@ bool valid_tiles(const xr_tiles& t) {
            (t.fwd_split == 0 || t.fwd_split == 1 || t.fwd_split == 2 || t.fwd_split == 4);
 }
 
-std::array<int, 5> tune_key(const xr_plan* p) {
-    return {p->g.n_vox, p->g.n_det_u, p->g.n_det_v, p->g.n_proj, p->axis_cond.empty() ? 0 : (int)p->axis_cond[0]};
+std::array<int, 6> tune_key(const xr_plan* p, bool batched) {
+    return {p->g.n_vox,  p->g.n_det_u, p->g.n_det_v, p->g.n_proj, p->axis_cond.empty() ? 0 : (int)p->axis_cond[0],
+            batched ? 1 : 0};
 }
 
 struct EventPair {
@@ -531,10 +532,11 @@ int xr_plan_get_tiles(const xr_plan* plan, xr_tiles* tiles) {
 
 // ------------------------------------------------------------ autotuner ----
 
-int xr_autotune(xr_context* ctx, xr_plan* plan, const float* vol_cols, const float* sino, xr_tiles* best,
-                double* best_ms) {
+// batched: the shapes as the batched kernels run them, otherwise as a standalone launch does (see launch_backward).
+static int autotune(xr_context* ctx, xr_plan* plan, const float* vol_cols, const float* sino, xr_tiles* best,
+                    double* best_ms, bool batched) {
     if (!ctx || !plan || !vol_cols || !sino) return fail(ctx, XR_ERR_INVALID, "bad args");
-    const auto key = tune_key(plan);
+    const auto key = tune_key(plan, batched);
     for (auto& kv : ctx->tune_cache) {
         if (kv.first == key) {
             plan->tiles = kv.second;
@@ -608,7 +610,7 @@ int xr_autotune(xr_context* ctx, xr_plan* plan, const float* vol_cols, const flo
             plan->tiles.bwd_gx = gx;
             double ms = 0;
             rc = time_it([&] { return backward_launch(plan, BWD_MLEM, proj.p, 0, codes.p, P, vol2.p, nullptr,
-                                                      nullptr, 0.f, 0); },
+                                                      nullptr, 0.f, 0, nullptr, batched); },
                          ms);
             if (rc != XR_OK) break;
             if (ms < bbest) {
@@ -628,6 +630,11 @@ int xr_autotune(xr_context* ctx, xr_plan* plan, const float* vol_cols, const flo
     if (best) *best = win;
     if (best_ms) *best_ms = fbest + bbest;
     return XR_OK;
+}
+
+int xr_autotune(xr_context* ctx, xr_plan* plan, const float* vol_cols, const float* sino, xr_tiles* best,
+                double* best_ms) {
+    return autotune(ctx, plan, vol_cols, sino, best, best_ms, false);
 }
 
 // -------------------------------------------------------------- batches ----
@@ -715,7 +722,7 @@ int xr_batch_autotune(xr_batch* b) {
     xr_context* ctx = b->ctx;
     XR_HIP(ctx, hipStreamSynchronize(ctx->stream));
     for (auto& p : b->pr)
-        if (!p.xtt()) XR_TRY(xr_autotune(ctx, p.plan, p.vol, p.sino, nullptr, nullptr));
+        if (!p.xtt()) XR_TRY(autotune(ctx, p.plan, p.vol, p.sino, nullptr, nullptr, true));
     b->free_tables();
     return XR_OK;
 }

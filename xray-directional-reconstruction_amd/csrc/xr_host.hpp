@@ -34,7 +34,7 @@ struct xr_context {
     std::vector<Ev> events;
     std::vector<hipEvent_t> pool;
     // autotuner results per (N, U, V, P, axis)
-    std::vector<std::pair<std::array<int, 5>, xr_tiles>> tune_cache;
+    std::vector<std::pair<std::array<int, 6>, xr_tiles>> tune_cache;
 };
 
 struct xr_plan {
@@ -159,9 +159,10 @@ int forward_launch(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stri
                    double* d_loss, const float* vmax_known = nullptr, float* vmax_buf = nullptr,
                    bool no_alloc = false, const int32_t* views = nullptr);
 // vmax_out (MLEM / ART kinds): receives the atomic max of |updated voxel| as
-// float bits; the caller clears it first.
+// float bits; the caller clears it first.  literal_shape: see BwdArgs::literal.
 int backward_launch(xr_plan* p, int kind, const float* proj, int code_base, const int32_t* d_codes, int n_views,
-                    float* vol, float* tmp, float* factor, float alpha, int overwrite, unsigned* vmax_out = nullptr);
+                    float* vol, float* tmp, float* factor, float alpha, int overwrite, unsigned* vmax_out = nullptr,
+                    bool literal_shape = false);
 // Per-pixel L/(factor + 1e-5) table of the plan (computed once).
 int ensure_norm(xr_plan* p);
 // Detector rows per forward row chunk for the plan's tile setting and the

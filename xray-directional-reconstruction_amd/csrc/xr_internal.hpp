@@ -156,6 +156,7 @@ struct BwdArgs {
     float alpha;             // ART step lambda/subsetSize
     int overwrite;           // FDK: 1 -> vol = sum, 0 -> vol += sum
     int zpl, gx, gy;          // tile shape: z voxels per lane (1, 2, 4), column groups along x, y (gx*gy = 16)
+    int literal;              // standalone launches: take zpl and gx as they are (see launch_backward)
     int tiles_x, tiles_y, tiles_z, n_tiles, per_xcd;
     int axis;                 // batched launches: 1 -> every view is axis aligned
     int wide;                 // untilted: footprints wider than the fixed staging width (set with the shape)

@@ -2795,6 +2795,7 @@ hipError_t launch_forward(const FwdArgs& a, int kind, bool axis, hipStream_t str
                : hipErrorInvalidValue;
 }
 
+constexpr int kDefaultGx = 4;  // plain kinds
 int default_zpl(int N) { return N > 128 ? 4 : (N > 64 ? 2 : 1); }
 
 inline bool bwd_xtt(int kind) { return kind == BWD_XTT_RAW || kind == BWD_XTT_MLEM || kind == BWD_XTT_ART; }
@@ -2841,7 +2842,7 @@ bool backward_shape(BwdArgs& a, int zpl, int gx, bool xtt) {
     if (zpl == 0) zpl = default_zpl(a.d.N);
     // default column layout: 8 x 8 columns (plain); 2 x 4 for XTT (measured
     // 144.6 against 146.2 ms for 4 x 2 at 256^3 x 13, 4 x 360 views)
-    if (gx == 0) gx = xtt ? 2 : 4;
+    if (gx == 0) gx = xtt ? 2 : kDefaultGx;
     if (!(zpl == 1 || zpl == 2 || zpl == 4)) return false;
     if (!(gx == 1 || gx == 2 || gx == 4 || gx == 8 || gx == 16)) return false;
     const int waves = xtt ? 8 : 16;
@@ -2960,7 +2961,12 @@ static hipError_t start_backward_xtt(const BwdArgs& a, bool axis, hipStream_t st
 
 hipError_t launch_backward(BwdArgs a, int kind, bool axis, hipStream_t stream) {
     bool small = false;
-    if (a.zpl == 0 && a.gx == 0)
+    // The shape that xr_plan_get_tiles reports for a plan that leaves it open stands for the same
+    // choice, so that setting it, or tuning that finds it fastest, does not lose the shapes that a
+    // setting cannot name.  (The batched kernels have the set shapes alone: their tuning is literal.)
+    const bool open = (a.zpl == 0 && a.gx == 0) ||
+                      (!a.literal && !bwd_xtt(kind) && a.zpl == default_zpl(a.d.N) && a.gx == kDefaultGx);
+    if (open)
         small = backward_choose(a, kind, axis);
     else if (!backward_shape(a, a.zpl, a.gx, bwd_xtt(kind)))
         return hipErrorInvalidValue;

@@ -414,7 +414,8 @@ int forward_rows(const xr_plan* p, int kind) {
 }
 
 int backward_launch(xr_plan* p, int kind, const float* proj, int code_base, const int32_t* d_codes, int n_views,
-                    float* vol, float* tmp, float* factor, float alpha, int overwrite, unsigned* vmax_out) {
+                    float* vol, float* tmp, float* factor, float alpha, int overwrite, unsigned* vmax_out,
+                    bool literal_shape) {
     xr_context* ctx = p->ctx;
     BwdArgs a{};
     a.d = p->dims;
@@ -434,6 +435,7 @@ int backward_launch(xr_plan* p, int kind, const float* proj, int code_base, cons
     a.vmax_out = (kind == BWD_MLEM || kind == BWD_ART) ? vmax_out : nullptr;
     a.zpl = p->tiles.bwd_zpl;
     a.gx = p->tiles.bwd_gx;
+    a.literal = literal_shape;
     bool axis = true;
     for (int c = 0; c < p->n_cond; c++) axis = axis && p->axis_cond[c];
     if ((kind == BWD_XTT_RAW || kind == BWD_XTT_MLEM || kind == BWD_XTT_ART) && p->d_orient) {
