@@ -85,17 +85,20 @@ __device__ __forceinline__ void tap_offsets(int t, int& d0, int& d1, int& d2) {
 // operand from global memory (one 16-byte load per lane, tap and 8 channels);
 // weights as plain rows instead of whole operands: 346 us for the first.
 // ---------------------------------------------------------------------------
-template <int MT>
+// Volumes of at most 8 or 4 layers take MFMA tiles of W = 8 or 4 layers by 2 or 4
+// columns of D1 (256 x 256 x 4, 24 channels, inference: 1203 -> 336 us).
+template <int MT, int W>
 struct ConvTile {
-    static constexpr int T0 = 2, T1 = MT == 1 ? 2 : 4, T2 = MT == 4 ? 32 : 16;
+    static constexpr int T0 = 2, T1 = W < 16 ? 32 * MT / W : (MT == 1 ? 2 : 4), T2 = W < 16 ? W : (MT == 4 ? 32 : 16);
+    static constexpr int R = 16 / W;  // columns of D1 per MFMA tile
     static constexpr int H1 = T1 + 2, H2 = T2 + 2, halo = (T0 + 2) * H1 * H2;
     static constexpr int stride = halo + 4;  // LDS distance of two chunks, 16-byte units
     static constexpr int64_t lds(int nchunk) { return 16 * (int64_t)stride * nchunk + 4 * 28 * nchunk; }
 };
 
-template <int MT, int NT>
+template <int MT, int NT, int W>
 __global__ __launch_bounds__(256, 2) void k_conv3(const ConvArgs a) {
-    using T = ConvTile<MT>;
+    using T = ConvTile<MT, W>;
     extern __shared__ bf16x8 conv_lds[];
     const int nch = a.Cin / 8, nq = 27 * nch;
     bf16x8* const halo = conv_lds;
@@ -125,8 +128,9 @@ __global__ __launch_bounds__(256, 2) void k_conv3(const ConvArgs a) {
     const lds_bf16x8* base[MT];
 #pragma unroll
     for (int m = 0; m < MT; m++) {
-        const int g = (wave * MT + m) / (T::T2 / 16), half = (wave * MT + m) % (T::T2 / 16);
-        base[m] = (const lds_bf16x8*)halo + (g / T::T1 * T::H1 + g % T::T1) * T::H2 + 16 * half + row;
+        const int g = (wave * MT + m) / (T::T2 / W), half = (wave * MT + m) % (T::T2 / W);
+        const int q0 = g / (T::T1 / T::R), q1 = g % (T::T1 / T::R) * T::R + row / W;
+        base[m] = (const lds_bf16x8*)halo + (q0 * T::H1 + q1) * T::H2 + W * half + row % W;
     }
     const __bf16* wop[NT];
 #pragma unroll
@@ -166,8 +170,8 @@ __global__ __launch_bounds__(256, 2) void k_conv3(const ConvArgs a) {
     // D layout of the 16x16 MFMA: lane holds column (lane & 15), rows 4*kg + i.
 #pragma unroll
     for (int m = 0; m < MT; m++) {
-        const int g = (wave * MT + m) / (T::T2 / 16), half = (wave * MT + m) % (T::T2 / 16);
-        const int v0 = o0 + g / T::T1, v1 = o1 + g % T::T1;
+        const int g = (wave * MT + m) / (T::T2 / W), half = (wave * MT + m) % (T::T2 / W);
+        const int v0 = o0 + g / (T::T1 / T::R), v1 = o1 + g % (T::T1 / T::R) * T::R + 4 * kg / W;
         if (v0 >= a.D0 || v1 >= a.D1) continue;
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
@@ -176,7 +180,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3(const ConvArgs a) {
             const float b = a.bias ? a.bias[co] : 0.f;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int v2 = o2 + 16 * half + 4 * kg + i;
+                const int v2 = o2 + W * half + 4 * kg % W + i;
                 if (v2 >= a.D2) continue;
                 const int64_t v = ((int64_t)v0 * a.D1 + v1) * a.D2 + v2;
                 float val = acc[m][nt][i] + b;
@@ -714,15 +718,15 @@ bool conv3_tiled_ok(const ConvArgs& a) {
            a.Ktpad == a.Cin / 8 * kTapsPad * 8 && nt <= 6;
 }
 
-template <int MT, int NT>
+template <int MT, int NT, int W>
 hipError_t conv3_run(const ConvArgs& a, unsigned tiles, int pieces, hipStream_t s) {
-    hipLaunchKernelGGL((k_conv3<MT, NT>), dim3(tiles, pieces), dim3(256), ConvTile<MT>::lds(a.Cin / 8), s, a);
+    hipLaunchKernelGGL((k_conv3<MT, NT, W>), dim3(tiles, pieces), dim3(256), (ConvTile<MT, W>::lds(a.Cin / 8)), s, a);
     return hipGetLastError();
 }
 
-template <int MT>
+template <int MT, int W>
 hipError_t conv3_pieces(const ConvArgs& a, int nt, hipStream_t s) {
-    using T = ConvTile<MT>;
+    using T = ConvTile<MT, W>;
     const int64_t tiles = (int64_t)((a.D0 + T::T0 - 1) / T::T0) * ((a.D1 + T::T1 - 1) / T::T1) * ((a.D2 + T::T2 - 1) / T::T2);
     if (tiles > INT32_MAX) return hipErrorInvalidValue;
     // at most 6 output tiles per block (accumulators in registers), fewer where
@@ -730,12 +734,12 @@ hipError_t conv3_pieces(const ConvArgs& a, int nt, hipStream_t s) {
     const int want = (int)std::max<int64_t>((nt + 5) / 6, std::min<int64_t>(nt, (512 + tiles - 1) / tiles));
     const int per = (nt + want - 1) / want, pieces = (nt + per - 1) / per;
     switch (per) {
-        case 1: return conv3_run<MT, 1>(a, (unsigned)tiles, pieces, s);
-        case 2: return conv3_run<MT, 2>(a, (unsigned)tiles, pieces, s);
-        case 3: return conv3_run<MT, 3>(a, (unsigned)tiles, pieces, s);
-        case 4: return conv3_run<MT, 4>(a, (unsigned)tiles, pieces, s);
-        case 5: return conv3_run<MT, 5>(a, (unsigned)tiles, pieces, s);
-        default: return conv3_run<MT, 6>(a, (unsigned)tiles, pieces, s);
+        case 1: return conv3_run<MT, 1, W>(a, (unsigned)tiles, pieces, s);
+        case 2: return conv3_run<MT, 2, W>(a, (unsigned)tiles, pieces, s);
+        case 3: return conv3_run<MT, 3, W>(a, (unsigned)tiles, pieces, s);
+        case 4: return conv3_run<MT, 4, W>(a, (unsigned)tiles, pieces, s);
+        case 5: return conv3_run<MT, 5, W>(a, (unsigned)tiles, pieces, s);
+        default: return conv3_run<MT, 6, W>(a, (unsigned)tiles, pieces, s);
     }
 }
 
@@ -780,11 +784,16 @@ hipError_t launch_conv3(const ConvArgs& a, hipStream_t s) {
     }
     if (nt > 9 || a.Cin / 8 > 24) return hipErrorInvalidValue;
     // the largest tile whose halo of all channels leaves room for two blocks in
-    // a CU's 160 KB; the smallest tile takes 24 chunks in 110 KB
+    // a CU's 160 KB (the smallest takes 24 chunks in 110 KB) and that is not half
+    // empty: 256 x 256 x 8, 24 channels, inference with tiles of 32, 16, 8 layers
+    // 1253, 1089, 475 us
     const int nch = a.Cin / 8;
-    if (ConvTile<4>::lds(nch) <= 80 * 1024) return conv3_pieces<4>(a, nt, s);
-    if (ConvTile<2>::lds(nch) <= 80 * 1024) return conv3_pieces<2>(a, nt, s);
-    return conv3_pieces<1>(a, nt, s);
+    constexpr int64_t room = 80 * 1024;
+    if (a.D2 <= 4) return ConvTile<2, 4>::lds(nch) <= room ? conv3_pieces<2, 4>(a, nt, s) : conv3_pieces<1, 4>(a, nt, s);
+    if (a.D2 <= 8) return ConvTile<2, 8>::lds(nch) <= room ? conv3_pieces<2, 8>(a, nt, s) : conv3_pieces<1, 8>(a, nt, s);
+    if (a.D2 > 16 && ConvTile<4, 16>::lds(nch) <= room) return conv3_pieces<4, 16>(a, nt, s);
+    if (ConvTile<2, 16>::lds(nch) <= room) return conv3_pieces<2, 16>(a, nt, s);
+    return conv3_pieces<1, 16>(a, nt, s);
 }
 
 hipError_t launch_conv3_wgrad(const WgradArgs& a, hipStream_t s) {
