@@ -370,7 +370,8 @@ int forward_launch(xr_plan* p, int kind, const float* vol, int64_t vol_cond_stri
         a.coef = p->d_orient;  // forwardOrth: per-voxel rotation, general path
         axis = false;
     }
-    a.lanes_z = lanes_along_z(kind == FWD_XTT ? p->n_basis : 1, p->g.n_vox, n_slots);
+    // (the weight pass reads no volume)
+    a.lanes_z = kind != FWD_WEIGHT && lanes_along_z(kind == FWD_XTT ? p->n_basis : 1, p->g.n_vox, n_slots);
     bool copies = false;
     if (!axis && kind != FWD_WEIGHT && !no_alloc)
         XR_TRY(lane_copies(p, kind, vol, vol_cond_stride, code_base, views, n_slots, a, copies));
