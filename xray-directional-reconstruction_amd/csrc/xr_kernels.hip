@@ -1452,17 +1452,13 @@ __device__ __forceinline__ float backward_update(const BwdArgs& a, const float (
 }
 
 // Bilinear sample of texels (iu, iv), (iu + 1, iv), (iu, iv + 1), (iu + 1, iv + 1).
-// Tilted: four weighted terms and no difference of texels, so that an infinite
-// texel (a pixel without a count) beside a finite one gives infinity, not NaN.
+// Tilted: weighted terms alone and no difference, so that an infinite texel (a
+// pixel without a count) beside a finite one gives infinity, not NaN.
 template <bool TILT>
 __device__ __forceinline__ float blend(float fu, float fv, float r00, float r01, float r10, float r11) {
     const float gu = 1.0f - fu;
-    if (TILT) {
-        const float gv = 1.0f - fv;
-        return fmaf(gu * gv, r00, fmaf(fu * gv, r01, fmaf(fu * fv, r11, gu * fv * r10)));
-    }
     const float top = fmaf(fu, r01, gu * r00), bot = fmaf(fu, r11, gu * r10);
-    return fmaf(fv, bot - top, top);
+    return TILT ? fmaf(fv, bot, (1.0f - fv) * top) : fmaf(fv, bot - top, top);
 }
 
 // One voxel tile o of a backprojection launch; step selects the view list
