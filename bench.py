@@ -457,7 +457,8 @@ def grad_measure(ctx, xr, geom, sino, lam=1e-3):
     rb_ms = (rec[2][2] - rec[1][2]) / 3
     tables_ms = rec[1][1] - 3 * rf_ms  # the plan's weight pass (fixed-point bound of the forward)
     vv = float(N1) ** 3 * P
-    flops = 8.0 * (N - 2) ** 3 * N
+    # two products of each slice, each folded into its even and odd modes: 2 x 2 x M x M x M/2
+    flops = 2.0 * (N - 2) ** 3 * N
     return {"workload": "gradient slot on the %d^3 grid (%d views, %dx%d detector) + Poisson integration of %d^3"
                         % (N1, P, U, V, N),
             "slot_epoch_ms": round(f_ms + b_ms, 3), "forward_ms": round(f_ms, 3), "backward_ms": round(b_ms, 3),
@@ -664,6 +665,7 @@ def main():
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "kernel": dom_name,
                 "kernel_ms": round(dom_ms, 3), "launches_per_pass": 1,
+                "limited_by": "VALU issue (profiles/pmc_traffic_512_720.md)",
                 "algorithmic_bytes": "4 B per voxel-view x %d^3 voxels x %d views per launch" % (N, P)}
     out = {
         "metric": METRIC, "value": round(gups, 2), "unit": "GUPS", "n_gpus": 1, "steps": args.steps,

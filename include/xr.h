@@ -401,7 +401,9 @@ int xr_grad_reconstruct(xr_context* ctx, const xr_geometry* g, const xr_scan* s,
  * (FP32, as the reference) on the interior.  gx, gy: (n+1)^3 device arrays,
  * vol: n^3 device array, reference layouts; n >= 3.  Solved exactly by type-I
  * sine transforms in FP64 (the reference factorises the matrix with Eigen's
- * SparseLU in FP32), result rounded to FP32. */
+ * SparseLU in FP32), result rounded to FP32.  The context keeps the solve's
+ * workspace (up to 1200 MiB, or one slice where that is more) until it is
+ * destroyed. */
 int xr_poisson_solve(xr_context* ctx, int n, const float* gx, const float* gy, float* vol);
 
 /* ---- batched multi-problem solver ---------------------------------------- */

@@ -430,11 +430,16 @@ __global__ void k_band_rows(const ViewGeom* __restrict__ vg, const Dims d, int n
 //    i / L, L the longest interval of the 64 columns looked at together.
 // (u, v) and the acceptance tests are those of col_forms and voxel_uv, so the
 // images do not depend on the lane axis nor on the packing.
-// Per voxel about 45 VALU instructions (nine FMAs for the three forms, the
-// reciprocal, the splits, four rounded products) and four LDS adds.  Measured
-// against whole columns of z in every lane: 120^3 x 3 coefficients, 4 x 60
-// views tilted by 0, 20, 45 and 90 degrees, 31.8 -> 2.1 ms per launch; 128^3,
-// 45 views at 30 degrees, 0.96 -> 0.39 ms.
+// Bound by VALU issue (0.77 to 0.85 where a CU has blocks; a launch of few
+// views leaves 30 to 40 % of the chip's time idle at its end).  A visited voxel
+// costs about 45 VALU instructions (nine FMAs for the three forms, the
+// reciprocal, the splits, four rounded products) and four LDS adds; with the
+// intervals, their packing and the slots that it leaves empty the counters
+// read 151 VALU per 64 voxel-views of the volume (128^3, 45 views at 30
+// degrees) and 176 (120^3 x 3 coefficients).  Measured against whole columns
+// of z in every lane: 120^3 x 3 coefficients, 4 x 60 views tilted by 0, 20, 45
+// and 90 degrees, 31.8 -> 2.3 ms per launch; 128^3, 45 views at 30 degrees, 0.96
+// -> 0.40 ms.
 // ---------------------------------------------------------------------------
 
 // XTT voxel value sum_k mu_k (S_k.G)^2 |B x S_k|^2 vs ratio (ir.cu:1780-1794)
@@ -625,9 +630,9 @@ __device__ __forceinline__ void splat_tilted(const FwdArgs& a, const ViewGeom& g
 // Columns whose z extent lies inside the window (t is monotone in z) run
 // without tests; a partial last chunk only masks its lanes (such depths used to
 // take masked loads and tests throughout).
-// Measured, column pairs of eight chunks -> now: 64^3 / 90 views 94 -> 64 us;
-// 203^3 / 20 views 321 -> 226 us; 512^3 / 720 views, bound by VALU issue, 58.8 ->
-// 57.2 ms.
+// Measured, column pairs of eight chunks -> now: 64^3 / 90 views 94 -> 58 us;
+// 203^3 / 20 views 321 -> 207 us; 512^3 / 720 views, bound by VALU issue, 58.8
+// against 57.7 ms.
 // ---------------------------------------------------------------------------
 // MIXED: the untilted views of a launch that also holds tilted ones.  Their images
 // keep the bits of splat_tilted (v by voxel_uv, four weighted terms rounded to
@@ -1208,8 +1213,8 @@ __global__ __launch_bounds__(64 * kFwdWaves) __attribute__((amdgpu_waves_per_eu(
 // Bound by VALU issue (about 15 instructions per 64 voxel-views of a whole
 // column), the footprint's edges and, with few views, the tile's start.
 // Measured, before -> now: MLEM 512^3 / 720 views 60.4 -> 48.7 ms, 64^3 / 90
-// views 184 -> 41 us, 203^3 / 20 views 249 -> 154 us; FDK 320^3 / 401 views
-// 18.2 -> 7.3 ms; ART 128^3 tilted by 30 degrees, 45 views 478 -> 210 us.
+// views 184 -> 41 us, 203^3 / 20 views 249 -> 152 us; FDK 320^3 / 401 views
+// 18.2 -> 7.8 ms; ART 128^3 tilted by 30 degrees, 45 views 478 -> 178 us.
 // ---------------------------------------------------------------------------
 template <int KIND>
 struct IsXtt {
@@ -2852,8 +2857,10 @@ bool backward_shape(BwdArgs& a, int zpl, int gx, bool xtt) {
 // Plain, untilted: the z depth zpl (1 to 5) that covers the volume's 64-voxel
 // chunks with the least work, tiles_z (zpl + 2): a column's terms and a
 // footprint's edges cost about as much per view as two chunks (three chunks,
-// 160^3 / 180 views: zpl 3 615, 4 724, 2 971 us; five chunks, 320^3 / 60 views:
-// zpl 5 1171, 2 1605, 4 1759 us).
+// raw sums, 160^3 / 180 views: zpl 3 615, 4 724, 2 971 us; five chunks, 320^3 / 60
+// views: zpl 5, 4, 2 raw 1127, 1867, 2021 us; FDK 926, 1667, 1904; ART 911, 1662,
+// 1875; MLEM, whose two sums per voxel spill some registers at zpl 5, 1007, 1746,
+// 1945).
 // Footprints of any width (w > 16 where the magnification is largest): the depth
 // whose footprint fits the staging buffer 0.4 edges off the centre; the few tiles
 // nearer the source read the image directly.  (By the nearest voxel 512^3
